@@ -94,23 +94,31 @@ enum Mode : int {
 };
 
 // Time-loop scalars, double-buffered like the reference's n/n+1 pairs.
-// minKey / maxKey accumulate the CFL minimum and the maximum pressure of the
-// step with parity cur as order-preserving integer keys (atomic min / max,
-// exact and order-free); the finalize kernel turns them into dt and pmax
-// and resets the other parity's pair for the next step.
 struct Scalars {
   double t[2];
   double dt[2];
   double pmax;
   int err;        // MHY_ERR_* raised by a kernel (energy abort, NaN)
   int pad;
-  unsigned long long minKey[2], maxKey[2];
 };
 
-// Integer keys ordered like the doubles they encode.  minKey only sees
+// Accumulators of the CFL minimum and the maximum pressure of a step, as
+// order-preserving integer keys (atomic min / max, exact and order-free):
+// slot s of the step with parity cur is k[cur][s], [0] the minimum, [1] the
+// maximum.  Device-scope atomics on one line run one after the other, about
+// 6 ns each (1024 blocks with a min and a max each on one line: 13 of the
+// 21 us of the reduction on a 1024^2 mesh), so the blocks spread over
+// kDtSlots lines of 128 bytes (one per XCD); the node update folds the slots
+// into dt, and the first thread of it resets the other parity's for the next step.
+constexpr int kDtSlots = 8;
+struct DtKeys {
+  unsigned long long k[2][kDtSlots][16];
+};
+
+// Integer keys ordered like the doubles they encode.  The minimum only sees
 // values >= +0 or NaN (CFL ratios), whose bit patterns already order as
-// unsigned integers, with every NaN above the initial DBL_MAX; maxKey maps
-// the sign so that all doubles order, and NaN is filtered before.
+// unsigned integers, with every NaN above the initial DBL_MAX; the maximum
+// maps the sign so that all doubles order, and NaN is filtered before.
 MHY_HD unsigned long long dkeyPos(double v) { return __builtin_bit_cast(unsigned long long, v); }
 MHY_HD double dkeyPosInv(unsigned long long k) { return __builtin_bit_cast(double, k); }
 MHY_HD unsigned long long dkeySigned(double v) {
@@ -177,6 +185,7 @@ struct FieldsT {
   double *XL2;       // end-of-Lagrange node coordinate along the second sweep
   unsigned char* envx;  // compact1: the cell's material fields are stored (1) or derived (0)
   Scalars* sc;
+  DtKeys* keys;
 };
 
 // Parameters of one launch: fields, options, parity and sweep direction.
@@ -190,6 +199,8 @@ struct KPT {
   int fuseFinal; // sweep 2 finishes each cell (final remap) instead of storing U2
   int geomLoad;  // the sweeps read the Lagrange volume and centroid (V_L, Xc_L, Yc_L)
                  // instead of forming them again from the node velocities
+  int dtFold;    // the node update forms dt_{n+1} from the accumulators (whole steps);
+                 // 0: it reads the dt a finalize kernel left (phase-level calls)
   long ncell, nnode;
 };
 

@@ -92,6 +92,9 @@ struct mhy_ctx {
   // MAHYCO_FUSE_FINAL=0 keeps it a separate kernel); finalDone records that
   // the current iteration's final remap is already done
   bool fuseFinal = true, finalDone = false;
+  // whole steps: the node update folds the dt accumulators itself; the
+  // phase-level calls launch a finalize kernel in the dt phase instead
+  bool dtFold = false;
   // sweep 1 runs the cell part of the Lagrange phase (wave sweeps only;
   // environment MAHYCO_FUSE_LAGRANGE=0 keeps it a separate kernel)
   bool fuseLag = true;
@@ -238,6 +241,7 @@ KP makeKP(const mhy_ctx* x) {
   kp.sweep = 1;
   kp.xdir = 1;
   kp.fuseFinal = 0;
+  kp.dtFold = x->dtFold ? 1 : 0;
   // the stored Lagrange geometry exists unless the fused first sweep keeps
   // it in registers only
   kp.geomLoad = (!x->fuseLag || x->geomStored) ? 1 : 0;
@@ -407,7 +411,7 @@ int phaseEucStart(mhy_ctx* x) {
   const unsigned nb = (unsigned)std::min<long>(kReduceBlocks, (x->ncell + kBlock - 1) / kBlock);
   timed(x, K_DT, [&] {
     hipLaunchKernelGGL(ks[x->o.nbmat - 1], dim3(nb), dim3(kBlock), 0, x->stream, kp, x->ef);
-    hipLaunchKernelGGL(k_euc_dt_finalize, dim3(1), dim3(64), 0, x->stream, kp);
+    if (!x->dtFold) hipLaunchKernelGGL(k_euc_dt_finalize, dim3(1), dim3(64), 0, x->stream, kp);
   });
   return checkLaunch(x, "eucclhyd start");
 }
@@ -478,7 +482,7 @@ int phaseDt(mhy_ctx* x) {
     const unsigned nb = (unsigned)std::min<long>(kReduceBlocks, (x->ncell + kBlock - 1) / kBlock);
     timed(x, K_DT, [&] {
       launchR(x, k_dt_reduce<double>, k_dt_reduce<float>, dim3(nb), dim3(kBlock), kp);
-      launchR(x, k_dt_finalize<double>, k_dt_finalize<float>, dim3(1), dim3(64), kp);
+      if (!x->dtFold) launchR(x, k_dt_finalize<double>, k_dt_finalize<float>, dim3(1), dim3(64), kp);
     });
   }
   return checkLaunch(x, "dt");
@@ -493,13 +497,14 @@ bool lagFused(const mhy_ctx* x) { return x->fuseLag && (x->x_then_y_n || x->fuse
 int phaseLagrange(mhy_ctx* x) {
   if (x->euc) return phaseEucLagrange(x);
   KP kp = makeKP(x);
-  // (a grid's y dimension holds at most 65535 node rows)
-  if (x->o.mode == MODE_FULL && x->o.nx >= 2 && x->o.ny >= 2 && x->o.ny - 1 <= 65535 && x->splitNode) {
-    const dim3 gi((unsigned)((x->o.nx - 1 + kBlock - 1) / kBlock), (unsigned)(x->o.ny - 1));
-    const long nedge = 2L * (x->o.nx + 1) + 2L * (x->o.ny - 1);
+  // interior rows, then enough rows of blocks for the boundary nodes (a
+  // grid's y dimension holds at most 65535)
+  const long gx = (x->o.nx - 1 + kBlock - 1) / kBlock, nedge = 2L * (x->o.nx + 1) + 2L * (x->o.ny - 1);
+  const long rows = x->o.ny - 1 + (nedge + gx * kBlock - 1) / std::max(gx * kBlock, 1L);
+  if (x->o.mode == MODE_FULL && x->o.nx >= 2 && x->o.ny >= 2 && rows <= 65535 && x->splitNode) {
     timed(x, K_NODE, [&] {
-      launchR(x, k_lagrange_node_inner<double>, k_lagrange_node_inner<float>, gi, dim3(kBlock), kp);
-      launchR(x, k_lagrange_node_edge<double>, k_lagrange_node_edge<float>, gridFor(nedge), dim3(kBlock), kp);
+      launchR(x, k_lagrange_node_euler<double>, k_lagrange_node_euler<float>, dim3((unsigned)gx, (unsigned)rows),
+              dim3(kBlock), kp);
     });
   } else {
     timed(x, K_NODE, [&] {
@@ -673,6 +678,12 @@ void endIteration(mhy_ctx* x) {
 }
 
 int runIteration(mhy_ctx* x) {
+  // (the advection mode has its own dt kernel)
+  struct Fold {
+    mhy_ctx* x;
+    explicit Fold(mhy_ctx* c) : x(c) { x->dtFold = x->euc || x->o.mode != MODE_ADVECTION; }
+    ~Fold() { x->dtFold = false; }
+  } fold(x);
   int st;
   if ((st = phaseDt(x)) != MHY_OK) return st;
   if ((st = phaseLagrange(x)) != MHY_OK) return st;
@@ -890,6 +901,9 @@ static int setupEucclhyd(mhy_ctx* x, const mhy_config& c, bool batchMember) {
     void* p = nullptr;
     if ((e = hipMalloc(&p, sizeof(Scalars))) == hipSuccess) x->allocs.push_back(p);
     f.sc = static_cast<Scalars*>(p);
+    p = nullptr;
+    if (e == hipSuccess && (e = hipMalloc(&p, sizeof(DtKeys))) == hipSuccess) x->allocs.push_back(p);
+    f.keys = static_cast<DtKeys*>(p);
   }
 #undef AD
   if (e != hipSuccess) return fail(x, MHY_ERR_DEVICE, std::string("device allocation: ") + hipGetErrorString(e));
@@ -922,8 +936,12 @@ static int setupEucclhyd(mhy_ctx* x, const mhy_config& c, bool batchMember) {
   std::memset(&s0, 0, sizeof(s0));
   s0.t[0] = 0.0;
   s0.dt[0] = h.deltat_init;
-  for (int q = 0; q < 2; ++q) s0.minKey[q] = dkeyPos(DBL_MAX), s0.maxKey[q] = dkeySigned(-DBL_MAX);
-  if (hipMemcpy(f.sc, &s0, sizeof(s0), hipMemcpyHostToDevice) != hipSuccess)
+  DtKeys k0;
+  std::memset(&k0, 0, sizeof(k0));
+  for (int q = 0; q < 2; ++q)
+    for (int i = 0; i < kDtSlots; ++i) k0.k[q][i][0] = dkeyPos(DBL_MAX), k0.k[q][i][1] = dkeySigned(-DBL_MAX);
+  if (hipMemcpy(f.sc, &s0, sizeof(s0), hipMemcpyHostToDevice) != hipSuccess ||
+      hipMemcpy(f.keys, &k0, sizeof(k0), hipMemcpyHostToDevice) != hipSuccess)
     return fail(x, MHY_ERR_DEVICE, "upload scalars");
   x->init = HostInit();
   x->cur = 0;
@@ -1133,6 +1151,9 @@ static int createContext(const mhy_config* cfg, mhy_ctx** out, bool batchMember)
     void* p = nullptr;
     if ((e = hipMalloc(&p, sizeof(Scalars))) == hipSuccess) x->allocs.push_back(p);
     f.sc = static_cast<Scalars*>(p);
+    p = nullptr;
+    if (e == hipSuccess && (e = hipMalloc(&p, sizeof(DtKeys))) == hipSuccess) x->allocs.push_back(p);
+    f.keys = static_cast<DtKeys*>(p);
   }
 #undef AR
 #undef AD
@@ -1179,8 +1200,12 @@ static int createContext(const mhy_config* cfg, mhy_ctx** out, bool batchMember)
   std::memset(&s0, 0, sizeof(s0));
   s0.t[0] = 0.0;
   s0.dt[0] = h.deltat_init;
-  for (int q = 0; q < 2; ++q) s0.minKey[q] = dkeyPos(DBL_MAX), s0.maxKey[q] = dkeySigned(-DBL_MAX);
-  if (hipMemcpy(f.sc, &s0, sizeof(s0), hipMemcpyHostToDevice) != hipSuccess)
+  DtKeys k0;
+  std::memset(&k0, 0, sizeof(k0));
+  for (int q = 0; q < 2; ++q)
+    for (int i = 0; i < kDtSlots; ++i) k0.k[q][i][0] = dkeyPos(DBL_MAX), k0.k[q][i][1] = dkeySigned(-DBL_MAX);
+  if (hipMemcpy(f.sc, &s0, sizeof(s0), hipMemcpyHostToDevice) != hipSuccess ||
+      hipMemcpy(f.keys, &k0, sizeof(k0), hipMemcpyHostToDevice) != hipSuccess)
     return bail(fail(x, MHY_ERR_DEVICE, "upload scalars"));
   // computeNodeMass of the prologue (VnrRemap.cc:341)
   {
@@ -1788,10 +1813,6 @@ int batchEnqueueStepR(mhy_batch* b, int cur, bool xty, bool timing) {
     if (timing) (void)hipEventRecord(b->ev[2 * k + 1], b->stream);
   };
   launch(BK_DT, k_dt_reduce_batch<R, false>, k_dt_reduce_batch<R, true>, cur);
-  {
-    BatchLaunchT<R> bl{static_cast<const KPT<R>*>(b->dTable), nullptr, nullptr, n, cur, 0u, nullptr};
-    hipLaunchKernelGGL(k_dt_finalize_batch<R>, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, b->stream, bl);
-  }
   launch(BK_NODE, k_lagrange_node_batch<R, false>, k_lagrange_node_batch<R, true>, cur);
   static const Fn cellLoop[3] = {k_lagrange_cell_batch<R, 1, false>, k_lagrange_cell_batch<R, 2, false>,
                                  k_lagrange_cell_batch<R, 3, false>};
@@ -1904,6 +1925,7 @@ int mhy_batch_create(const mhy_config* cfgs, int n, mhy_batch** out) {
       kp.sweep = ((v >> 1) & 1) + 1;
       kp.xdir = (v >> 2) & 1;
       kp.fuseFinal = (v >> 3) & 1;
+      kp.dtFold = 1;
       table[(size_t)v * n + i] = kp;
     }
   // virtual-block layout of every kernel

@@ -269,22 +269,34 @@ __global__ __launch_bounds__(256) void k_euc_start(KP kp, EucFields e) {
   if (threadIdx.x == 0) {
     double lo = smn[0];
     for (int k = 1; k < (int)(blockDim.x >> 6); ++k) lo = smin(lo, smn[k]);
-    atomicMin(&f.sc->minKey[cur], dkeyPos(lo));
+    atomicMin(&f.keys->k[cur][blockIdx.x % kDtSlots][0], dkeyPos(lo));
   }
 }
 
 // computedeltat (EucclhydRemap.cc:203-227) and updateTime: dt_{n+1} =
 // min(cfl * minimum, 1.05 dt_n); below deltat_min the run stops with
-// MHY_ERR_DT_MIN.  Resets the minimum of the next step's parity.
-__global__ void k_euc_dt_finalize(KP kp) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
+// MHY_ERR_DT_MIN.  Resets the minimum of the next step's parity.  Nothing of
+// the step itself reads dt_{n+1} (the nodes move with dt_n), so in whole steps
+// one thread of the node kernel does it (kp.dtFold) and the launch of its
+// own, 4.6 us, is left to the phase-level calls.
+__device__ __forceinline__ void eucDtStore(const KP& kp) {
   Scalars* sc = kp.f.sc;
-  const double lo = dkeyPosInv(sc->minKey[kp.cur]);
+  unsigned long long key = kp.f.keys->k[kp.cur][0][0];
+#pragma unroll
+  for (int s = 1; s < kDtSlots; ++s) {
+    const unsigned long long a = kp.f.keys->k[kp.cur][s][0];
+    key = (a < key) ? a : key;
+  }
+  const double lo = dkeyPosInv(key);
   const double dt1 = smin(kEucCfl * lo, sc->dt[kp.cur] * 1.05);
   sc->dt[kp.nxt] = dt1;
   sc->t[kp.nxt] = sc->t[kp.cur] + dt1;
   if (dt1 < kp.o.deltat_min) raiseErr(sc, MHY_ERR_DT_MIN);
-  sc->minKey[kp.nxt] = dkeyPos(DBL_MAX);
+#pragma unroll
+  for (int s = 0; s < kDtSlots; ++s) kp.f.keys->k[kp.nxt][s][0] = dkeyPos(DBL_MAX);
+}
+__global__ void k_euc_dt_finalize(KP kp) {
+  if (threadIdx.x == 0 && blockIdx.x == 0) eucDtStore(kp);
 }
 
 // EOS and mean pressure only: the dumps at t_n print the pressure of state
@@ -305,6 +317,7 @@ __global__ __launch_bounds__(256) void k_euc_eos(KP kp) {
 template <int M>
 __global__ __launch_bounds__(256) void k_euc_node(KP kp, EucFields e) {
   const long p = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (p == 0 && kp.dtFold) eucDtStore(kp);
   if (p >= kp.nnode) return;
   const Opts& o = kp.o;
   const auto& f = kp.f;

@@ -25,16 +25,12 @@ __global__ void k_dt_reduce(KPT<R> kp);
 template <class R>
 __global__ void k_dt_finalize(KPT<R> kp);
 template <class R>
-__global__ void k_dt_finalize_batch(BatchLaunchT<R> bl);
-template <class R>
 __global__ void k_dt_hold(KPT<R> kp);
 template <class R>
 __global__ void k_lagrange_node(KPT<R> kp);
-// the same node update on the fixed Euler grid, interior and boundary nodes
+// the same node update on the fixed Euler grid, laid out by node row
 template <class R>
-__global__ void k_lagrange_node_inner(KPT<R> kp);
-template <class R>
-__global__ void k_lagrange_node_edge(KPT<R> kp);
+__global__ void k_lagrange_node_euler(KPT<R> kp);
 template <class R, int M>
 __global__ void k_lagrange_cell(KPT<R> kp);
 template <class R, bool ONE>

@@ -41,7 +41,7 @@ __device__ __forceinline__ D2 nodeX(const KPT<R>& kp, long j, long i) {
 // reduction of PhaseLagrange.cc:55-61.  Min and max ignore NaN values like
 // the reference's reducers.  Each block reduces its cells and adds them to
 // the step's accumulators with one 64-bit atomic min / max (exact and
-// order-free, no fence); k_dt_finalize then forms dt and t (computeTime).
+// order-free, no fence); the node update then forms dt and t (computeTime).
 // b: block index among the nb blocks working on this problem.  The
 // reduction is FP64 in both forms (FP32 inputs are widened).
 template <class R>
@@ -76,9 +76,9 @@ __device__ __forceinline__ void dtReduceBody(const KPT<R>& kp, unsigned b, unsig
   if (threadIdx.x == 0) {
     double lo = smn[0], hi = smx[0];
     for (int k = 1; k < (int)(blockDim.x >> 6); ++k) lo = smin(lo, smn[k]), hi = (smx[k] > hi) ? smx[k] : hi;
-    Scalars* sc = f.sc;
-    atomicMin(&sc->minKey[kp.cur], dkeyPos(lo));
-    atomicMax(&sc->maxKey[kp.cur], dkeySigned(hi));
+    unsigned long long* slot = f.keys->k[kp.cur][b % kDtSlots];
+    atomicMin(&slot[0], dkeyPos(lo));
+    atomicMax(&slot[1], dkeySigned(hi));
   }
 }
 
@@ -87,22 +87,50 @@ __global__ __launch_bounds__(256) void k_dt_reduce(KPT<R> kp) {
   dtReduceBody(kp, blockIdx.x, gridDim.x);
 }
 
-// dt_{n+1} = min(CFL minimum, 1.05 dt_n) and t_{n+1} (VnrRemap.cc:45-50,
-// computeTime); resets the accumulators of the next step's parity.
-__device__ __forceinline__ void dtFinalize(Scalars* sc, int cur, int nxt) {
-  const double lo = dkeyPosInv(sc->minKey[cur]);
-  const double dtn = sc->dt[cur];
-  const double dt1 = smin(lo, 1.05 * dtn);
-  sc->dt[nxt] = dt1;
-  sc->t[nxt] = sc->t[cur] + dt1;
-  sc->pmax = dkeySignedInv(sc->maxKey[cur]);
-  sc->minKey[nxt] = dkeyPos(DBL_MAX);
-  sc->maxKey[nxt] = dkeySigned(-DBL_MAX);
+// dt_{n+1} = min(CFL minimum, 1.05 dt_n) (VnrRemap.cc:45-50) and the maximum
+// pressure, from the step's accumulators (the same value for every thread
+// that folds them).
+struct DtNow {
+  double dt1, pmax;
+};
+template <class R>
+__device__ __forceinline__ DtNow dtFold(const FieldsT<R>& f, int cur) {
+  unsigned long long lo = f.keys->k[cur][0][0], hi = f.keys->k[cur][0][1];
+#pragma unroll
+  for (int s = 1; s < kDtSlots; ++s) {
+    const unsigned long long a = f.keys->k[cur][s][0], b = f.keys->k[cur][s][1];
+    lo = (a < lo) ? a : lo;
+    hi = (b > hi) ? b : hi;
+  }
+  return {smin(dkeyPosInv(lo), 1.05 * f.sc->dt[cur]), dkeySignedInv(hi)};
+}
+// stores dt_{n+1}, t_{n+1} (computeTime) and the maximum pressure and resets
+// the accumulators of the next step's parity (one thread)
+template <class R>
+__device__ __forceinline__ void dtStore(const FieldsT<R>& f, int cur, int nxt, DtNow d) {
+  Scalars* sc = f.sc;
+  sc->dt[nxt] = d.dt1;
+  sc->t[nxt] = sc->t[cur] + d.dt1;
+  sc->pmax = d.pmax;
+#pragma unroll
+  for (int s = 0; s < kDtSlots; ++s) {
+    f.keys->k[nxt][s][0] = dkeyPos(DBL_MAX);
+    f.keys->k[nxt][s][1] = dkeySigned(-DBL_MAX);
+  }
+}
+// dt_{n+1} for the node update; first: the one thread that stores it.  The
+// step's other kernels come later and read the stored value.
+template <class R>
+__device__ __forceinline__ double dtForNodes(const KPT<R>& kp, bool first) {
+  if (!kp.dtFold) return kp.f.sc->dt[kp.nxt];
+  const DtNow d = dtFold(kp.f, kp.cur);
+  if (first) dtStore(kp.f, kp.cur, kp.nxt, d);
+  return d.dt1;
 }
 
 template <class R>
 __global__ void k_dt_finalize(KPT<R> kp) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) dtFinalize(kp.f.sc, kp.cur, kp.nxt);
+  if (threadIdx.x == 0 && blockIdx.x == 0) dtStore(kp.f, kp.cur, kp.nxt, dtFold(kp.f, kp.cur));
 }
 
 // sansLagrange: deltat_nplus1 = deltat_n (VnrRemap.cc:143-146)
@@ -122,7 +150,7 @@ __global__ void k_dt_hold(KPT<R> kp) {
 // is carried over unchanged (VnrRemap.cc:152-154).  Arithmetic is FP64 in
 // both forms.
 template <class R>
-__device__ __forceinline__ void lagrangeNodeAt(const KPT<R>& kp, long p, long j, long i) {
+__device__ __forceinline__ void lagrangeNodeAt(const KPT<R>& kp, double dt1, long p, long j, long i) {
   const Opts& o = kp.o;
   const auto& f = kp.f;
   const long nx = o.nx, ny = o.ny;
@@ -141,9 +169,7 @@ __device__ __forceinline__ void lagrangeNodeAt(const KPT<R>& kp, long p, long j,
     f.uy[kp.nxt][p] = uyn;
     return;
   }
-  const Scalars* sc = f.sc;
-  const double dt1 = sc->dt[kp.nxt], dtn = sc->dt[kp.cur];
-  const double dt = 0.5 * (dt1 + dtn);
+  const double dt = 0.5 * (dt1 + f.sc->dt[kp.cur]);
   // corner normals of the four cells at this node: C(cell, node) depends on
   // the node and its two neighbours along the cell's edges
   const D2 X0 = nodeX(kp, j, i);
@@ -206,35 +232,14 @@ __device__ __forceinline__ void lagrangeNodeAt(const KPT<R>& kp, long p, long j,
   }
 }
 
+// Interior node (j, i) of the fixed Euler grid (MODE_FULL): the four cells
+// exist and the corner normals are the raw half-edge sums.  The same operands
+// in the same order as lagrangeNodeAt, so the results are bitwise its own.
 template <class R>
-__device__ __forceinline__ void lagrangeNodeBody(const KPT<R>& kp, unsigned b) {
-  const long p = (long)b * blockDim.x + threadIdx.x;
-  if (p >= kp.nnode) return;
-  const long nx = kp.o.nx;
-  const long j = (long)((unsigned)p / (unsigned)(nx + 1)), i = p - j * (nx + 1);
-  lagrangeNodeAt(kp, p, j, i);
-}
-
-template <class R>
-__global__ __launch_bounds__(256) void k_lagrange_node(KPT<R> kp) {
-  lagrangeNodeBody(kp, blockIdx.x);
-}
-
-// The same node update split by position, for the fixed Euler grid
-// (MODE_FULL): the interior nodes, whose four cells all exist and whose
-// corner normals are the raw half-edge sums, run in a kernel of their own
-// (blockIdx.y = node row, no index division, few registers); the boundary
-// nodes, with their conditions, run the general body above.  Each node is
-// updated by exactly one of the two, from the same operands in the same
-// order, so the results are bitwise those of k_lagrange_node.
-template <class R>
-__global__ __launch_bounds__(256) void k_lagrange_node_inner(KPT<R> kp) {
+__device__ __forceinline__ void lagrangeNodeInner(const KPT<R>& kp, double dt1, int j, int i) {
   const Opts& o = kp.o;
   const auto& f = kp.f;
   const int nx = o.nx;
-  const int i = 1 + (int)(blockIdx.x * blockDim.x + threadIdx.x);
-  const int j = 1 + (int)blockIdx.y;
-  if (i >= nx) return;
   const int p = j * (nx + 1) + i;
   const int c0 = j * nx + i;  // cells (j, i), (j, i-1), (j-1, i), (j-1, i-1)
   const int cc[4] = {c0, c0 - 1, c0 - nx, c0 - nx - 1};
@@ -244,9 +249,7 @@ __global__ __launch_bounds__(256) void k_lagrange_node_inner(KPT<R> kp) {
   const double Mp = msum / 4.0;
   f.Mp[p] = Mp;
   const double uxn = (double)f.ux[kp.cur][p], uyn = (double)f.uy[kp.cur][p];
-  const Scalars* sc = f.sc;
-  const double dt1 = sc->dt[kp.nxt], dtn = sc->dt[kp.cur];
-  const double dt = 0.5 * (dt1 + dtn);
+  const double dt = 0.5 * (dt1 + f.sc->dt[kp.cur]);
   const D2 X0 = eulerNode(o, j, i);
   const D2 Cn[4] = {lpcNpcAxis(X0, eulerNode(o, j, i + 1), eulerNode(o, j + 1, i)),
                     lpcNpcAxis(X0, eulerNode(o, j + 1, i), eulerNode(o, j, i - 1)),
@@ -263,13 +266,43 @@ __global__ __launch_bounds__(256) void k_lagrange_node_inner(KPT<R> kp) {
   f.uy[kp.nxt][p] = u1.y;
 }
 
-// the boundary nodes: bottom row, top row, then the left and right columns
-// without their corners
+// One thread per node, any mode (b: block index inside the problem).
 template <class R>
-__global__ __launch_bounds__(256) void k_lagrange_node_edge(KPT<R> kp) {
+__device__ __forceinline__ void lagrangeNodeBody(const KPT<R>& kp, unsigned b) {
+  const double dt1 = dtForNodes(kp, b == 0 && threadIdx.x == 0);
+  const long p = (long)b * blockDim.x + threadIdx.x;
+  if (p >= kp.nnode) return;
   const long nx = kp.o.nx, ny = kp.o.ny;
-  const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  long j, i;
+  const long j = (long)((unsigned)p / (unsigned)(nx + 1)), i = p - j * (nx + 1);
+  if (kp.o.mode == MODE_FULL && i > 0 && j > 0 && i < nx && j < ny) lagrangeNodeInner(kp, dt1, (int)j, (int)i);
+  else lagrangeNodeAt(kp, dt1, p, j, i);
+}
+
+template <class R>
+__global__ __launch_bounds__(256) void k_lagrange_node(KPT<R> kp) {
+  lagrangeNodeBody(kp, blockIdx.x);
+}
+
+// The node update on the fixed Euler grid, laid out by position: blockIdx.y
+// < ny - 1 is one row of interior nodes (no index division, one test per
+// thread); the rows of blocks after them share the boundary nodes (bottom
+// row, top row, then the left and right columns without their corners), which
+// run the general body with its conditions.  One launch for both: as kernels of
+// their own the boundary nodes took 5 to 7 us on any mesh, and the time-step
+// finalize another 2 to 5 us; folded in here they overlap the interior rows
+// (one step of 256^2 cells 60.8 -> 55.8 us, of 500 x 333 cells with PenteBorne
+// 112 -> 103 us, the accumulators in lines of their own included).
+template <class R>
+__global__ __launch_bounds__(256) void k_lagrange_node_euler(KPT<R> kp) {
+  const int nx = kp.o.nx, ny = kp.o.ny;
+  const double dt1 = dtForNodes(kp, blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0);
+  if ((int)blockIdx.y < ny - 1) {
+    const int i = 1 + (int)(blockIdx.x * blockDim.x + threadIdx.x);
+    if (i < nx) lagrangeNodeInner(kp, dt1, 1 + (int)blockIdx.y, i);
+    return;
+  }
+  const int e = (((int)blockIdx.y - (ny - 1)) * (int)gridDim.x + (int)blockIdx.x) * 256 + (int)threadIdx.x;
+  int j, i;
   if (e < nx + 1) {
     j = 0, i = e;
   } else if (e < 2 * (nx + 1)) {
@@ -281,7 +314,7 @@ __global__ __launch_bounds__(256) void k_lagrange_node_edge(KPT<R> kp) {
   } else {
     return;
   }
-  lagrangeNodeAt(kp, j * (nx + 1) + i, j, i);
+  lagrangeNodeAt(kp, dt1, (long)j * (nx + 1) + i, j, i);
 }
 
 // Cell kernel: the cell part of the Lagrange phase (lagrangeCellCompute,
@@ -325,14 +358,6 @@ __global__ __launch_bounds__(256) void k_dt_reduce_batch(BatchLaunchT<R> bl) {
     __syncthreads();  // the shared scratch is reused by the next virtual block
   });
 }
-// one thread per problem
-template <class R>
-__global__ __launch_bounds__(256) void k_dt_finalize_batch(BatchLaunchT<R> bl) {
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= bl.nprob) return;
-  const KPT<R>& kp = bl.table[bl.variant * bl.nprob + p];
-  dtFinalize(kp.f.sc, kp.cur, kp.nxt);
-}
 template <class R, bool ONE>
 __global__ __launch_bounds__(256) void k_lagrange_node_batch(BatchLaunchT<R> bl) {
   batchRun<ONE>(bl, [&](const KPT<R>& kp, unsigned b, unsigned, unsigned) { lagrangeNodeBody(kp, b); });
@@ -351,11 +376,9 @@ __global__ __launch_bounds__(256) void k_lagrange_cell_batch(BatchLaunchT<R> bl)
 #define MHY_LAGRANGE_INST(R)                                                 \
   template __global__ void k_dt_reduce<R>(KPT<R>);                           \
   template __global__ void k_dt_finalize<R>(KPT<R>);                         \
-  template __global__ void k_dt_finalize_batch<R>(BatchLaunchT<R>);          \
   template __global__ void k_dt_hold<R>(KPT<R>);                             \
   template __global__ void k_lagrange_node<R>(KPT<R>);                       \
-  template __global__ void k_lagrange_node_inner<R>(KPT<R>);                 \
-  template __global__ void k_lagrange_node_edge<R>(KPT<R>);                  \
+  template __global__ void k_lagrange_node_euler<R>(KPT<R>);                 \
   template __global__ void k_lagrange_cell<R, 1>(KPT<R>);                    \
   template __global__ void k_lagrange_cell<R, 2>(KPT<R>);                    \
   template __global__ void k_lagrange_cell<R, 3>(KPT<R>);                    \
