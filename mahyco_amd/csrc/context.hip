@@ -92,6 +92,10 @@ struct mhy_ctx {
   // MAHYCO_FUSE_FINAL=0 keeps it a separate kernel); finalDone records that
   // the current iteration's final remap is already done
   bool fuseFinal = true, finalDone = false;
+  // the limiter of the sweeps compiled for this context's options
+  // (fixedLimiter), or 0: the sweeps that read their options at run time
+  // (MAHYCO_FIXED_OPTIONS=0 forces those)
+  int fixLim = 0;
   // whole steps: the node update folds the dt accumulators itself; the
   // phase-level calls launch a finalize kernel in the dt phase instead
   bool dtFold = false;
@@ -444,8 +448,8 @@ int phaseEucFinal(mhy_ctx* x) {
 template <int L>
 EucSweepFn eucSweepFor(bool xd, bool pp, bool o3) {
   if (o3) return xd ? k_sweep_o3<double, L, true> : k_sweep_o3<double, L, false>;
-  if (pp) return xd ? k_sweep_wave<double, L, true, true> : k_sweep_wave<double, L, true, false>;
-  return xd ? k_sweep_wave<double, L, false, true> : k_sweep_wave<double, L, false, false>;
+  if (pp) return xd ? k_sweep_wave<double, L, true, true, RunOpts> : k_sweep_wave<double, L, true, false, RunOpts>;
+  return xd ? k_sweep_wave<double, L, false, true, RunOpts> : k_sweep_wave<double, L, false, false, RunOpts>;
 }
 EucSweepFn eucSweepKernel(bool xd, int m, bool pp, bool conservative, bool o3) {
   switch (m + (conservative ? 8 : 4)) {
@@ -467,7 +471,11 @@ int phaseEucSweep(mhy_ctx* x, int sweep, int stage) {
   const bool o3 = (x->o.order == 3), pp = (x->o.pp == 1);
   const dim3 grid = o3 ? sweepO3Grid(xd, x->o.nx, x->o.ny) : sweepWaveGrid(xd, x->o.nx, x->o.ny, false, pp);
   const dim3 block(o3 ? kBlock : sweepWaveBlock(xd, false, pp));
-  const EucSweepFn k = eucSweepKernel(xd, x->o.nbmat, pp, x->o.conservative == 1, o3);
+  const Opts& o = x->o;
+  const bool fixedForm = x->fixLim == MHY_LIM_SUPERBEE && pp && o.conservative == 0 &&
+                         (o.pp_mixte != 1 || o.limiter_pure == MHY_LIM_ARITHMETICG);
+  const EucSweepFn k = fixedForm ? sweepFixedEuc(xd, o.nbmat, o.pp_mixte == 1, sweep)
+                                 : eucSweepKernel(xd, o.nbmat, pp, o.conservative == 1, o3);
   timed(x, xd ? K_SWEEP_X : K_SWEEP_Y, [&] { hipLaunchKernelGGL(k, grid, block, 0, x->stream, kp); });
   return checkLaunch(x, "eucclhyd sweep");
 }
@@ -521,30 +529,55 @@ int phaseLagrange(mhy_ctx* x) {
 }
 
 // sweep kernels for the direction, the material count and the PenteBorne
-// option: the wave-shuffle kernels (default) or the per-cell stencil kernels
-// (FP64 form only)
+// option, with their options at run time: the wave-shuffle kernels (default),
+// the fused and walking ones, or the per-cell stencil kernels (FP64 form only)
 template <class R>
-void (*sweepWaveKernel(bool xd, int m, bool pp, bool lag = false))(KPT<R>) {
-  using Fn = void (*)(KPT<R>);
-  static const Fn kl[2][3][2] = {
-      {{k_sweep_wave_lag<R, 1, false, false>, k_sweep_wave_lag<R, 1, true, false>},
-       {k_sweep_wave_lag<R, 2, false, false>, k_sweep_wave_lag<R, 2, true, false>},
-       {k_sweep_wave_lag<R, 3, false, false>, k_sweep_wave_lag<R, 3, true, false>}},
-      {{k_sweep_wave_lag<R, 1, false, true>, k_sweep_wave_lag<R, 1, true, true>},
-       {k_sweep_wave_lag<R, 2, false, true>, k_sweep_wave_lag<R, 2, true, true>},
-       {k_sweep_wave_lag<R, 3, false, true>, k_sweep_wave_lag<R, 3, true, true>}}};
-  if (lag) return kl[xd ? 1 : 0][m - 1][pp ? 1 : 0];
-  static const Fn kw[2][3][2] = {
-      {{k_sweep_wave<R, 1, false, false>, k_sweep_wave<R, 1, true, false>},
-       {k_sweep_wave<R, 2, false, false>, k_sweep_wave<R, 2, true, false>},
-       {k_sweep_wave<R, 3, false, false>, k_sweep_wave<R, 3, true, false>}},
-      {{k_sweep_wave<R, 1, false, true>, k_sweep_wave<R, 1, true, true>},
-       {k_sweep_wave<R, 2, false, true>, k_sweep_wave<R, 2, true, true>},
-       {k_sweep_wave<R, 3, false, true>, k_sweep_wave<R, 3, true, true>}}};
+SweepFn<R> sweepWaveKernel(bool xd, int m, bool pp) {
+  static const SweepFn<R> kw[2][3][2] = {
+      {{k_sweep_wave<R, 1, false, false, RunOpts>, k_sweep_wave<R, 1, true, false, RunOpts>},
+       {k_sweep_wave<R, 2, false, false, RunOpts>, k_sweep_wave<R, 2, true, false, RunOpts>},
+       {k_sweep_wave<R, 3, false, false, RunOpts>, k_sweep_wave<R, 3, true, false, RunOpts>}},
+      {{k_sweep_wave<R, 1, false, true, RunOpts>, k_sweep_wave<R, 1, true, true, RunOpts>},
+       {k_sweep_wave<R, 2, false, true, RunOpts>, k_sweep_wave<R, 2, true, true, RunOpts>},
+       {k_sweep_wave<R, 3, false, true, RunOpts>, k_sweep_wave<R, 3, true, true, RunOpts>}}};
   return kw[xd ? 1 : 0][m - 1][pp ? 1 : 0];
 }
-KernelFn sweepKernel(bool wave, bool xd, int m, bool pp) {
-  if (wave) return sweepWaveKernel<double>(xd, m, pp);
+// the first sweep with the fused Lagrange update
+template <class R>
+SweepFn<R> lagSweepKernel(bool xd, int m) {
+  static const SweepFn<R> kl[2][3] = {
+      {k_sweep_wave_lag<R, 1, false, RunOpts>, k_sweep_wave_lag<R, 2, false, RunOpts>,
+       k_sweep_wave_lag<R, 3, false, RunOpts>},
+      {k_sweep_wave_lag<R, 1, true, RunOpts>, k_sweep_wave_lag<R, 2, true, RunOpts>,
+       k_sweep_wave_lag<R, 3, true, RunOpts>}};
+  return kl[xd ? 1 : 0][m - 1];
+}
+// column-walking y sweep
+template <class R>
+SweepFn<R> walkKernel(int m, bool pp) {
+  static const SweepFn<R> kk[3][2] = {{k_sweep_walk<R, 1, false, RunOpts>, k_sweep_walk<R, 1, true, RunOpts>},
+                                      {k_sweep_walk<R, 2, false, RunOpts>, k_sweep_walk<R, 2, true, RunOpts>},
+                                      {k_sweep_walk<R, 3, false, RunOpts>, k_sweep_walk<R, 3, true, RunOpts>}};
+  return kk[m - 1][pp ? 1 : 0];
+}
+// the sweep compiled for a limiter's fixed options (lim from fixedLimiter), or
+// null where there is none: mixed-form PenteBorne, the PenteBorne mixte
+// option, walking PenteBorne sweeps, and a second sweep without the final
+// remap (lag: with the fused Lagrange update)
+template <class R>
+SweepFn<R> fixedKernel(const mhy_ctx* x, const KP& kp, bool xd, bool lag, bool walk) {
+  const int lim = x->fixLim, m = x->o.nbmat;
+  if (lim == 0 || !kp.geomLoad || (kp.sweep == 2 && !kp.fuseFinal)) return nullptr;
+  const int kind = lag ? 0 : kp.sweep;
+  if (x->o.pp == 1) {
+    if constexpr (kMixed<R>) return nullptr;
+    else return (x->o.pp_mixte == 1 || walk) ? nullptr : sweepFixedPP(xd, lim, m, kind);
+  }
+  if (walk) return sweepFixedWalk<R>(lim, m, kind);
+  return xd ? sweepFixedX<R>(lim, m, kind) : sweepFixedY<R>(lim, m, kind);
+}
+// the per-cell stencil kernels
+KernelFn sweepKernel(bool xd, int m, bool pp) {
   static const KernelFn kc[2][3][2] = {
       {{k_sweep_cell<1, false, false>, k_sweep_cell<1, true, false>},
        {k_sweep_cell<2, false, false>, k_sweep_cell<2, true, false>},
@@ -576,17 +609,18 @@ int phaseSweepStage(mhy_ctx* x, int sweep, int stage) {
                            : gridFor(x->ncell);
     const dim3 block(wave ? sweepWaveBlock(xd, x->mixed, x->o.pp == 1) : kBlock);
     const bool lagSweep = (sweep == 1 && lagFused(x));
-    if (!xd && wave && x->walkY && !lagSweep) {
-      static const KernelFn kd[3][2] = {{k_sweep_walk<double, 1, false>, k_sweep_walk<double, 1, true>},
-                                        {k_sweep_walk<double, 2, false>, k_sweep_walk<double, 2, true>},
-                                        {k_sweep_walk<double, 3, false>, k_sweep_walk<double, 3, true>}};
-      static const KernelFnF kf[3][2] = {{k_sweep_walk<float, 1, false>, k_sweep_walk<float, 1, true>},
-                                         {k_sweep_walk<float, 2, false>, k_sweep_walk<float, 2, true>},
-                                         {k_sweep_walk<float, 3, false>, k_sweep_walk<float, 3, true>}};
-      const int mi = x->o.nbmat - 1, pi = x->o.pp == 1 ? 1 : 0;
-      timed(x, K_SWEEP_Y, [&] {
-        launchR(x, kd[mi][pi], kf[mi][pi], sweepWalkGrid(x->o.nx, x->o.ny), dim3(kBlock), kp);
-      });
+    const bool walk = !xd && wave && x->walkY && !lagSweep;
+    const KernelId kid = lagSweep ? (xd ? K_LAGSWEEP_X : K_LAGSWEEP_Y) : (xd ? K_SWEEP_X : K_SWEEP_Y);
+    const int m = x->o.nbmat;
+    const bool pp = x->o.pp == 1;
+    // each form's kernel with fixed options, else the run-time one
+    auto launchForm = [&](SweepFn<double> runD, SweepFn<float> runF, dim3 g, dim3 b) {
+      const SweepFn<double> fd = x->mixed ? nullptr : fixedKernel<double>(x, kp, xd, lagSweep, walk);
+      const SweepFn<float> ff = x->mixed ? fixedKernel<float>(x, kp, xd, lagSweep, walk) : nullptr;
+      timed(x, kid, [&] { launchR(x, fd ? fd : runD, ff ? ff : runF, g, b, kp); });
+    };
+    if (walk) {
+      launchForm(walkKernel<double>(m, pp), walkKernel<float>(m, pp), sweepWalkGrid(x->o.nx, x->o.ny), dim3(kBlock));
     } else if (o3) {  // third order: LDS-tile kernel, no PenteBorne (checked at creation)
       static const KernelFn kd[2][3] = {
           {k_sweep_o3<double, 1, false>, k_sweep_o3<double, 2, false>, k_sweep_o3<double, 3, false>},
@@ -597,21 +631,12 @@ int phaseSweepStage(mhy_ctx* x, int sweep, int stage) {
       const int di = xd ? 1 : 0, mi = x->o.nbmat - 1;
       timed(x, xd ? K_SWEEP_X : K_SWEEP_Y, [&] { launchR(x, kd[di][mi], kf[di][mi], grid, block, kp); });
     } else if (lagSweep) {  // with the cell part of the Lagrange phase
-      const KernelId kid = xd ? K_LAGSWEEP_X : K_LAGSWEEP_Y;
-      if (x->mixed) {
-        const KernelFnF k = sweepWaveKernel<float>(xd, x->o.nbmat, x->o.pp == 1, true);
-        timed(x, kid, [&] { hipLaunchKernelGGL(k, grid, block, 0, x->stream, retype<float>(kp)); });
-      } else {
-        const KernelFn k = sweepWaveKernel<double>(xd, x->o.nbmat, x->o.pp == 1, true);
-        timed(x, kid, [&] { hipLaunchKernelGGL(k, grid, block, 0, x->stream, kp); });
-      }
-    } else if (x->mixed) {
-      const KernelFnF k = sweepWaveKernel<float>(xd, x->o.nbmat, x->o.pp == 1);
-      timed(x, xd ? K_SWEEP_X : K_SWEEP_Y,
-            [&] { hipLaunchKernelGGL(k, grid, block, 0, x->stream, retype<float>(kp)); });
+      launchForm(lagSweepKernel<double>(xd, m), lagSweepKernel<float>(xd, m), grid, block);
+    } else if (wave) {
+      launchForm(sweepWaveKernel<double>(xd, m, pp), sweepWaveKernel<float>(xd, m, pp), grid, block);
     } else {
-      const KernelFn k = sweepKernel(wave, xd, x->o.nbmat, x->o.pp == 1);
-      timed(x, xd ? K_SWEEP_X : K_SWEEP_Y, [&] { hipLaunchKernelGGL(k, grid, block, 0, x->stream, kp); });
+      const KernelFn k = sweepKernel(xd, m, pp);
+      timed(x, kid, [&] { hipLaunchKernelGGL(k, grid, block, 0, x->stream, kp); });
     }
   } else if (x->sweepWave && xd) {
     const dim3 grid = dualWaveGrid(true, x->o.nx, x->o.ny, x->mixed);
@@ -803,6 +828,12 @@ extern "C" {
 
 const char* mhy_last_error(const mhy_ctx* x) { return x ? x->err.c_str() : "null context"; }
 
+// the limiter of the fixed-option sweeps of these options, or 0
+static int pickFixed(const Opts& o) {
+  const char* fx = std::getenv("MAHYCO_FIXED_OPTIONS");
+  return (fx && std::string(fx) == "0") ? 0 : fixedLimiter(o);
+}
+
 // Set-up of an Eucclhyd problem (Eucclhyd::simulate prologue,
 // eucclhyd_remap/EucclhydRemap.cc:273-286): options, initial state on the
 // host, device arrays (FP64), upload.  Returns MHY_OK or the failure code
@@ -858,6 +889,7 @@ static int setupEucclhyd(mhy_ctx* x, const mhy_config& c, bool batchMember) {
     o.bcv_left[d] = b.vleft[d], o.bcv_right[d] = b.vright[d], o.bcv_bottom[d] = b.vbottom[d], o.bcv_top[d] = b.vtop[d];
   o.flux_left = b.flux_left, o.flux_right = b.flux_right, o.flux_bottom = b.flux_bottom, o.flux_top = b.flux_top;
   o.flux_any = (b.flux_left + b.flux_right + b.flux_bottom + b.flux_top) > 0;
+  x->fixLim = pickFixed(o);
 
   hipError_t e = hipSuccess;
   if ((e = hipGetDevice(&x->device)) != hipSuccess) return fail(x, MHY_ERR_DEVICE, hipGetErrorString(e));
@@ -1087,6 +1119,7 @@ static int createContext(const mhy_config* cfg, mhy_ctx** out, bool batchMember)
   o.periodic_right = b.periodic_right;
   o.flux_left = b.flux_left, o.flux_right = b.flux_right, o.flux_bottom = b.flux_bottom, o.flux_top = b.flux_top;
   o.flux_any = (b.flux_left + b.flux_right + b.flux_bottom + b.flux_top) > 0;
+  x->fixLim = pickFixed(o);
   // one perfect-gas material, Lagrange + remap: the final remap stores the
   // material fields only where they differ from the means (MAHYCO_COMPACT=0
   // stores them everywhere, as for several materials)
@@ -1733,12 +1766,12 @@ template <class R, bool ONE>
 void (*sweepBatchKernel(bool xd, int m, bool pp))(BatchLaunchT<R>) {
   using Fn = void (*)(BatchLaunchT<R>);
   static const Fn t[2][3][2] = {
-      {{k_sweep_wave_batch<R, 1, false, false, ONE>, k_sweep_wave_batch<R, 1, true, false, ONE>},
-       {k_sweep_wave_batch<R, 2, false, false, ONE>, k_sweep_wave_batch<R, 2, true, false, ONE>},
-       {k_sweep_wave_batch<R, 3, false, false, ONE>, k_sweep_wave_batch<R, 3, true, false, ONE>}},
-      {{k_sweep_wave_batch<R, 1, false, true, ONE>, k_sweep_wave_batch<R, 1, true, true, ONE>},
-       {k_sweep_wave_batch<R, 2, false, true, ONE>, k_sweep_wave_batch<R, 2, true, true, ONE>},
-       {k_sweep_wave_batch<R, 3, false, true, ONE>, k_sweep_wave_batch<R, 3, true, true, ONE>}}};
+      {{k_sweep_wave_batch<R, 1, false, false, ONE, RunOpts>, k_sweep_wave_batch<R, 1, true, false, ONE, RunOpts>},
+       {k_sweep_wave_batch<R, 2, false, false, ONE, RunOpts>, k_sweep_wave_batch<R, 2, true, false, ONE, RunOpts>},
+       {k_sweep_wave_batch<R, 3, false, false, ONE, RunOpts>, k_sweep_wave_batch<R, 3, true, false, ONE, RunOpts>}},
+      {{k_sweep_wave_batch<R, 1, false, true, ONE, RunOpts>, k_sweep_wave_batch<R, 1, true, true, ONE, RunOpts>},
+       {k_sweep_wave_batch<R, 2, false, true, ONE, RunOpts>, k_sweep_wave_batch<R, 2, true, true, ONE, RunOpts>},
+       {k_sweep_wave_batch<R, 3, false, true, ONE, RunOpts>, k_sweep_wave_batch<R, 3, true, true, ONE, RunOpts>}}};
   return t[xd ? 1 : 0][m - 1][pp ? 1 : 0];
 }
 template <class R, bool ONE>
@@ -1768,6 +1801,7 @@ struct mhy_batch {
   bool dualWaveY = true;  // nodal remap along y with the wave kernel
   bool walkY = false;     // cell sweeps along y with the column-walking kernel
   bool o3 = false;        // third-order remap (LDS-tile cell sweeps)
+  int fixLim = 0;         // every problem has this fixed limiter (fixedLimiter), or 0
   void* dTable = nullptr;  // KPT<double> or KPT<float> entries
   unsigned* dStart = nullptr;  // BK_COUNT x (n+1)
   unsigned* dGx = nullptr;     // BK_COUNT x n
@@ -1802,10 +1836,11 @@ int batchEnqueueStepR(mhy_batch* b, int cur, bool xty, bool timing) {
   // fnLoop walks contiguous virtual-block ranges (blocks[k] workgroups);
   // fnOne runs one workgroup per virtual block (blocks[k] == 0)
   using Fn = void (*)(BatchLaunchT<R>);
+  // (null fnLoop: one workgroup per virtual block whatever blocks[k])
   auto launch = [&](int k, Fn fnLoop, Fn fnOne, int variant, unsigned block = kBlock) {
     BatchLaunchT<R> bl{static_cast<const KPT<R>*>(b->dTable), b->dStart + (size_t)k * (n + 1),
                        b->dGx + (size_t)k * n, n, variant, b->total[k], b->dOwner + b->ownerOff[k]};
-    const bool one = b->blocks[k] == 0 || b->blocks[k] >= b->total[k];
+    const bool one = !fnLoop || b->blocks[k] == 0 || b->blocks[k] >= b->total[k];
     const unsigned grid = one ? b->total[k] : b->blocks[k];
     const Fn fn = one ? fnOne : fnLoop;
     if (timing) (void)hipEventRecord(b->ev[2 * k], b->stream);
@@ -1825,6 +1860,10 @@ int batchEnqueueStepR(mhy_batch* b, int cur, bool xty, bool timing) {
     const int v = cur + 2 * (sweep - 1) + 4 * (xd ? 1 : 0);
     if (b->o3)
       launch(xd ? BK_SWX : BK_SWY, o3BatchKernel<R, false>(xd, b->m), o3BatchKernel<R, true>(xd, b->m), v + 8 * fuse);
+    else if (b->fixLim && !(!xd && b->walkY))
+      launch(xd ? BK_SWX : BK_SWY, nullptr,
+             xd ? sweepFixedXBatch<R>(b->fixLim, b->m, sweep) : sweepFixedYBatch<R>(b->fixLim, b->m, sweep),
+             v + 8 * fuse, sweepWaveBlock(xd, b->mixed, b->pp));
     else if (!xd && b->walkY)
       launch(BK_SWY, walkBatchKernel<R, false>(b->m, b->pp), walkBatchKernel<R, true>(b->m, b->pp), v + 8 * fuse);
     else
@@ -1907,6 +1946,9 @@ int mhy_batch_create(const mhy_config* cfgs, int n, mhy_batch** out) {
     b->ctx[i]->sweepWave = true;
     b->ctx[i]->fuseFinal = true;
     b->cells += b->ctx[i]->ncell;
+    // (kind 1 and 2 of the limited-slope sweeps, one limiter for all)
+    const int lim = (b->pp || b->o3) ? 0 : b->ctx[i]->fixLim;
+    b->fixLim = (i == 0 || b->fixLim == lim) ? lim : 0;
   }
   b->cur0 = b->cur = b->ctx[0]->cur;
   b->xty0 = b->xty = b->ctx[0]->x_then_y_n;

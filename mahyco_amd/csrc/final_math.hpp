@@ -4,7 +4,7 @@
 // the second remap sweep, which finishes each cell from its registers.
 #pragma once
 
-#include "common.hpp"
+#include "options.hpp"
 
 namespace mhy {
 
@@ -27,7 +27,7 @@ struct FinalOut {
 // material's mass and energy content can lie below the FP32 range).  The
 // mixed form (R = float) takes the EOS sound speeds' square roots in FP32,
 // the precision they are stored in.
-template <class R, int M>
+template <class R, int M, class P = RunOpts>
 __device__ __forceinline__ void finalCompute(const KPT<R>& kp, long c, const double* U, FinalOut<R, M>& out) {
   const Opts& o = kp.o;
   const auto& f = kp.f;
@@ -110,10 +110,10 @@ __device__ __forceinline__ void finalCompute(const KPT<R>& kp, long c, const dou
 #pragma unroll
   for (int k = 0; k < M; ++k) {
     const double g = o.gammap[k];
-    if (o.eos[k] == MHY_EOS_PERFECT_GAS) {
+    if (P::eos(o, k) == MHY_EOS_PERFECT_GAS) {
       pk[k] = (g - 1.0) * rk[k] * ek[k];
       ck[k] = kMixed<R> ? (double)sqrtf(float(g * (g - 1.0) * ek[k])) : sqrt(g * (g - 1.0) * ek[k]);
-    } else if (o.eos[k] == MHY_EOS_VOID) {
+    } else if (P::eos(o, k) == MHY_EOS_VOID) {
       pk[k] = (double)at(f.p_k[cur][k], c);
       ck[k] = (double)at(f.c_k[cur][k], c);
       ek[k] = (double)at(f.e_k[cur][k], c);
@@ -138,7 +138,7 @@ __device__ __forceinline__ void finalCompute(const KPT<R>& kp, long c, const dou
   }
 #pragma unroll
   for (int k = 0; k < M; ++k)
-    if (o.eos[k] == MHY_EOS_VOID) e1 += mu[k] * ek[k];
+    if (P::eos(o, k) == MHY_EOS_VOID) e1 += mu[k] * ek[k];
   out.rho = (R)rho1;
   out.e = (R)e1;
   out.q = (R)q1;
@@ -195,10 +195,10 @@ __device__ __forceinline__ void finalStore(const KPT<R>& kp, long c, const Final
   }
 }
 
-template <class R, int M>
+template <class R, int M, class P = RunOpts>
 __device__ __forceinline__ void finalCell(const KPT<R>& kp, long c, const double* U) {
   FinalOut<R, M> out;
-  finalCompute<R, M>(kp, c, U, out);
+  finalCompute<R, M, P>(kp, c, U, out);
   finalStore<R, M>(kp, c, out);
 }
 

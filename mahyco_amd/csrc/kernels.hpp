@@ -1,9 +1,9 @@
 // Kernel entry points of the hot path (defined in lagrange.hip,
-// sweep_wave.hip, sweep_cell.hip, remap.hip).  R is the storage type of the
+// sweep_wave.hpp, sweep_walk.hpp, sweep_cell.hip, remap.hip).  R is the storage type of the
 // bulk fields: double (FP64 form) or float (mixed form).
 #pragma once
 
-#include "common.hpp"
+#include "options.hpp"
 
 namespace mhy {
 
@@ -39,7 +39,7 @@ template <class R, bool ONE>
 __global__ void k_lagrange_node_batch(BatchLaunchT<R> bl);
 template <class R, int M, bool ONE>
 __global__ void k_lagrange_cell_batch(BatchLaunchT<R> bl);
-template <class R, int M, bool PP, bool XD, bool ONE>
+template <class R, int M, bool PP, bool XD, bool ONE, class P>
 __global__ void k_sweep_wave_batch(BatchLaunchT<R> bl);
 template <class R, bool XD, bool ONE>
 __global__ void k_dual_wave_batch(BatchLaunchT<R> bl);
@@ -54,15 +54,37 @@ __global__ void k_sweep_o3(KPT<R> kp);
 template <class R, int M, bool XD, bool ONE>
 __global__ void k_sweep_o3_batch(BatchLaunchT<R> bl);
 dim3 sweepO3Grid(bool xd, long nx, long ny);
-template <class R, int M, bool PP, bool XD>
+// P: where the options come from (RunOpts, or FixOpts for the common sets)
+template <class R, int M, bool PP, bool XD, class P>
 __global__ void k_sweep_wave(KPT<R> kp);
-// the first sweep with the cell part of the Lagrange phase fused in
-template <class R, int M, bool PP, bool XD>
+// the first sweep with the cell part of the Lagrange phase fused in (limited slopes)
+template <class R, int M, bool XD, class P>
 __global__ void k_sweep_wave_lag(KPT<R> kp);
+// the sweeps with fixed options for a limiter (fixedLimiter), m materials;
+// kind: 0 fused Lagrange sweep, 1 first sweep, 2 second sweep with the final
+// remap
+template <class R>
+using SweepFn = void (*)(KPT<R>);
+template <class R>
+using SweepBatchFn = void (*)(BatchLaunchT<R>);
+template <class R>
+SweepFn<R> sweepFixedX(int lim, int m, int kind);
+template <class R>
+SweepFn<R> sweepFixedY(int lim, int m, int kind);
+template <class R>
+SweepFn<R> sweepFixedWalk(int lim, int m, int kind);
+template <class R>
+SweepBatchFn<R> sweepFixedXBatch(int lim, int m, int kind);
+template <class R>
+SweepBatchFn<R> sweepFixedYBatch(int lim, int m, int kind);
+// PenteBorne, FP64: VNR without the mixte option; Eucclhyd (superBee,
+// pure-cell limiter arithmeticG with the mixte option)
+SweepFn<double> sweepFixedPP(bool xd, int lim, int m, int kind);
+SweepFn<double> sweepFixedEuc(bool xd, int m, bool mixte, int kind);
 dim3 sweepWaveGrid(bool xd, long nx, long ny, bool mixed, bool pp);
 unsigned sweepWaveBlock(bool xd, bool mixed, bool pp);
 // y sweeps with one lane per column walking down a band of rows
-template <class R, int M, bool PP>
+template <class R, int M, bool PP, class P>
 __global__ void k_sweep_walk(KPT<R> kp);
 template <class R, int M, bool PP, bool ONE>
 __global__ void k_sweep_walk_batch(BatchLaunchT<R> bl);

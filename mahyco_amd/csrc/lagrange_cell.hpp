@@ -23,7 +23,7 @@ namespace mhy {
 // End-of-Lagrange positions of the nodes of cell (j, i), order BL, BR, TR,
 // TL: the moving-mesh coordinates, or the Euler node moved by dt1 * u^{n+1}
 // (updatePosition, PhaseLagrange.cc:203-208).
-template <class R>
+template <class R, class P = RunOpts>
 __device__ __forceinline__ void lagNodes(const KPT<R>& kp, double dt1, long j, long i, D2* X) {
   const Opts& o = kp.o;
   const auto& f = kp.f;
@@ -35,7 +35,7 @@ __device__ __forceinline__ void lagNodes(const KPT<R>& kp, double dt1, long j, l
   const long dp[4] = {0, 1, nx + 2, nx + 1};
 #pragma unroll
   for (int s = 0; s < 4; ++s) {
-    if (o.mode == MODE_LAGRANGE) {
+    if (P::mode(o) == MODE_LAGRANGE) {
       X[s] = {at(f.X[kp.nxt] + dp[s], p0), at(f.Y[kp.nxt] + dp[s], p0)};
     } else {
       const D2 e = eulerNode(o, jj[s], ii[s]);
@@ -95,7 +95,7 @@ struct LagCell {
 // arithmetic), so that mass stays conserved to FP64 round-off whatever the
 // FP32 density storage (periodic cells, whose density is reset to its
 // initial value, keep mu_k V rho).
-template <class R, int M>
+template <class R, int M, class P = RunOpts>
 __device__ __forceinline__ bool lagrangeCellCompute(const KPT<R>& kp, long c, long j, long i, bool store,
                                                     LagCell<M>& out) {
   const Opts& o = kp.o;
@@ -131,7 +131,7 @@ __device__ __forceinline__ bool lagrangeCellCompute(const KPT<R>& kp, long c, lo
     }
   }
   D2 X[4];
-  lagNodes(kp, dt1, j, i, X);
+  lagNodes<R, P>(kp, dt1, j, i, X);
   const double V = lagVolume(X);
 
   double rk1[NMAT];
@@ -141,10 +141,10 @@ __device__ __forceinline__ bool lagrangeCellCompute(const KPT<R>& kp, long c, lo
     // absent materials keep the stale buffer value in the reference; their
     // volume fraction is exactly zero, so the value never contributes
     rk1[k] = (fk[k] > o.threshold) ? Mk0[k] / (fk[k] * V)
-                                   : (o.mode == MODE_FULL ? 0.0 : (double)at(f.rho_k[nxt][k], c));
+                                   : (P::mode(o) == MODE_FULL ? 0.0 : (double)at(f.rho_k[nxt][k], c));
     rho1 += fk[k] * rk1[k];
   }
-  const bool periodicCell = o.periodic_right && (i == 0 || i == nx - 1);
+  const bool periodicCell = P::periodic(o) && (i == 0 || i == nx - 1);
   if (periodicCell) {
     const long L = j * nx;  // updatePeriodicBoundaryConditions
     rho1 = (double)at(f.rho0, L);
@@ -153,7 +153,7 @@ __device__ __forceinline__ bool lagrangeCellCompute(const KPT<R>& kp, long c, lo
   }
 
   double q1 = 0.0, e1 = 0.0;
-  if (o.mode != MODE_ADVECTION) {
+  if (P::mode(o) != MODE_ADVECTION) {
     // mixed form: the step-start densities from the FP64 masses and volume,
     // so that 1/rho1 - 1/rho0 (divided by dt in div u) carries no FP32
     // rounding of the stored density
@@ -166,8 +166,8 @@ __device__ __forceinline__ bool lagrangeCellCompute(const KPT<R>& kp, long c, lo
     } else {
       q1 = 0.0;
     }
-    const double P = sc->pmax;
-    if (q1 > P) q1 = P;
+    const double qmax = sc->pmax;
+    if (q1 > qmax) q1 = qmax;
     double qk1[NMAT], ek1[NMAT], pk1[NMAT], ck1[NMAT];
 #pragma unroll
     for (int k = 0; k < m; ++k) qk1[k] = fk[k] * q1;
@@ -194,10 +194,10 @@ __device__ __forceinline__ bool lagrangeCellCompute(const KPT<R>& kp, long c, lo
 #pragma unroll
     for (int k = 0; k < m; ++k) {
       const double g = o.gammap[k];
-      if (o.eos[k] == MHY_EOS_PERFECT_GAS) {
+      if (P::eos(o, k) == MHY_EOS_PERFECT_GAS) {
         pk1[k] = (g - 1.0) * rk1[k] * ek1[k];
         ck1[k] = sqrt(g * (g - 1.0) * ek1[k]);
-      } else if (o.eos[k] == MHY_EOS_VOID) {
+      } else if (P::eos(o, k) == MHY_EOS_VOID) {
         pk1[k] = pk0[k];
         ck1[k] = at(f.c_k[cur][k], c);
         ek1[k] = ek0[k];
@@ -219,13 +219,13 @@ __device__ __forceinline__ bool lagrangeCellCompute(const KPT<R>& kp, long c, lo
     if (rho1 > 0.) c1 = sqrt(o.gammap[0] * (o.gammap[0] - 1.0) * e1);
 #pragma unroll
     for (int k = 0; k < m; ++k)
-      if (o.eos[k] == MHY_EOS_VOID) e1 += mu0[k] * ek1[k];
+      if (P::eos(o, k) == MHY_EOS_VOID) e1 += mu0[k] * ek1[k];
     if (store) {
       at(f.divu[nxt], c) = div1;
 #pragma unroll
       for (int k = 0; k < m; ++k) at(f.q_k[nxt][k], c) = qk1[k];
     }
-    if (o.mode == MODE_LAGRANGE) {
+    if (P::mode(o) == MODE_LAGRANGE) {
       if (store) {
         at(f.rho[nxt], c) = rho1;
         at(f.q[nxt], c) = q1;

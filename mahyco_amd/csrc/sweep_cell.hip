@@ -253,14 +253,14 @@ __global__ __launch_bounds__(256) void k_sweep_cell(KP kp) {
       const double xf = XD ? 0.5 * (o.dx * (double)b + o.dx * (double)b) : 0.5 * (o.dy * (double)b + o.dy * (double)b);
       const double sx = 0.0 + (xf - u0.xc);
 #pragma unroll
-      for (int q = 0; q < NC; ++q) out[q] = u0.phi[q] + gradQ<XD, double>(o, n, q) * sx;
+      for (int q = 0; q < NC; ++q) out[q] = u0.phi[q] + gradQ<XD, PP, RunOpts, double>(o, n, q) * sx;
     };
     if (hasM) faceValue(a, s[0], s[1], s[2], s[3], in[0], in[1], in[2], in[3], vm, phiM);
     if (hasP) faceValue(a + 1, s[1], s[2], s[3], s[4], in[1], in[2], in[3], in[4], vp, phiP);
   } else if (o.order > 1) {
     // PenteBorne: phi_f = Av(minus cell) - Ar(plus cell) (PhaseRemap1.cc:361-364)
     double Ar0[NC], Av0[NC], Dual[M];
-    ppFluxes<M, XD, double>(o, nbr(s[1], s[2], s[3], in[1], in[3]), vm, vp, dtn, pb, Ar0, Av0, Dual);
+    ppFluxes<M, XD, RunOpts, double>(o, nbr(s[1], s[2], s[3], in[1], in[3]), vm, vp, dtn, pb, Ar0, Av0, Dual);
     if (pb) {
       const double w = (Lm + Lp) * 0.5;
 #pragma unroll
@@ -268,13 +268,13 @@ __global__ __launch_bounds__(256) void k_sweep_cell(KP kp) {
     }
     if (hasM) {
       double ArM[NC], AvM[NC], DM[M];
-      ppFluxes<M, XD, double, false, true>(o, nbr(s[0], s[1], s[2], in[0], in[2]), fnv(a - 1), vm, dtn, false, ArM, AvM, DM);
+      ppFluxes<M, XD, RunOpts, double, false, true>(o, nbr(s[0], s[1], s[2], in[0], in[2]), fnv(a - 1), vm, dtn, false, ArM, AvM, DM);
 #pragma unroll
       for (int q = 0; q < NC; ++q) phiM[q] = AvM[q] - Ar0[q];
     }
     if (hasP) {
       double ArP[NC], AvP[NC], DP[M];
-      ppFluxes<M, XD, double, true, false>(o, nbr(s[2], s[3], s[4], in[2], in[4]), vp, fnv(a + 2), dtn, false, ArP, AvP, DP);
+      ppFluxes<M, XD, RunOpts, double, true, false>(o, nbr(s[2], s[3], s[4], in[2], in[4]), vp, fnv(a + 2), dtn, false, ArP, AvP, DP);
 #pragma unroll
       for (int q = 0; q < NC; ++q) phiP[q] = Av0[q] - ArP[q];
     }
@@ -413,7 +413,7 @@ __device__ __forceinline__ void sweepO3Cell(const KPT<R>& kp, const double* sY, 
     phiM[q] = hasM ? o3Flux(swM, y, e[0], e[1], e[2]) : 0.0;
     phiP[q] = hasP ? o3Flux(swP, y + 1, e[1], e[2], e[3]) : 0.0;
   }
-  sweepUpdateCell<R, L, false, XD, double>(kp, c, i, j, a, hasM, hasP, vm, vp, Lm, Lp, phiM, phiP);
+  sweepUpdateCell<R, L, false, XD, RunOpts, double>(kp, c, i, j, a, hasM, hasP, vm, vp, Lm, Lp, phiM, phiP);
 }
 
 // One tile; blk: its linear block index.  R: bulk storage type.  The face

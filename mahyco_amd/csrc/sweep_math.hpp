@@ -10,7 +10,7 @@
 // face value), vnr_remap/PrepareRemap.cc + remap/PhaseRemap1.cc (Phi forms).
 #pragma once
 
-#include "common.hpp"
+#include "options.hpp"
 
 namespace mhy {
 namespace sw {
@@ -258,21 +258,21 @@ __device__ __forceinline__ T faceDiffP(const Nbr<T>& n, int q) {
 // with the complete option every component (the Eucclhyd momentum and
 // kinetic energy are rescaled from their own integrals), else the volumes,
 // and the masses too in a pure neighbourhood.
-template <int L>
+template <int L, class P>
 __device__ __forceinline__ int ppIntegrated(const Opts& o, bool vp) {
   constexpr int M = kMat<L>;
-  return (o.pp_complet == 1) ? (kEuc<L> ? kNC<L> : 3 * M) : (vp ? 2 * M : M);
+  return P::complet(o) ? (kEuc<L> ? kNC<L> : 3 * M) : (vp ? 2 * M : M);
 }
 
 // Finishing of a PenteBorne flux vector (UtilesRemap-Impl.h:259-313,
 // :436-487): masses and energies from the volume fluxes, the VNR
 // pseudo-viscosity with the volume flux, the Eucclhyd momentum and kinetic
 // energy with the mass flux.
-template <int L, class T>
+template <int L, class P, class T>
 __device__ __forceinline__ void finishPP(const Opts& o, bool pureVariant, const T* phi, T* F) {
   constexpr int NC = kNC<L>;
   constexpr int M = kMat<L>;
-  if (o.pp_complet == 1) {
+  if (P::complet(o)) {
     T sfv = T(0.), sfm = T(0.);
 #pragma unroll
     for (int k = 0; k < M; ++k) sfv += F[k];
@@ -313,12 +313,12 @@ __device__ __forceinline__ void finishPP(const Opts& o, bool pureVariant, const 
 
 // Limited gradient of component q (XD: gradplus is the plus face; along y the
 // reference passes the bottom (minus) face as gradplus, PhaseRemap1.cc:262-265).
-template <bool XD, class T>
+template <bool XD, bool PP, class P, class T>
 __device__ __forceinline__ T gradQ(const Opts& o, const Nbr<T>& n, int q) {
-  if (o.order <= 1) return T(0.0);  // gradients are only formed for order > 1
+  if (P::order(o) <= 1) return T(0.0);  // gradients are only formed for order > 1
   const T gM = n.dM ? n.dM[q] : faceDiffM<XD, T>(n, q);
   const T gP = n.dP ? n.dP[q] : faceDiffP<XD, T>(n, q);
-  const int lim = (o.pp == 1 && n.vp) ? o.limiter_pure : o.limiter;
+  const int lim = (PP && n.vp) ? P::limiterPure(o) : P::limiter(o);
   const T gp = XD ? gP : gM, gm = XD ? gM : gP;
   return limitedGradient<T>(lim, gp, gm, n.phip[q], n.phim[q], n.h0, n.hp, n.hm);
 }
@@ -327,12 +327,12 @@ __device__ __forceinline__ T gradQ(const Opts& o, const Nbr<T>& n, int q) {
 // plus face (Av, type 1), and the dual flux (PB) of the mass components.
 // vminus / vplus: normal velocities of the minus / plus faces.  WANT_AR /
 // WANT_AV select the face fluxes the caller uses (the other stays zero).
-template <int L, bool XD, class T, bool WANT_AR = true, bool WANT_AV = true>
+template <int L, bool XD, class P, class T, bool WANT_AR = true, bool WANT_AV = true>
 __device__ __forceinline__ void ppFluxes(const Opts& o, const Nbr<T>& n, T vminus, T vplus, T dtn, bool dual, T* Ar,
                                          T* Av, T* Dual) {
   constexpr int NC = kNC<L>;
   constexpr int M = kMat<L>;
-  const int lz = n.vp ? o.limiter_pure : o.limiter;
+  const int lz = n.vp ? P::limiterPure(o) : P::limiter(o);
   const T h0 = n.h0, hp = n.hp, hm = n.hm;
   const T thr = T(o.threshold);
   const T ar = -vminus;  // outer normal . e = -1 on the minus face
@@ -345,14 +345,14 @@ __device__ __forceinline__ void ppFluxes(const Opts& o, const Nbr<T>& n, T vminu
   for (int q = 0; q < NC; ++q) Ar[q] = Av[q] = T(0.0);
 #pragma unroll
   for (int k = 0; k < M; ++k) Dual[k] = T(0.0);
-  const int nInt = ppIntegrated<L>(o, n.vp);
+  const int nInt = ppIntegrated<L, P>(o, n.vp);
 #pragma unroll
   for (int q = 0; q < (kEuc<L> ? NC : 3 * M); ++q) {
     const bool needF = (WANT_AR || WANT_AV) && q < nInt;
     const bool needD = dual && q >= M && q < 2 * M;
     if (!needF && !needD) continue;
     const T phi = n.phi[q], phip = n.phip[q], phim = n.phim[q];
-    const T g = gradQ<XD, T>(o, n, q);
+    const T g = gradQ<XD, true, P, T>(o, n, q);
     const Profile<T> pr = profile<T>(lz, thr, phi, phip, phim, h0, hp, hm, g);
     const bool flat = ((phip - phi) * (phim - phi)) >= T(0.);
     if (needF) {
@@ -362,13 +362,13 @@ __device__ __forceinline__ void ppFluxes(const Opts& o, const Nbr<T>& n, T vminu
     if (needD) Dual[q - M] = flat ? phi * ppdv : sweptIntegral<T>(pr, h0, phim, phip, T(0.), ppdv);
   }
   if (WANT_AR) {
-    finishPP<L, T>(o, n.vp, n.phi, Ar);
+    finishPP<L, P, T>(o, n.vp, n.phi, Ar);
     if (ppvR == T(0.))
 #pragma unroll
       for (int q = 0; q < NC; ++q) Ar[q] = T(0.0);
   }
   if (WANT_AV) {
-    finishPP<L, T>(o, n.vp, n.phi, Av);
+    finishPP<L, P, T>(o, n.vp, n.phi, Av);
     if (ppvV == T(0.))
 #pragma unroll
       for (int q = 0; q < NC; ++q) Av[q] = T(0.0);

@@ -29,7 +29,7 @@ __device__ __forceinline__ void twoSumAcc(double& s, double& comp, double v) {
 // cell's remap vector at the start of the sweep when the caller holds it in
 // registers (the first sweep with the Lagrange update fused), else null and
 // it is read from U_L / U_1.  L: the vector layout (kMat, kNC).
-template <class R, int L, bool PP, bool XD, class T>
+template <class R, int L, bool PP, bool XD, class P, class T>
 __device__ __forceinline__ void sweepUnew(const KPT<R>& kp, long c, long i, long j, long a, bool hasM, bool hasP,
                                           double vm, double vp, double Lm, double Lp, const T* phiM, const T* phiP,
                                           double* Unew, double* Gdual, const double* Uown = nullptr) {
@@ -38,7 +38,7 @@ __device__ __forceinline__ void sweepUnew(const KPT<R>& kp, long c, long i, long
   const Opts& o = kp.o;
   const auto& f = kp.f;
   const long nx = o.nx, ny = o.ny;
-  double* const* Uin = (kp.sweep == 1) ? f.UL : f.U1;
+  double* const* Uin = (P::sweep(kp) == 1) ? f.UL : f.U1;
   auto uOld = [&](int q) { return Uown ? Uown[q] : at(Uin[q], c); };
   const double dtn = f.sc->dt[kp.cur];
   // computeUremap (PhaseRemap1.cc:468-503): a cell receives -G through its
@@ -55,7 +55,7 @@ __device__ __forceinline__ void sweepUnew(const KPT<R>& kp, long c, long i, long
     if (hasM) red[q] = red[q] + (-Gm[q]);
     if (hasP) red[q] = red[q] + Gp[q];
   }
-  if (o.flux_any) {
+  if (P::fluxAny(o)) {
     // remap/BoundaryFluxes.cc:14-120: flux through one face of the cell with
     // the face value of the opposite face; the first matching rule applies
     int rule = 0;  // 1: through the minus face, 2: through the plus face
@@ -95,8 +95,8 @@ __device__ __forceinline__ void sweepUnew(const KPT<R>& kp, long c, long i, long
 #pragma unroll
     for (int q = 0; q < NC; ++q) Unew[q] = uOld(q) - red[q];
   }
-  const bool withG = (o.methode == 0 || o.methode == 1);
-  const int q0 = (o.methode == 0) ? M : 0;
+  const bool withG = (P::methode(o) == 0 || P::methode(o) == 1);
+  const int q0 = (P::methode(o) == 0) ? M : 0;
 #pragma unroll
   for (int k = 0; k < M; ++k) Gdual[k] = (withG && hasM) ? Gm[q0 + k] : 0.0;
   if (withG && !hasP) {
@@ -109,7 +109,7 @@ __device__ __forceinline__ void sweepUnew(const KPT<R>& kp, long c, long i, long
 // The update of cell c and its stores: the final remap of the cell from
 // registers (second sweep, fused; VNR) or the new remap vector, and the flux
 // of its minus face for the dual remap.
-template <class R, int L, bool PP, bool XD, class T>
+template <class R, int L, bool PP, bool XD, class P, class T>
 __device__ __forceinline__ void sweepUpdateCell(const KPT<R>& kp, long c, long i, long j, long a, bool hasM,
                                                 bool hasP, double vm, double vp, double Lm, double Lp,
                                                 const T* phiM, const T* phiP, const double* Uown = nullptr) {
@@ -117,20 +117,20 @@ __device__ __forceinline__ void sweepUpdateCell(const KPT<R>& kp, long c, long i
   constexpr int M = kMat<L>;
   const auto& f = kp.f;
   double Unew[NC], Gd[M];
-  sweepUnew<R, L, PP, XD, T>(kp, c, i, j, a, hasM, hasP, vm, vp, Lm, Lp, phiM, phiP, Unew, Gd, Uown);
+  sweepUnew<R, L, PP, XD, P, T>(kp, c, i, j, a, hasM, hasP, vm, vp, Lm, Lp, phiM, phiP, Unew, Gd, Uown);
   bool stored = false;
   if constexpr (!kEuc<L>) {
-    if (kp.fuseFinal) {
-      finalCell<R, M>(kp, c, Unew);  // remapVariables on the cell, U2 stays in registers
+    if (P::fuse(kp)) {
+      finalCell<R, M, P>(kp, c, Unew);  // remapVariables on the cell, U2 stays in registers
       stored = true;
     }
   }
   if (!stored) {
-    double* const* Uout = (kp.sweep == 1) ? f.U1 : f.U2;
+    double* const* Uout = (P::sweep(kp) == 1) ? f.U1 : f.U2;
 #pragma unroll
     for (int q = 0; q < NC; ++q) at(Uout[q], c) = Unew[q];
   }
-  if (kp.o.methode == 0 || kp.o.methode == 1) {
+  if (P::methode(kp.o) == 0 || P::methode(kp.o) == 1) {
     const long fm = XD ? j * (kp.o.nx + 1) + a : a * kp.o.nx + i;
 #pragma unroll
     for (int k = 0; k < M; ++k) at(f.G[k], fm) = Gd[k];
@@ -151,13 +151,13 @@ struct CellOut {
   double DF[kMat<L>];
 };
 
-template <class R, int L, bool FUSE>
+template <class R, int L, bool FUSE, class P>
 __device__ __forceinline__ void storeCellOut(const KPT<R>& kp, long c, long fm, const CellOut<R, L>& out, bool withG) {
   const auto& f = kp.f;
   if constexpr (FUSE) {
     finalStore<R, kMat<L>>(kp, c, out.fin);
   } else {
-    double* const* Uout = (kp.sweep == 1) ? f.U1 : f.U2;
+    double* const* Uout = (P::sweep(kp) == 1) ? f.U1 : f.U2;
 #pragma unroll
     for (int q = 0; q < kNC<L>; ++q) at(Uout[q], c) = out.U[q];
   }
@@ -202,13 +202,16 @@ template <class R, int L, bool PP>
 constexpr int kStageFuseBytes = (kFuse8<R, kMat<L>> + kMat<L> + (PP ? kMat<L> : 0)) * 8 + kFuse4<R, kMat<L>> * 4;
 template <class R, int L, bool PP>
 constexpr int kStageVecBytes = (kNC<L> + kMat<L> + (PP ? kMat<L> : 0)) * 8;
-// (the Eucclhyd layouts never stage the final fields)
-template <class R, int L, bool PP>
-constexpr int kStageBytes = (!kEuc<L> && kStageFuseBytes<R, L, PP> > kStageVecBytes<R, L, PP>)
-                                ? kStageFuseBytes<R, L, PP>
-                                : kStageVecBytes<R, L, PP>;
-template <class R, int L, bool PP>
-constexpr int kStageWords = (kStageBytes<R, L, PP> + 7) / 8;
+// (the Eucclhyd layouts never stage the final fields; a kernel of fixed
+// options stages one of the two, and no PB flux)
+template <class R, int L, bool PP, class P>
+constexpr int kStageBytes =
+    P::kSweep == 1   ? kStageVecBytes<R, L, false>
+    : P::kSweep == 2 ? kStageFuseBytes<R, L, false>
+    : (!kEuc<L> && kStageFuseBytes<R, L, PP> > kStageVecBytes<R, L, PP>) ? kStageFuseBytes<R, L, PP>
+                                                                        : kStageVecBytes<R, L, PP>;
+template <class R, int L, bool PP, class P>
+constexpr int kStageWords = (kStageBytes<R, L, PP, P> + 7) / 8;
 
 // LDS staging of the CellOut of a tile of TILE cells, in a buffer of
 // kStageWords * TILE doubles: 8-byte member w of element e at
