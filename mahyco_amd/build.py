@@ -22,16 +22,16 @@ ARCH = os.environ.get("MAHYCO_OFFLOAD_ARCH", "gfx950")
 
 HIP_SOURCES = ["sweep_fixed_pp.hip", "sweep_wave.hip", "sweep_wave_mixed.hip", "sweep_walk.hip", "sweep_fixed_walk.hip",
                "sweep_fixed_x_fp64.hip", "sweep_fixed_y_fp64.hip", "sweep_fixed_x_mixed.hip", "sweep_fixed_y_mixed.hip",
-               "lagrange.hip", "sweep_cell.hip", "remap.hip", "eucclhyd.hip", "context.hip"]
+               "lagrange.hip", "sweep_cell.hip", "remap.hip", "dual_both.hip", "eucclhyd.hip", "context.hip"]
 HOST_SOURCES = ["host/donnees.cc", "host/json_input.cc", "host/init.cc", "host/init_euc.cc", "host/output.cc"]
 COMMON = ["-O3", "-std=c++17", "-fPIC", "-ffp-contract=off", "-Wall", "-Wno-unused-function"]
 DEVICE = [f"--offload-arch={ARCH}", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
           "-munsafe-fp-atomics"]
-# per-source device flags: the column walker loops over rows, and
+# per-source device flags: the column walkers loop over rows, and
 # machine-level hoisting of constants out of that loop would hold registers
 # through every row
 WALK_FLAGS = ["-mllvm", "-disable-machine-licm"]
-SOURCE_FLAGS = {"sweep_walk.hip": WALK_FLAGS, "sweep_fixed_walk.hip": WALK_FLAGS}
+SOURCE_FLAGS = {"sweep_walk.hip": WALK_FLAGS, "sweep_fixed_walk.hip": WALK_FLAGS, "dual_both.hip": WALK_FLAGS}
 
 
 def hipcc():

@@ -179,10 +179,12 @@ struct FieldsT {
   // per-step intermediates
   double *UL[NCMAX], *U1[NCMAX], *U2[NCMAX];
   double *VL, *XcL, *YcL, *rL, *qL;
-  double *G[NMAT];   // face fluxes of the current sweep for the dual remap (A1/A2)
+  double *G[NMAT];   // face fluxes of the first sweep for the dual remap (A1/A2)
+  double *G2[NMAT];  // of the second sweep (the same arrays where each sweep's nodal remap follows it)
   double *DF[NMAT];  // PB dual flux per cell of the current sweep
   double *UD1[3];    // nodal vector after dual sweep 1 (M ux, M uy, M)
   double *XL2;       // end-of-Lagrange node coordinate along the second sweep
+  R *uxl, *uyl;         // Lagrange node velocity, where it has a buffer of its own (or null)
   unsigned char* envx;  // compact1: the cell's material fields are stored (1) or derived (0)
   Scalars* sc;
   DtKeys* keys;
@@ -201,6 +203,8 @@ struct KPT {
                  // instead of forming them again from the node velocities
   int dtFold;    // the node update forms dt_{n+1} from the accumulators (whole steps);
                  // 0: it reads the dt a finalize kernel left (phase-level calls)
+  R *ul, *vl;    // the step's Lagrange node velocity: uxl, uyl, or the n+1 buffers in place
+  int dualRows;  // node rows per band of the nodal remap of both sweeps
   long ncell, nnode;
 };
 

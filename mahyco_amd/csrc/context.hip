@@ -23,11 +23,11 @@ using namespace mhy;
 namespace {
 
 enum KernelId {
-  K_DT = 0, K_NODE, K_CELL, K_SWEEP_X, K_SWEEP_Y, K_DUAL_X, K_DUAL_Y, K_FINAL, K_LAGSWEEP_X, K_LAGSWEEP_Y, K_COUNT
+  K_DT = 0, K_NODE, K_CELL, K_SWEEP_X, K_SWEEP_Y, K_DUAL_X, K_DUAL_Y, K_FINAL, K_LAGSWEEP_X, K_LAGSWEEP_Y, K_DUAL, K_COUNT
 };
 const char* kKernelNames[K_COUNT] = {"dt_reduce", "lagrange_node", "lagrange_cell",    "sweep_x",
                                      "sweep_y",   "dual_x",        "dual_y",           "remap_final",
-                                     "lagrange_sweep_x", "lagrange_sweep_y"};
+                                     "lagrange_sweep_x", "lagrange_sweep_y", "dual_both"};
 
 constexpr int kBlock = 256;
 constexpr int kReduceBlocks = 1024;
@@ -121,6 +121,12 @@ struct mhy_ctx {
   // faster (fewer waves leave the chip underfilled); MAHYCO_DUAL_Y=walk /
   // wave / node forces a kernel
   bool dualWalkY = false;
+  // whole steps: the nodal remap of both sweeps in one kernel after the second
+  // cell sweep (fixed options; MAHYCO_DUAL_Y forces one kernel per sweep).  The
+  // contexts that may use it keep the Lagrange velocity and the second sweep's
+  // face fluxes in buffers of their own.
+  bool dualBoth = false;
+  int dualRows = 32;  // node rows per band
   // nodal remap along y on LDS tiles of 16 node columns x dualTileRows
   // rows: 48 (MAHYCO_DUAL_Y=tile), 32 or 64 (tile32, tile64)
   bool dualTileY = false;
@@ -236,6 +242,12 @@ int* allocI(mhy_ctx* x, long n, hipError_t& e) {
   return static_cast<int*>(p);
 }
 
+// the Lagrange node velocity of the step with kp's parity
+void setLagrangeVelocity(KP& kp) {
+  kp.ul = kp.f.uxl ? kp.f.uxl : kp.f.ux[kp.nxt];
+  kp.vl = kp.f.uyl ? kp.f.uyl : kp.f.uy[kp.nxt];
+}
+
 KP makeKP(const mhy_ctx* x) {
   KP kp;
   kp.f = x->f;
@@ -251,14 +263,17 @@ KP makeKP(const mhy_ctx* x) {
   kp.geomLoad = (!x->fuseLag || x->geomStored) ? 1 : 0;
   kp.ncell = x->ncell;
   kp.nnode = x->nnode;
+  setLagrangeVelocity(kp);
+  kp.dualRows = x->dualRows;
   return kp;
 }
 
 // candidate ids of the tuner's sites
-enum { TD_TILE = 0, TD_WAVE = 1, TD_WALK = 2, TD_TILE32 = 3, TD_TILE64 = 4 };  // nodal remap along y
+// nodal remap along y (TD_BOTH: of both sweeps, in one kernel)
+enum { TD_TILE = 0, TD_WAVE = 1, TD_WALK = 2, TD_TILE32 = 3, TD_TILE64 = 4, TD_BOTH = 5 };
 enum { TS_WAVE = 0, TS_WALK = 1 };               // cell sweep along y
 enum { TL_FUSED = 0, TL_SEPARATE = 1 };          // Lagrange cell update of y-first steps
-const char* kDualNames[5] = {"tile", "wave", "walk", "tile32", "tile64"};
+const char* kDualNames[6] = {"tile", "wave", "walk", "tile32", "tile64", "both"};
 const char* kSweepNames[2] = {"wave", "walk"};
 const char* kLagNames[2] = {"fused", "separate"};
 
@@ -340,7 +355,8 @@ void tuneStepDone(mhy_ctx* x) {
     auto add = [&](const char* k, const char* v) {
       t.choice += std::string(t.choice.empty() ? "" : " ") + k + "=" + v;
     };
-    if (t.ncand[0]) add("dual_y", kDualNames[t.cand[0][t.best[0]]]);
+    if (x->dualBoth) add("dual_y", kDualNames[TD_BOTH]);
+    else if (t.ncand[0]) add("dual_y", kDualNames[t.cand[0][t.best[0]]]);
     if (t.ncand[1]) add("sweep_y", kSweepNames[t.cand[1][t.best[1]]]);
     if (t.ncand[2]) add("lagrange_y", kLagNames[t.cand[2][t.best[2]]]);
     else if (!t.forcedLag.empty()) add("lagrange_y", t.forcedLag.c_str());
@@ -669,6 +685,18 @@ int phaseSweepStage(mhy_ctx* x, int sweep, int stage) {
   return checkLaunch(x, "sweep");
 }
 
+// nodal remap of both sweeps (whole steps)
+int phaseDualBoth(mhy_ctx* x) {
+  const KP kp = makeKP(x);
+  const bool xfirst = x->x_then_y_n;
+  const int items = dualBothItems(x->o.nx, x->o.ny, x->dualRows, xfirst);
+  timed(x, K_DUAL, [&] {
+    launchR(x, dualBothKernel<double>(x->fixLim, x->o.nbmat, xfirst), dualBothKernel<float>(x->fixLim, x->o.nbmat, xfirst),
+            dim3((unsigned)((items + 3) / 4)), dim3(kBlock), kp);
+  });
+  return checkLaunch(x, "dual");
+}
+
 int phaseSweep(mhy_ctx* x, int sweep) {
   int st = phaseSweepStage(x, sweep, MHY_STAGE_CELLS);
   return st != MHY_OK ? st : phaseSweepStage(x, sweep, MHY_STAGE_NODES);
@@ -713,8 +741,14 @@ int runIteration(mhy_ctx* x) {
   if ((st = phaseDt(x)) != MHY_OK) return st;
   if ((st = phaseLagrange(x)) != MHY_OK) return st;
   if (x->o.mode != MODE_LAGRANGE) {
-    if ((st = phaseSweep(x, 1)) != MHY_OK) return st;
-    if ((st = phaseSweep(x, 2)) != MHY_OK) return st;
+    if (x->dualBoth) {
+      if ((st = phaseSweepStage(x, 1, MHY_STAGE_CELLS)) != MHY_OK) return st;
+      if ((st = phaseSweepStage(x, 2, MHY_STAGE_CELLS)) != MHY_OK) return st;
+      if ((st = phaseDualBoth(x)) != MHY_OK) return st;
+    } else {
+      if ((st = phaseSweep(x, 1)) != MHY_OK) return st;
+      if ((st = phaseSweep(x, 2)) != MHY_OK) return st;
+    }
     if ((st = phaseFinal(x)) != MHY_OK) return st;
   }
   x->iteration++;
@@ -1120,6 +1154,13 @@ static int createContext(const mhy_config* cfg, mhy_ctx** out, bool batchMember)
   o.flux_left = b.flux_left, o.flux_right = b.flux_right, o.flux_bottom = b.flux_bottom, o.flux_top = b.flux_top;
   o.flux_any = (b.flux_left + b.flux_right + b.flux_bottom + b.flux_top) > 0;
   x->fixLim = pickFixed(o);
+  x->dualBoth = x->fixLim != 0 && x->sweepWave && !std::getenv("MAHYCO_DUAL_Y");
+  x->dualRows = dualBothRows(dualBothItems(c.nx, c.ny, 2, true));
+  if (x->dualBoth && x->tune.on) {  // no choice left at that site
+    x->tune.ncand[0] = 0;
+    x->tune.steps = 2 * mhy_ctx::kTuneRounds * (x->tune.ncand[1] + x->tune.ncand[2]);
+    x->tune.on = x->tune.steps > 0;
+  }
   // one perfect-gas material, Lagrange + remap: the final remap stores the
   // material fields only where they differ from the means (MAHYCO_COMPACT=0
   // stores them everywhere, as for several materials)
@@ -1174,7 +1215,12 @@ static int createContext(const mhy_config* cfg, mhy_ctx** out, bool batchMember)
     if (o.pp == 1) AD(f.qL, C);
     x->nface = std::max((long)(c.nx + 1) * c.ny, (long)c.nx * (c.ny + 1));
     if (o.methode == 0 || o.methode == 1)
-      for (int k = 0; k < m; ++k) AD(f.G[k], x->nface);
+      for (int k = 0; k < m; ++k) {
+        AD(f.G[k], x->nface);
+        f.G2[k] = f.G[k];
+        if (x->dualBoth) AD(f.G2[k], x->nface);
+      }
+    if (x->dualBoth) AR(f.uxl, N), AR(f.uyl, N);
     if (o.methode == 2)
       for (int k = 0; k < m; ++k) AD(f.DF[k], C);
     for (int d = 0; d < 3; ++d) AD(f.UD1[d], N);
@@ -1629,6 +1675,9 @@ int mhy_kernel_bytes(const mhy_ctx* x, int k, double* bytes) {
       w = lagIn + lagOut + C * nc * d + fl;
       break;
     }
+    case K_DUAL:  // face fluxes of both sweeps, Lagrange velocity, Mp ; new velocity
+      w = 2.0 * F * m * d + N * 5 * r;
+      break;
     case K_DUAL_X:
     case K_DUAL_Y:
       // face fluxes (or PB cell fluxes) + sweep 1: u, Mp ; UD1, XL2
@@ -1757,7 +1806,7 @@ void ctxMesh(const mhy_ctx* x, long& nx, long& ny) { nx = x->o.nx, ny = x->o.ny;
 namespace {
 using namespace mhy;
 
-enum BatchKernel { BK_DT = 0, BK_NODE, BK_CELL, BK_SWX, BK_SWY, BK_DUX, BK_DUY, BK_COUNT };
+enum BatchKernel { BK_DT = 0, BK_NODE, BK_CELL, BK_SWX, BK_SWY, BK_DUX, BK_DUY, BK_DUAL, BK_COUNT };
 constexpr int kVariants = 16;  // cur (1 bit), sweep-1 (1), xdir (1), fuseFinal (1)
 constexpr unsigned kCand[] = {0u, 1024u, 2048u, 4096u, 8192u};  // 0: one workgroup per virtual block
 constexpr int kNCand = sizeof(kCand) / sizeof(kCand[0]);
@@ -1801,7 +1850,9 @@ struct mhy_batch {
   bool dualWaveY = true;  // nodal remap along y with the wave kernel
   bool walkY = false;     // cell sweeps along y with the column-walking kernel
   bool o3 = false;        // third-order remap (LDS-tile cell sweeps)
-  int fixLim = 0;         // every problem has this fixed limiter (fixedLimiter), or 0
+  int fixLim = 0;         // limited slopes: every problem has this fixed limiter (fixedLimiter), or 0
+  int dualLim = 0;        // the same with PenteBorne too: nodal remap of both sweeps in one kernel
+  int dualRows = 32;      // node rows per band of that kernel
   void* dTable = nullptr;  // KPT<double> or KPT<float> entries
   unsigned* dStart = nullptr;  // BK_COUNT x (n+1)
   unsigned* dGx = nullptr;     // BK_COUNT x n
@@ -1816,6 +1867,7 @@ struct mhy_batch {
   bool tune = true, useGraph = true;
   int tuneStep = 0;
   float tuneMs[BK_COUNT][kNCand] = {};
+  bool ran[BK_COUNT] = {};  // launched (and timed) in the last tuning step
   hipEvent_t ev[2 * BK_COUNT] = {};
   hipGraphExec_t exec[2] = {nullptr, nullptr};
   std::string err;
@@ -1843,6 +1895,7 @@ int batchEnqueueStepR(mhy_batch* b, int cur, bool xty, bool timing) {
     const bool one = !fnLoop || b->blocks[k] == 0 || b->blocks[k] >= b->total[k];
     const unsigned grid = one ? b->total[k] : b->blocks[k];
     const Fn fn = one ? fnOne : fnLoop;
+    b->ran[k] = true;
     if (timing) (void)hipEventRecord(b->ev[2 * k], b->stream);
     hipLaunchKernelGGL(fn, dim3(grid), dim3(block), 0, b->stream, bl);
     if (timing) (void)hipEventRecord(b->ev[2 * k + 1], b->stream);
@@ -1869,7 +1922,10 @@ int batchEnqueueStepR(mhy_batch* b, int cur, bool xty, bool timing) {
     else
       launch(xd ? BK_SWX : BK_SWY, sweepBatchKernel<R, false>(xd, b->m, b->pp),
              sweepBatchKernel<R, true>(xd, b->m, b->pp), v + 8 * fuse, sweepWaveBlock(xd, b->mixed, b->pp));
-    if (xd) launch(BK_DUX, k_dual_wave_batch<R, true, false>, k_dual_wave_batch<R, true, true>, v);
+    if (b->dualLim) {
+      if (sweep == 2)
+        launch(BK_DUAL, nullptr, dualBothBatchKernel<R>(b->dualLim, b->m, xty), cur);
+    } else if (xd) launch(BK_DUX, k_dual_wave_batch<R, true, false>, k_dual_wave_batch<R, true, true>, v);
     else if (b->dualWaveY)
       launch(BK_DUY, k_dual_wave_batch<R, false, false>, k_dual_wave_batch<R, false, true>, v, dualWaveBlock(false, b->mixed));
     else launch(BK_DUY, k_dual_batch<R, false, false>, k_dual_batch<R, false, true>, v);
@@ -1949,6 +2005,8 @@ int mhy_batch_create(const mhy_config* cfgs, int n, mhy_batch** out) {
     // (kind 1 and 2 of the limited-slope sweeps, one limiter for all)
     const int lim = (b->pp || b->o3) ? 0 : b->ctx[i]->fixLim;
     b->fixLim = (i == 0 || b->fixLim == lim) ? lim : 0;
+    const int dual = b->ctx[i]->dualBoth ? b->ctx[i]->fixLim : 0;
+    b->dualLim = (i == 0 || b->dualLim == dual) ? dual : 0;
   }
   b->cur0 = b->cur = b->ctx[0]->cur;
   b->xty0 = b->xty = b->ctx[0]->x_then_y_n;
@@ -1959,6 +2017,9 @@ int mhy_batch_create(const mhy_config* cfgs, int n, mhy_batch** out) {
   // same layout, so the mixed form uploads the same entries)
   static_assert(sizeof(KPT<float>) == sizeof(KP), "parameter blocks differ");
   std::vector<KP> table((size_t)kVariants * n);
+  long waves2 = 0;
+  for (const mhy_ctx* x : b->ctx) waves2 += dualBothItems(x->o.nx, x->o.ny, 2, true);
+  b->dualRows = dualBothRows(waves2);
   for (int v = 0; v < kVariants; ++v)
     for (int i = 0; i < n; ++i) {
       KP kp = makeKP(b->ctx[i]);
@@ -1968,6 +2029,8 @@ int mhy_batch_create(const mhy_config* cfgs, int n, mhy_batch** out) {
       kp.xdir = (v >> 2) & 1;
       kp.fuseFinal = (v >> 3) & 1;
       kp.dtFold = 1;
+      setLagrangeVelocity(kp);
+      kp.dualRows = b->dualRows;
       table[(size_t)v * n + i] = kp;
     }
   // virtual-block layout of every kernel
@@ -1992,6 +2055,7 @@ int mhy_batch_create(const mhy_config* cfgs, int n, mhy_batch** out) {
           break;
         case BK_DUX: g = dualWaveGrid(true, nx, ny, b->mixed); break;
         case BK_DUY: g = b->dualWaveY ? dualWaveGrid(false, nx, ny, b->mixed) : gridFor(x->nnode); break;
+        case BK_DUAL: g = dim3((unsigned)((dualBothItems(nx, ny, b->dualRows, false) + 3) / 4)); break;
         default: g = gridFor(x->nnode); break;  // per-node dual along y
       }
       start[(size_t)k * (n + 1) + i] = acc;
@@ -2062,7 +2126,8 @@ int mhy_batch_run(mhy_batch* b, int nsteps) {
       if ((st = batchEnqueueStep(b, b->cur, b->xty, true)) != MHY_OK) return st;
       if (hipStreamSynchronize(b->stream) != hipSuccess) return batchFail(b, MHY_ERR_DEVICE, "batch sync");
       const bool verbose = std::getenv("MAHYCO_BATCH_VERBOSE") != nullptr;
-      for (int k = 0; k < BK_COUNT; ++k) {  // every kernel runs once per step
+      for (int k = 0; k < BK_COUNT; ++k) {  // a kernel runs at most once per step
+        if (!b->ran[k]) continue;
         float ms = 0.f;
         if (hipEventElapsedTime(&ms, b->ev[2 * k], b->ev[2 * k + 1]) == hipSuccess) b->tuneMs[k][cand] += ms;
         if (verbose) std::fprintf(stderr, "[batch tune] kernel %d blocks %u: %.4f ms\n", k, kCand[cand], ms);

@@ -104,6 +104,15 @@ dim3 dualTileGrid(long nx, long ny, int rows);
 unsigned dualTileBlock();
 dim3 dualWalkGrid(long nx, long ny);
 unsigned dualWaveBlock(bool xd, bool mixed);
+// nodal remap of both sweeps in one kernel (fixed options, lim from
+// fixedLimiter), on bands of dualBothRows(waves at 2 rows) node
+// rows; dualBothItems: waves in all
+template <class R>
+SweepFn<R> dualBothKernel(int lim, int m, bool xfirst);
+template <class R>
+SweepBatchFn<R> dualBothBatchKernel(int lim, int m, bool xfirst);
+int dualBothItems(long nx, long ny, int rows, bool xfirst);
+int dualBothRows(long waves2);
 template <class R, int M>
 __global__ void k_remap_final(KPT<R> kp);
 template <class R>

@@ -165,8 +165,8 @@ __device__ __forceinline__ void lagrangeNodeAt(const KPT<R>& kp, double dt1, lon
   f.Mp[p] = Mp;
   const double uxn = (double)f.ux[kp.cur][p], uyn = (double)f.uy[kp.cur][p];
   if (o.mode == MODE_ADVECTION) {
-    f.ux[kp.nxt][p] = uxn;
-    f.uy[kp.nxt][p] = uyn;
+    kp.ul[p] = uxn;
+    kp.vl[p] = uyn;
     return;
   }
   const double dt = 0.5 * (dt1 + f.sc->dt[kp.cur]);
@@ -224,8 +224,8 @@ __device__ __forceinline__ void lagrangeNodeAt(const KPT<R>& kp, double dt1, lon
     if (j == 0 && i == 0) corner(o.bc_bottom, o.bc_left, o.bcv_left);
     if (j == 0 && i == nx) corner(o.bc_bottom, o.bc_right, o.bcv_right);
   }
-  f.ux[kp.nxt][p] = u1.x;
-  f.uy[kp.nxt][p] = u1.y;
+  kp.ul[p] = u1.x;
+  kp.vl[p] = u1.y;
   if (o.mode == MODE_LAGRANGE) {
     f.X[kp.nxt][p] = X0.x + u1.x * dt1;
     f.Y[kp.nxt][p] = X0.y + u1.y * dt1;
@@ -262,8 +262,8 @@ __device__ __forceinline__ void lagrangeNodeInner(const KPT<R>& kp, double dt1, 
     r = d2add(r, d2mul(Cn[q], pq));
   }
   const D2 u1 = d2add(D2{uxn, uyn}, d2mul(r, dt / Mp));
-  f.ux[kp.nxt][p] = u1.x;
-  f.uy[kp.nxt][p] = u1.y;
+  kp.ul[p] = u1.x;
+  kp.vl[p] = u1.y;
 }
 
 // One thread per node, any mode (b: block index inside the problem).

@@ -39,7 +39,7 @@ __device__ __forceinline__ void lagNodes(const KPT<R>& kp, double dt1, long j, l
       X[s] = {at(f.X[kp.nxt] + dp[s], p0), at(f.Y[kp.nxt] + dp[s], p0)};
     } else {
       const D2 e = eulerNode(o, jj[s], ii[s]);
-      X[s] = {e.x + (double)at(f.ux[kp.nxt] + dp[s], p0) * dt1, e.y + (double)at(f.uy[kp.nxt] + dp[s], p0) * dt1};
+      X[s] = {e.x + (double)at(kp.ul + dp[s], p0) * dt1, e.y + (double)at(kp.vl + dp[s], p0) * dt1};
     }
   }
 }

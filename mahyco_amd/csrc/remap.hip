@@ -47,7 +47,7 @@ __device__ __forceinline__ void dualBody(const KPT<R>& kp, unsigned b) {
     }
     const long q = p + (d - 3) * stride;
     if (kp.sweep == 1) {
-      const double ux1 = (double)at(f.ux[kp.nxt], q), uy1 = (double)at(f.uy[kp.nxt], q);
+      const double ux1 = (double)at(kp.ul, q), uy1 = (double)at(kp.vl, q);
       dpx[d] = ux1, dpy[d] = uy1;
       const long jq = q / (nx + 1), iq = q - jq * (nx + 1);
       const D2 e = eulerNode(o, jq, iq);
@@ -63,7 +63,7 @@ __device__ __forceinline__ void dualBody(const KPT<R>& kp, unsigned b) {
   if (kp.sweep == 1) {
     // Lagrange coordinate of this node along the second sweep's axis
     const D2 e = eulerNode(o, j, i);
-    at(f.XL2, p) = XD ? e.y + (double)at(f.uy[kp.nxt], p) * dt1 : e.x + (double)at(f.ux[kp.nxt], p) * dt1;
+    at(f.XL2, p) = XD ? e.y + (double)at(kp.vl, p) * dt1 : e.x + (double)at(kp.ul, p) * dt1;
   }
   // divided differences between slots k and k+1 (k = 1..4), each formed
   // once: the plus side of slot d is the minus side of slot d+1
@@ -118,14 +118,15 @@ __device__ __forceinline__ void dualBody(const KPT<R>& kp, unsigned b) {
     auto cidx = [&](long b, long tt) { return XD ? tt * nx + b : b * nx + tt; };
     // the along-sweep neighbour's face / cell: a uniform step, folded into the base
     const long dA = XD ? 1 : nx;
+    double* const* G = (kp.sweep == 1) ? f.G : f.G2;
     for (int k = 0; k < m; ++k) {
       double pk = 0, mk = 0;
       if (o.methode == 0 || o.methode == 1) {
         for (int s = 0; s < nf; ++s) {
           const long tt = tf[s];
-          const double Gf = at(f.G[k], gidx(a, tt));
-          double tp = Gf + at(f.G[k] + dA, gidx(a, tt));
-          double tm = Gf + at(f.G[k] - dA, gidx(a, tt));
+          const double Gf = at(G[k], gidx(a, tt));
+          double tp = Gf + at(G[k] + dA, gidx(a, tt));
+          double tm = Gf + at(G[k] - dA, gidx(a, tt));
           if (o.methode == 1) tp = at(f.rL, cidx(a, tt)) * tp, tm = at(f.rL - dA, cidx(a, tt)) * tm;
           pk += tp;
           mk += tm;
@@ -168,7 +169,7 @@ __device__ __forceinline__ void dualBody(const KPT<R>& kp, unsigned b) {
   double U0, U1, U2;
   if (kp.sweep == 1) {
     const double Mp = at(f.Mp, p);
-    U0 = Mp * at(f.ux[kp.nxt], p), U1 = Mp * at(f.uy[kp.nxt], p), U2 = Mp;
+    U0 = Mp * at(kp.ul, p), U1 = Mp * at(kp.vl, p), U2 = Mp;
   } else {
     U0 = at(f.UD1[0], p), U1 = at(f.UD1[1], p), U2 = at(f.UD1[2], p);
   }
@@ -263,14 +264,15 @@ __device__ __forceinline__ void dualNodeFinish(const KPT<R>& kp, long a, long t,
     auto cidx = [&](long b, long tt) { return XD ? tt * nx + b : b * nx + tt; };
     // the along-sweep neighbour's face / cell: a uniform step, folded into the base
     const long dA = XD ? 1 : nx;
+    double* const* G = (kp.sweep == 1) ? f.G : f.G2;
     for (int k = 0; k < m; ++k) {
       double pk = 0, mk = 0;
       if (o.methode == 0 || o.methode == 1) {
         for (int s2 = 0; s2 < nf; ++s2) {
           const long tt = tf[s2];
-          const double Gf = at(f.G[k], gidx(a, tt));
-          double tp = Gf + at(f.G[k] + dA, gidx(a, tt));
-          double tm = Gf + at(f.G[k] - dA, gidx(a, tt));
+          const double Gf = at(G[k], gidx(a, tt));
+          double tp = Gf + at(G[k] + dA, gidx(a, tt));
+          double tm = Gf + at(G[k] - dA, gidx(a, tt));
           if (o.methode == 1) tp = at(f.rL, cidx(a, tt)) * tp, tm = at(f.rL - dA, cidx(a, tt)) * tm;
           pk += tp;
           mk += tm;
@@ -314,7 +316,7 @@ __device__ __forceinline__ void dualNodeFinish(const KPT<R>& kp, long a, long t,
   double U0, U1, U2;
   if (kp.sweep == 1) {
     const double Mp = at(f.Mp, p);
-    U0 = Mp * at(f.ux[kp.nxt], p), U1 = Mp * at(f.uy[kp.nxt], p), U2 = Mp;
+    U0 = Mp * at(kp.ul, p), U1 = Mp * at(kp.vl, p), U2 = Mp;
   } else {
     U0 = at(f.UD1[0], p), U1 = at(f.UD1[1], p), U2 = at(f.UD1[2], p);
   }
@@ -370,7 +372,7 @@ __device__ __forceinline__ void dualWaveBody(const KPT<R>& kp, unsigned b) {
   double xl0 = 0.0;
   if (in) {
     if (kp.sweep == 1) {
-      const double ux1 = (double)at(f.ux[kp.nxt], p), uy1 = (double)at(f.uy[kp.nxt], p);
+      const double ux1 = (double)at(kp.ul, p), uy1 = (double)at(kp.vl, p);
       dpx0 = T(ux1), dpy0 = T(uy1);
       const D2 e = eulerNode(o, j, i);
       xl0 = XD ? e.x + ux1 * dt1 : e.y + uy1 * dt1;
@@ -484,7 +486,7 @@ __device__ __forceinline__ void dualWalkBody(const KPT<R>& kp, long item) {
     if (rin && inT) {
       const long p = r * (nx + 1) + t;
       if (kp.sweep == 1) {
-        const double ux1 = (double)at(f.ux[kp.nxt], p), uy1 = (double)at(f.uy[kp.nxt], p);
+        const double ux1 = (double)at(kp.ul, p), uy1 = (double)at(kp.vl, p);
         dx = T(ux1), dy = T(uy1);
         const D2 e = eulerNode(o, r, t);
         xl = e.y + uy1 * dt1;
@@ -594,7 +596,7 @@ __device__ __forceinline__ void dualTileBody(const KPT<R>& kp, unsigned b) {
     if (inRow(L) && inT) {
       const long p = a * (nx + 1) + t;
       if (kp.sweep == 1) {
-        const double ux1 = (double)at(f.ux[kp.nxt], p), uy1 = (double)at(f.uy[kp.nxt], p);
+        const double ux1 = (double)at(kp.ul, p), uy1 = (double)at(kp.vl, p);
         dx = T(ux1), dy = T(uy1);
         const D2 e = eulerNode(o, a, t);
         xl = e.y + uy1 * dt1;

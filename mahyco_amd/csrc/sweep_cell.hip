@@ -31,7 +31,7 @@ __device__ __forceinline__ double widthCell(const KPT<R>& kp, double dt1, long j
   auto node = [&](long jj, long ii) {
     const long p = jj * (kp.o.nx + 1) + ii;
     const D2 e = eulerNode(kp.o, jj, ii);
-    return D2{e.x + (double)kp.f.ux[kp.nxt][p] * dt1, e.y + (double)kp.f.uy[kp.nxt][p] * dt1};
+    return D2{e.x + (double)kp.ul[p] * dt1, e.y + (double)kp.vl[p] * dt1};
   };
   double h = 0.;
   if (XD) {  // bottom then top face
@@ -219,7 +219,7 @@ __global__ __launch_bounds__(256) void k_sweep_cell(KP kp) {
     long n1, n2;
     if (XD) n1 = j * (nx + 1) + b, n2 = (j + 1) * (nx + 1) + b;
     else n1 = b * (nx + 1) + i, n2 = b * (nx + 1) + i + 1;
-    const double* u = XD ? f.ux[kp.nxt] : f.uy[kp.nxt];
+    const double* u = XD ? kp.ul : kp.vl;
     return 0.0 + ((0.0 + u[n1]) + u[n2]) * 0.5;
   };
   // Euler length of face b (Init.cc:528-533)
@@ -334,12 +334,13 @@ __global__ __launch_bounds__(256) void k_sweep_cell(KP kp) {
   if (o.methode == 0 || o.methode == 1) {
     const int q0 = (o.methode == 0) ? M : 0;
     const long fm = XD ? j * (nx + 1) + a : a * nx + i;
+    double* const* G = sweepG<RunOpts>(kp);
 #pragma unroll
-    for (int k = 0; k < M; ++k) f.G[k][fm] = hasM ? Gm[q0 + k] : 0.0;
+    for (int k = 0; k < M; ++k) G[k][fm] = hasM ? Gm[q0 + k] : 0.0;
     if (!hasP) {
       const long fp = XD ? j * (nx + 1) + a + 1 : (a + 1) * nx + i;
 #pragma unroll
-      for (int k = 0; k < M; ++k) f.G[k][fp] = 0.0;
+      for (int k = 0; k < M; ++k) G[k][fp] = 0.0;
     }
   }
 }
@@ -377,7 +378,7 @@ __device__ __forceinline__ void sweepO3Cell(const KPT<R>& kp, const double* sY, 
     long n1, n2;
     if (XD) n1 = j * (nx + 1) + b, n2 = (j + 1) * (nx + 1) + b;
     else n1 = b * (nx + 1) + i, n2 = b * (nx + 1) + i + 1;
-    const R* u = XD ? f.ux[kp.nxt] : f.uy[kp.nxt];
+    const R* u = XD ? kp.ul : kp.vl;
     return 0.0 + ((0.0 + (double)u[n1]) + (double)u[n2]) * 0.5;
   };
   // Euler length of face b (Init.cc:528-533)

@@ -21,6 +21,12 @@ __device__ __forceinline__ void twoSumAcc(double& s, double& comp, double v) {
   s = t;
 }
 
+// the sweep's face fluxes for the dual remap
+template <class P, class R>
+__device__ __forceinline__ double* const* sweepG(const KPT<R>& kp) {
+  return (P::sweep(kp) == 1) ? kp.f.G : kp.f.G2;
+}
+
 // Cell c (along index a, row j, column i) with face values phiM / phiP at
 // its minus / plus faces (valid when hasM / hasP), face normal velocities
 // vm / vp and Euler face lengths Lm / Lp: its new remap vector Unew and the
@@ -102,7 +108,7 @@ __device__ __forceinline__ void sweepUnew(const KPT<R>& kp, long c, long i, long
   if (withG && !hasP) {
     const long fp = XD ? j * (nx + 1) + a + 1 : (a + 1) * nx + i;
 #pragma unroll
-    for (int k = 0; k < M; ++k) f.G[k][fp] = 0.0;
+    for (int k = 0; k < M; ++k) sweepG<P>(kp)[k][fp] = 0.0;
   }
 }
 
@@ -133,7 +139,7 @@ __device__ __forceinline__ void sweepUpdateCell(const KPT<R>& kp, long c, long i
   if (P::methode(kp.o) == 0 || P::methode(kp.o) == 1) {
     const long fm = XD ? j * (kp.o.nx + 1) + a : a * kp.o.nx + i;
 #pragma unroll
-    for (int k = 0; k < M; ++k) at(f.G[k], fm) = Gd[k];
+    for (int k = 0; k < M; ++k) at(sweepG<P>(kp)[k], fm) = Gd[k];
   }
 }
 
@@ -163,7 +169,7 @@ __device__ __forceinline__ void storeCellOut(const KPT<R>& kp, long c, long fm, 
   }
   if (withG) {
 #pragma unroll
-    for (int k = 0; k < kMat<L>; ++k) at(f.G[k], fm) = out.G[k];
+    for (int k = 0; k < kMat<L>; ++k) at(sweepG<P>(kp)[k], fm) = out.G[k];
   }
 }
 

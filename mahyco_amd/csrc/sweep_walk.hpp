@@ -32,7 +32,7 @@ template <class R>
 __device__ __forceinline__ D2 lagNodeK(const KPT<R>& kp, double dt1, long j, long i) {
   const long p = j * (kp.o.nx + 1) + i;
   const D2 e = eulerNode(kp.o, j, i);
-  return {e.x + (double)at(kp.f.ux[kp.nxt], p) * dt1, e.y + (double)at(kp.f.uy[kp.nxt], p) * dt1};
+  return {e.x + (double)at(kp.ul, p) * dt1, e.y + (double)at(kp.vl, p) * dt1};
 }
 
 // width across the y-sweep faces (HvLagrange, PhaseRemap2.cc): right then
@@ -69,7 +69,7 @@ __device__ __forceinline__ void sweepWalkYBody(const KPT<R>& kp, unsigned b) {
   const bool mixteOpt = PP && P::mixte(o);
   const bool pb = PP && P::methode(o) == 2;
   const bool formed = P::order(o) > 1;
-  const R* uy = f.uy[kp.nxt];
+  const R* uy = kp.vl;
 
   // rolling state: A = row r-2, B = row r-1
   T phA[NC], phB[NC], dMB[NC], gA[NC], avA[NC], faceA[NC], dualA[M];

@@ -65,7 +65,7 @@ template <class R>
 __device__ __forceinline__ D2 lagNodeW(const KPT<R>& kp, double dt1, long j, long i) {
   const long p = j * (kp.o.nx + 1) + i;
   const D2 e = eulerNode(kp.o, j, i);
-  return {e.x + (double)at(kp.f.ux[kp.nxt], p) * dt1, e.y + (double)at(kp.f.uy[kp.nxt], p) * dt1};
+  return {e.x + (double)at(kp.ul, p) * dt1, e.y + (double)at(kp.vl, p) * dt1};
 }
 
 // width across the sweep faces (HvLagrange, PhaseRemap1.cc:57-71, :104-119)
@@ -320,7 +320,7 @@ __device__ __forceinline__ void sweepWaveBody(const KPT<R>& kp, unsigned b) {
     // the face's second node is a uniform distance from the first (next row
     // along x, next column along y): one 32-bit offset serves both loads
     const long n1 = XD ? j * (nx + 1) + b : b * (nx + 1) + i;
-    const R* uu = XD ? f.ux[kp.nxt] : f.uy[kp.nxt];
+    const R* uu = XD ? kp.ul : kp.vl;
     return 0.0 + ((0.0 + (double)at(uu, n1)) + (double)at(uu + (XD ? nx + 1 : 1), n1)) * 0.5;
   };
   const double vm = in ? fnv(a) : 0.0;
