@@ -170,6 +170,7 @@ struct FieldsT {
   R *ux[2], *uy[2];
   double *X[2], *Y[2];  // moving node coordinates (MODE_LAGRANGE)
   double *vol[2];       // sum of the corner sub-volumes of the step start
+  double *cvol;         // cfl sqrt(vol) of the fixed Euler cells (null when the mesh moves)
   double *f_k[NMAT];
   R *mu_k[NMAT];
   double *M, *M_k[NMAT];

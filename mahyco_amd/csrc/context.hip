@@ -99,6 +99,10 @@ struct mhy_ctx {
   // whole steps: the node update folds the dt accumulators itself; the
   // phase-level calls launch a finalize kernel in the dt phase instead
   bool dtFold = false;
+  // the dt accumulators of the current parity hold the current state's (left
+  // by the nodal remap of the last step, or by the reduction kernel); keysNext:
+  // of the next parity.  Writing a field from the host empties them.
+  bool keysFull = false, keysNext = false;
   // sweep 1 runs the cell part of the Lagrange phase (wave sweeps only;
   // environment MAHYCO_FUSE_LAGRANGE=0 keeps it a separate kernel)
   bool fuseLag = true;
@@ -504,8 +508,9 @@ int phaseDt(mhy_ctx* x) {
     timed(x, K_DT, [&] { launchR(x, k_dt_hold<double>, k_dt_hold<float>, dim3(1), dim3(64), kp); });
   } else {
     const unsigned nb = (unsigned)std::min<long>(kReduceBlocks, (x->ncell + kBlock - 1) / kBlock);
+    if (x->keysFull && x->dtFold) return MHY_OK;
     timed(x, K_DT, [&] {
-      launchR(x, k_dt_reduce<double>, k_dt_reduce<float>, dim3(nb), dim3(kBlock), kp);
+      if (!x->keysFull) launchR(x, k_dt_reduce<double>, k_dt_reduce<float>, dim3(nb), dim3(kBlock), kp);
       if (!x->dtFold) launchR(x, k_dt_finalize<double>, k_dt_finalize<float>, dim3(1), dim3(64), kp);
     });
   }
@@ -685,15 +690,19 @@ int phaseSweepStage(mhy_ctx* x, int sweep, int stage) {
   return checkLaunch(x, "sweep");
 }
 
+// a whole step leaves the next one's dt accumulators
+bool leavesDt(const mhy_ctx* x) { return x->dualBoth && dualBothDt(x->dualRows); }
+
 // nodal remap of both sweeps (whole steps)
 int phaseDualBoth(mhy_ctx* x) {
   const KP kp = makeKP(x);
   const bool xfirst = x->x_then_y_n;
   const int items = dualBothItems(x->o.nx, x->o.ny, x->dualRows, xfirst);
   timed(x, K_DUAL, [&] {
-    launchR(x, dualBothKernel<double>(x->fixLim, x->o.nbmat, xfirst), dualBothKernel<float>(x->fixLim, x->o.nbmat, xfirst),
-            dim3((unsigned)((items + 3) / 4)), dim3(kBlock), kp);
+    launchR(x, dualBothKernel<double>(x->fixLim, x->o.nbmat, xfirst, x->dualRows),
+            dualBothKernel<float>(x->fixLim, x->o.nbmat, xfirst, x->dualRows), dim3((unsigned)((items + 3) / 4)), dim3(kBlock), kp);
   });
+  x->keysNext = dualBothDt(x->dualRows);
   return checkLaunch(x, "dual");
 }
 
@@ -727,6 +736,8 @@ int readScalars(mhy_ctx* x, Scalars& s) {
 void endIteration(mhy_ctx* x) {
   tuneStepDone(x);
   x->cur = 1 - x->cur;
+  x->keysFull = x->keysNext;
+  x->keysNext = false;
   if (x->o.mode != MODE_LAGRANGE) x->x_then_y_n = !x->x_then_y_n;
 }
 
@@ -744,12 +755,14 @@ int runIteration(mhy_ctx* x) {
     if (x->dualBoth) {
       if ((st = phaseSweepStage(x, 1, MHY_STAGE_CELLS)) != MHY_OK) return st;
       if ((st = phaseSweepStage(x, 2, MHY_STAGE_CELLS)) != MHY_OK) return st;
+      // (the nodal remap reads the final sound speed and pressure)
+      if ((st = phaseFinal(x)) != MHY_OK) return st;
       if ((st = phaseDualBoth(x)) != MHY_OK) return st;
     } else {
       if ((st = phaseSweep(x, 1)) != MHY_OK) return st;
       if ((st = phaseSweep(x, 2)) != MHY_OK) return st;
+      if ((st = phaseFinal(x)) != MHY_OK) return st;
     }
-    if ((st = phaseFinal(x)) != MHY_OK) return st;
   }
   x->iteration++;
   return MHY_OK;
@@ -861,6 +874,16 @@ double* fieldPtr(mhy_ctx* x, int field, long& n) {
 extern "C" {
 
 const char* mhy_last_error(const mhy_ctx* x) { return x ? x->err.c_str() : "null context"; }
+
+// node rows per band of the nodal remap of both sweeps (MAHYCO_DUAL_ROWS forces
+// 2, 4, 8, 16 or 32)
+static int pickDualRows(long waves2) {
+  if (const char* e = std::getenv("MAHYCO_DUAL_ROWS")) {
+    const int r = std::atoi(e);
+    if (r == 2 || r == 4 || r == 8 || r == 16 || r == 32) return r;
+  }
+  return dualBothRows(waves2);
+}
 
 // the limiter of the fixed-option sweeps of these options, or 0
 static int pickFixed(const Opts& o) {
@@ -1155,7 +1178,7 @@ static int createContext(const mhy_config* cfg, mhy_ctx** out, bool batchMember)
   o.flux_any = (b.flux_left + b.flux_right + b.flux_bottom + b.flux_top) > 0;
   x->fixLim = pickFixed(o);
   x->dualBoth = x->fixLim != 0 && x->sweepWave && !std::getenv("MAHYCO_DUAL_Y");
-  x->dualRows = dualBothRows(dualBothItems(c.nx, c.ny, 2, true));
+  x->dualRows = pickDualRows(dualBothItems(c.nx, c.ny, 2, true));
   if (x->dualBoth && x->tune.on) {  // no choice left at that site
     x->tune.ncand[0] = 0;
     x->tune.steps = 2 * mhy_ctx::kTuneRounds * (x->tune.ncand[1] + x->tune.ncand[2]);
@@ -1190,6 +1213,7 @@ static int createContext(const mhy_config* cfg, mhy_ctx** out, bool batchMember)
   } else {
     AD(f.vol[0], C);
     f.vol[1] = f.vol[0];  // Euler sub-volumes: constant
+    if (o.mode == MODE_FULL) AD(f.cvol, C);
   }
   for (int k = 0; k < m; ++k) AD(f.f_k[k], C), AR(f.mu_k[k], C), AD(f.M_k[k], C);
   AD(f.M, C);
@@ -1290,6 +1314,7 @@ static int createContext(const mhy_config* cfg, mhy_ctx** out, bool batchMember)
   {
     KP kp = makeKP(x);
     launchR(x, k_node_mass<double>, k_node_mass<float>, gridFor(N), dim3(kBlock), kp);
+    if (f.cvol) launchR(x, k_cfl_volume<double>, k_cfl_volume<float>, gridFor(C), dim3(kBlock), kp);
     if (hipStreamSynchronize(x->stream) != hipSuccess) return bail(fail(x, MHY_ERR_DEVICE, "node mass"));
   }
   x->init = HostInit();  // the host copy of the initial state is no longer needed
@@ -1359,13 +1384,15 @@ int captureStep(mhy_ctx* x) {
 // graphs is set, else eager launches.
 int stepOnce(mhy_ctx* x, bool graphs) {
   // no graph is captured before the tuner has fixed the kernel variants
-  if (!graphs || x->tune.on) return runIteration(x);
+  // nor from a state whose dt accumulators the reduction kernel has to fill first
+  if (!graphs || x->tune.on || (leavesDt(x) && !x->keysFull)) return runIteration(x);
   hipGraphExec_t& g = x->graph[2 * x->cur + (x->x_then_y_n ? 1 : 0)];
   if (!g) {
     const int st = captureStep(x);
     if (st != MHY_OK) return st;
   }
   HIPCHK(x, hipGraphLaunch(g, x->stream));
+  x->keysNext = leavesDt(x);
   x->iteration++;
   return MHY_OK;
 }
@@ -1507,6 +1534,11 @@ int mhy_set_field(mhy_ctx* x, int field, const double* in, long long n) {
   // that setting a mean field leaves the material fields as they were
   const int st = storeMaterialFields(x);
   if (st != MHY_OK) return st;
+  if (x->keysFull && !x->euc) {  // the time step of the new state is reduced again
+    launchR(x, k_dt_reset<double>, k_dt_reset<float>, dim3(1), dim3(64), makeKP(x));
+    HIPCHK(x, hipGetLastError());
+    x->keysFull = false;
+  }
   HIPCHK(x, hipStreamSynchronize(x->stream));
   if (x->mixed && isBulkField(field)) {
     std::vector<float> h(in, in + len);
@@ -1676,7 +1708,8 @@ int mhy_kernel_bytes(const mhy_ctx* x, int k, double* bytes) {
       break;
     }
     case K_DUAL:  // face fluxes of both sweeps, Lagrange velocity, Mp ; new velocity
-      w = 2.0 * F * m * d + N * 5 * r;
+      // and for the next dt cfl sqrt(vol), c, p
+      w = 2.0 * F * m * d + N * 5 * r + (dualBothDt(x->dualRows) ? C * (d + 2 * r) : 0.0);
       break;
     case K_DUAL_X:
     case K_DUAL_Y:
@@ -1880,10 +1913,12 @@ int batchFail(mhy_batch* b, int code, const std::string& msg) {
   return code;
 }
 
+bool batchLeavesDt(const mhy_batch* b) { return b->dualLim != 0 && dualBothDt(b->dualRows); }
+
 // one step of every problem with bulk storage type R; timing != 0 records
 // events around each launch
 template <class R>
-int batchEnqueueStepR(mhy_batch* b, int cur, bool xty, bool timing) {
+int batchEnqueueStepR(mhy_batch* b, int cur, bool xty, bool timing, bool reduce) {
   const int n = (int)b->ctx.size();
   // fnLoop walks contiguous virtual-block ranges (blocks[k] workgroups);
   // fnOne runs one workgroup per virtual block (blocks[k] == 0)
@@ -1900,7 +1935,8 @@ int batchEnqueueStepR(mhy_batch* b, int cur, bool xty, bool timing) {
     hipLaunchKernelGGL(fn, dim3(grid), dim3(block), 0, b->stream, bl);
     if (timing) (void)hipEventRecord(b->ev[2 * k + 1], b->stream);
   };
-  launch(BK_DT, k_dt_reduce_batch<R, false>, k_dt_reduce_batch<R, true>, cur);
+  // (the nodal remap of both sweeps leaves the next step's accumulators)
+  if (reduce) launch(BK_DT, k_dt_reduce_batch<R, false>, k_dt_reduce_batch<R, true>, cur);
   launch(BK_NODE, k_lagrange_node_batch<R, false>, k_lagrange_node_batch<R, true>, cur);
   static const Fn cellLoop[3] = {k_lagrange_cell_batch<R, 1, false>, k_lagrange_cell_batch<R, 2, false>,
                                  k_lagrange_cell_batch<R, 3, false>};
@@ -1924,7 +1960,7 @@ int batchEnqueueStepR(mhy_batch* b, int cur, bool xty, bool timing) {
              sweepBatchKernel<R, true>(xd, b->m, b->pp), v + 8 * fuse, sweepWaveBlock(xd, b->mixed, b->pp));
     if (b->dualLim) {
       if (sweep == 2)
-        launch(BK_DUAL, nullptr, dualBothBatchKernel<R>(b->dualLim, b->m, xty), cur);
+        launch(BK_DUAL, nullptr, dualBothBatchKernel<R>(b->dualLim, b->m, xty, b->dualRows), cur);
     } else if (xd) launch(BK_DUX, k_dual_wave_batch<R, true, false>, k_dual_wave_batch<R, true, true>, v);
     else if (b->dualWaveY)
       launch(BK_DUY, k_dual_wave_batch<R, false, false>, k_dual_wave_batch<R, false, true>, v, dualWaveBlock(false, b->mixed));
@@ -1934,8 +1970,10 @@ int batchEnqueueStepR(mhy_batch* b, int cur, bool xty, bool timing) {
   return e == hipSuccess ? MHY_OK : batchFail(b, MHY_ERR_DEVICE, std::string("batch launch: ") + hipGetErrorString(e));
 }
 
-int batchEnqueueStep(mhy_batch* b, int cur, bool xty, bool timing) {
-  return b->mixed ? batchEnqueueStepR<float>(b, cur, xty, timing) : batchEnqueueStepR<double>(b, cur, xty, timing);
+// reduce: the dt reduction kernel runs first
+int batchEnqueueStep(mhy_batch* b, int cur, bool xty, bool timing, bool reduce) {
+  return b->mixed ? batchEnqueueStepR<float>(b, cur, xty, timing, reduce)
+                  : batchEnqueueStepR<double>(b, cur, xty, timing, reduce);
 }
 
 // captures the two step parities of the lock-step ensemble as graphs:
@@ -1946,7 +1984,7 @@ int batchCapture(mhy_batch* b) {
     hipGraph_t g = nullptr;
     if (hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal) != hipSuccess)
       return batchFail(b, MHY_ERR_DEVICE, "graph capture begin");
-    int st = batchEnqueueStep(b, c, xty, false);
+    int st = batchEnqueueStep(b, c, xty, false, !batchLeavesDt(b));
     hipError_t e = hipStreamEndCapture(b->stream, &g);
     if (st != MHY_OK) return st;
     if (e != hipSuccess) return batchFail(b, MHY_ERR_DEVICE, std::string("graph capture: ") + hipGetErrorString(e));
@@ -2019,7 +2057,7 @@ int mhy_batch_create(const mhy_config* cfgs, int n, mhy_batch** out) {
   std::vector<KP> table((size_t)kVariants * n);
   long waves2 = 0;
   for (const mhy_ctx* x : b->ctx) waves2 += dualBothItems(x->o.nx, x->o.ny, 2, true);
-  b->dualRows = dualBothRows(waves2);
+  b->dualRows = pickDualRows(waves2);
   for (int v = 0; v < kVariants; ++v)
     for (int i = 0; i < n; ++i) {
       KP kp = makeKP(b->ctx[i]);
@@ -2115,15 +2153,22 @@ int mhy_batch_context(mhy_batch* b, int i, mhy_ctx** ctx) {
 int mhy_batch_run(mhy_batch* b, int nsteps) {
   if (!b || nsteps < 0) return MHY_ERR_ARG;
   if (b->ctx.empty() || !b->dTable) return MHY_ERR_ARG;
+  // the accumulators hold every problem's state after a step that leaves them,
+  // unless a field was written from the host since
+  const bool leaves = batchLeavesDt(b);
+  bool full = leaves;
+  for (const mhy_ctx* x : b->ctx) full = full && x->keysFull;
   for (int s = 0; s < nsteps; ++s) {
     int st;
+    const bool reduce = !full;
+    full = leaves;
     if (b->tuneStep < kTuneSteps) {
       // two consecutive steps (both sweep orders: a sweep kernel is sweep 1
       // in one and the heavier fused sweep 2 in the other) with every kernel
       // at candidate tuneStep / 2, timed
       const int cand = b->tuneStep / 2;
       for (int k = 0; k < BK_COUNT; ++k) b->blocks[k] = kCand[cand];
-      if ((st = batchEnqueueStep(b, b->cur, b->xty, true)) != MHY_OK) return st;
+      if ((st = batchEnqueueStep(b, b->cur, b->xty, true, reduce)) != MHY_OK) return st;
       if (hipStreamSynchronize(b->stream) != hipSuccess) return batchFail(b, MHY_ERR_DEVICE, "batch sync");
       const bool verbose = std::getenv("MAHYCO_BATCH_VERBOSE") != nullptr;
       for (int k = 0; k < BK_COUNT; ++k) {  // a kernel runs at most once per step
@@ -2137,12 +2182,12 @@ int mhy_batch_run(mhy_batch* b, int nsteps) {
         if (verbose)
           for (int k = 0; k < BK_COUNT; ++k) std::fprintf(stderr, "[batch tune] kernel %d -> %u\n", k, b->blocks[k]);
       }
-    } else if (b->useGraph) {
+    } else if (b->useGraph && !(reduce && leaves)) {
       if (!b->exec[0] && (st = batchCapture(b)) != MHY_OK) return st;
       if (hipGraphLaunch(b->exec[b->cur], b->stream) != hipSuccess)
         return batchFail(b, MHY_ERR_DEVICE, "graph launch");
     } else {
-      if ((st = batchEnqueueStep(b, b->cur, b->xty, false)) != MHY_OK) return st;
+      if ((st = batchEnqueueStep(b, b->cur, b->xty, false, reduce)) != MHY_OK) return st;
     }
     b->cur = 1 - b->cur;
     b->xty = !b->xty;
@@ -2156,6 +2201,7 @@ int mhy_batch_run(mhy_batch* b, int nsteps) {
     x->cur = b->cur;
     x->x_then_y_n = b->xty;
     x->iteration = (int)b->iteration;
+    if (nsteps > 0) x->keysFull = full;
     Scalars sc;
     if (hipMemcpy(&sc, x->f.sc, sizeof(Scalars), hipMemcpyDeviceToHost) != hipSuccess)
       return batchFail(b, MHY_ERR_DEVICE, "batch scalars");

@@ -5,7 +5,7 @@
 // One sweep at a time the nodal remap is bound by memory: it stores the nodal
 // momentum and mass and the Lagrange coordinate of the second axis for the
 // next sweep to read back, 8 of the 15 array passes of the pair.  Here a wave
-// covers 64 node columns (60 updated) and walks down a band of node rows: the
+// covers 64 node columns (59 or 58 updated) and walks down a band of node rows: the
 // row-wise sweep works on one node row, its along-x neighbours being the
 // adjacent lanes (DPP moves), and the column-wise sweep on the rows the wave
 // keeps in registers.  A classic limiter's gradient needs one neighbour on
@@ -15,6 +15,13 @@
 // sweeps, and the new velocity.  The Lagrange velocity has a buffer of its own
 // (kp.ul, kp.vl): the kernel writes the new one while other waves still read
 // the old in their halo.
+//
+// DT: the new velocity in registers also serves the next step's time step: the wave
+// forms the CFL ratio of the cells between its node rows (with the sound speed
+// and pressure the second cell sweep has stored) and adds its minimum and the
+// maximum pressure to the next step's accumulators, with one node column and one
+// row more of halo, instead of the reduction kernel, which reads the velocity back
+// and forms the speed of each node four times.
 //
 // Each dual face is formed once, by the node after it: the mass flux through
 // it (the two sides' fluxes are the same sum) and the upwind velocity, which
@@ -40,8 +47,10 @@ constexpr int kBHalo = 2;
 // takes the y faces left of a node from the lane before
 template <bool XFIRST>
 constexpr int kBLeft = XFIRST ? kBHalo : kBHalo + 1;
-template <bool XFIRST>
-constexpr int kBOut = 64 - kBHalo - kBLeft<XFIRST>;  // node columns updated per wave
+// node columns updated per wave: with DT the new velocity is also formed one
+// column further, for the cells right of the last updated column
+template <bool XFIRST, bool DT>
+constexpr int kBOut = (DT ? 63 : 64) - kBHalo - kBLeft<XFIRST>;
 
 // value of the lane before / after (the end lanes keep their own)
 template <class V>
@@ -91,13 +100,13 @@ __device__ __forceinline__ T slope(T gp, T gm) {
 }  // namespace
 
 // item: column group and band of this wave (kp.dualRows node rows per band)
-template <class R, int M, int LIM, bool XFIRST>
+template <class R, int M, int LIM, bool XFIRST, bool DT>
 __device__ __forceinline__ void dualBothBody(const KPT<R>& kp, int item) {
   using T = typename std::conditional<kMixed<R>, float, double>::type;
   const Opts& o = kp.o;
   const auto& f = kp.f;
   const int nx = o.nx, ny = o.ny;
-  constexpr int kOut = kBOut<XFIRST>, kLeft = kBLeft<XFIRST>;
+  constexpr int kOut = kBOut<XFIRST, DT>, kLeft = kBLeft<XFIRST>;
   const int groups = (nx + 1 + kOut - 1) / kOut;
   const int rows = kp.dualRows;
   if (item >= groups * ((ny + 1 + rows - 1) / rows)) return;  // the whole wave
@@ -105,7 +114,7 @@ __device__ __forceinline__ void dualBothBody(const KPT<R>& kp, int item) {
   const int t = (item % groups) * kOut - kLeft + lane;
   const int a0 = (item / groups) * rows;
   const int a1 = (a0 + rows - 1 < ny) ? a0 + rows - 1 : ny;
-  const bool output = lane >= kLeft && lane < 64 - kBHalo && t <= nx;
+  const bool output = lane >= kLeft && lane < kLeft + kOut && t <= nx;
   const bool intX = t > 0 && t < nx;  // interior along x
   // lanes and rows outside the domain read the nearest node or cell inside:
   // finite values that no updated node uses
@@ -118,6 +127,10 @@ __device__ __forceinline__ void dualBothBody(const KPT<R>& kp, int item) {
   double* const* Gy = XFIRST ? f.G2 : f.G;
   // means over the faces a dual face touches: 2 per cell row (column)
   const double wy = (t >= 1 && t <= nx - 1) ? 0.25 : 0.5;
+
+  // with DT the walk starts one row early: the cells below the first updated
+  // node row belong to this band
+  const int first = a0 - kBHalo - (DT ? 1 : 0);
 
   // what row r of the walk reads: its nodes, the x faces of cell row r and the
   // y faces of row r - 1 (x first), resp. of the rows the updates need
@@ -151,7 +164,7 @@ __device__ __forceinline__ void dualBothBody(const KPT<R>& kp, int item) {
 #pragma unroll
   for (int k = 0; k < M; ++k) qx[k] = gyP[k] = 0.0;
   if constexpr (XFIRST) {  // the cell row below the first node row of the walk
-    const int c0 = a0 - kBHalo - 1;
+    const int c0 = first - 1;
 #pragma unroll
     for (int k = 0; k < M; ++k) {
       const double g = at(Gx[k], (long)(c0 < 0 ? 0 : c0) * (nx + 1) + tn);
@@ -190,10 +203,17 @@ __device__ __forceinline__ void dualBothBody(const KPT<R>& kp, int item) {
     return updateNode(U, flux, after(flux), um, up, intX);
   };
 
-  Row nextRow = load(a0 - kBHalo);
-  for (int r = a0 - kBHalo; r <= a1 + kBHalo; ++r) {
+  double vmin = DBL_MAX, pmax = -DBL_MAX, spA = 0.0;
+  Row nextRow = load(first);
+  for (int r = first; r <= a1 + kBHalo; ++r) {
     const Row w = nextRow;
     if (r < a1 + kBHalo) nextRow = load(r + 1);
+    // the cell row between node rows r - 3 and r - 2, for the time step
+    double cvol = 0.0, cs = 0.0, pc = 0.0;
+    if constexpr (DT) {
+      const long cd = (long)(r - 3 < 0 ? 0 : (r - 3 > ny - 1 ? ny - 1 : r - 3)) * nx + tc;
+      cvol = at(f.cvol, cd), cs = (double)at(f.c[kp.nxt], cd), pc = (double)at(f.p[kp.nxt], cd);
+    }
     const double ux1 = (double)w.u, uy1 = (double)w.v, Mp = (double)w.m;
     Nodal U = {Mp * ux1, Mp * uy1, Mp};
     Vel<T> ph = {T(ux1), T(uy1)};
@@ -226,33 +246,70 @@ __device__ __forceinline__ void dualBothBody(const KPT<R>& kp, int item) {
       const Vel<T> p2 = {T(V.x / V.m), T(V.y / V.m)};
       V = sweepX(p2, xl, V, fluxX(w.gx, a));
     }
+    // remapVariables, nodes (PhaseRemapFinal.cc:207-234)
+    const R vx = (R)(V.x / V.m), vy = (R)(V.y / V.m);
     if (output && a >= a0 && a <= a1) {
-      // remapVariables, nodes (PhaseRemapFinal.cc:207-234)
       const long p = (long)a * (nx + 1) + t;
-      at(f.ux[kp.nxt], p) = V.x / V.m;
-      at(f.uy[kp.nxt], p) = V.y / V.m;
+      at(f.ux[kp.nxt], p) = vx;
+      at(f.uy[kp.nxt], p) = vy;
+    }
+    if constexpr (DT) {
+      // computeDeltaT (VnrRemap.cc:14-50) of the cell between node rows a-1 and
+      // a, in the reduction kernel's order of the four nodes
+      const double wx = (double)vx, wv = (double)vy;
+      const double sp = sqrt(wx * wx + wv * wv) * 0.25;
+      const double spAr = after(spA), spr = after(sp);
+      if (output && t < nx && a >= 1 && a >= a0 && a <= a1) {
+        const double uc = ((0.0 + spA + spAr) + spr) + sp;
+        vmin = smin(vmin, cvol / (o.cfl_euler * uc + cs));
+        pmax = (pc > pmax) ? pc : pmax;
+      }
+      spA = sp;
     }
     phA = phB, phB = ph, gA = gB, dB = dN;
     ylA = ylB, ylB = yl, fluxA = fluxB, upA = upB;
     UA = UB, UB = U;
   }
+  // the wave's extrema into the next step's accumulators (a slot that already
+  // holds a better value is left alone: it only improves)
+  if constexpr (!DT) return;
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    vmin = smin(vmin, __shfl_xor(vmin, off, 64));
+    const double v = __shfl_xor(pmax, off, 64);
+    pmax = (v > pmax) ? v : pmax;
+  }
+  if (lane == 0) {
+    unsigned long long* slot = f.keys->k[kp.nxt][item % kDtSlots];
+    const unsigned long long lo = dkeyPos(vmin), hi = dkeySigned(pmax);
+    if (lo < __hip_atomic_load(&slot[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMin(&slot[0], lo);
+    if (hi > __hip_atomic_load(&slot[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(&slot[1], hi);
+  }
 }
 
 // (a wave past the last band leaves at once: the kernel has no barrier)
-template <class R, int M, int LIM, bool XFIRST>
+template <class R, int M, int LIM, bool XFIRST, bool DT>
 __global__ __launch_bounds__(256) void k_dual_both(KPT<R> kp) {
-  dualBothBody<R, M, LIM, XFIRST>(kp, (int)(blockIdx.x * 4 + (threadIdx.x >> 6)));
+  dualBothBody<R, M, LIM, XFIRST, DT>(kp, (int)(blockIdx.x * 4 + (threadIdx.x >> 6)));
 }
 // all problems of an ensemble in one launch, one workgroup per virtual block
-template <class R, int M, int LIM, bool XFIRST>
+template <class R, int M, int LIM, bool XFIRST, bool DT>
 __global__ __launch_bounds__(256) void k_dual_both_batch(BatchLaunchT<R> bl) {
   batchRun<true>(bl, [&](const KPT<R>& kp, unsigned local, unsigned, unsigned) {
-    dualBothBody<R, M, LIM, XFIRST>(kp, (int)(local * 4 + (threadIdx.x >> 6)));
+    dualBothBody<R, M, LIM, XFIRST, DT>(kp, (int)(local * 4 + (threadIdx.x >> 6)));
   });
 }
 
+// The next step's CFL reduction rides along in bands of at least 16 rows, where
+// its extra halo row is cheap (us per step, in the kernel / as a kernel of its own:
+// 4096^2 1790 / 1809, 1531x1021 220 / 226); a mesh of shorter bands is bound by the
+// length of the walk, and the reduction kernel overlaps nothing but takes less
+// than the longer walk (256^2 45.5 / 43.4, 1173x391 164 / 159).
+bool dualBothDt(int rows) { return rows >= 16; }
+
 int dualBothItems(long nx, long ny, int rows, bool xfirst) {
-  const long out = xfirst ? kBOut<true> : kBOut<false>;
+  const long out = dualBothDt(rows) ? (xfirst ? kBOut<true, true> : kBOut<false, true>)
+                                    : (xfirst ? kBOut<true, false> : kBOut<false, false>);
   return (int)((nx + 1 + out - 1) / out * ((ny + 1 + rows - 1) / rows));
 }
 
@@ -274,31 +331,35 @@ int dualBothRows(long waves2) {
 
 namespace {
 template <class R, int M, int LIM>
-SweepFn<R> pick(bool xfirst) {
-  return xfirst ? k_dual_both<R, M, LIM, true> : k_dual_both<R, M, LIM, false>;
+SweepFn<R> pick(bool xfirst, bool dt) {
+  if (dt) return xfirst ? k_dual_both<R, M, LIM, true, true> : k_dual_both<R, M, LIM, false, true>;
+  return xfirst ? k_dual_both<R, M, LIM, true, false> : k_dual_both<R, M, LIM, false, false>;
 }
 template <class R, int M, int LIM>
-SweepBatchFn<R> pickBatch(bool xfirst) {
-  return xfirst ? k_dual_both_batch<R, M, LIM, true> : k_dual_both_batch<R, M, LIM, false>;
+SweepBatchFn<R> pickBatch(bool xfirst, bool dt) {
+  if (dt) return xfirst ? k_dual_both_batch<R, M, LIM, true, true> : k_dual_both_batch<R, M, LIM, false, true>;
+  return xfirst ? k_dual_both_batch<R, M, LIM, true, false> : k_dual_both_batch<R, M, LIM, false, false>;
 }
 }  // namespace
 template <class R>
-SweepFn<R> dualBothKernel(int lim, int m, bool xf) {
+SweepFn<R> dualBothKernel(int lim, int m, bool xf, int rows) {
+  const bool dt = dualBothDt(rows);
   const bool mm = lim == MHY_LIM_MINMOD;
-  if (m == 1) return mm ? pick<R, 1, MHY_LIM_MINMOD>(xf) : pick<R, 1, MHY_LIM_SUPERBEE>(xf);
-  if (m == 2) return mm ? pick<R, 2, MHY_LIM_MINMOD>(xf) : pick<R, 2, MHY_LIM_SUPERBEE>(xf);
-  return mm ? pick<R, 3, MHY_LIM_MINMOD>(xf) : pick<R, 3, MHY_LIM_SUPERBEE>(xf);
+  if (m == 1) return mm ? pick<R, 1, MHY_LIM_MINMOD>(xf, dt) : pick<R, 1, MHY_LIM_SUPERBEE>(xf, dt);
+  if (m == 2) return mm ? pick<R, 2, MHY_LIM_MINMOD>(xf, dt) : pick<R, 2, MHY_LIM_SUPERBEE>(xf, dt);
+  return mm ? pick<R, 3, MHY_LIM_MINMOD>(xf, dt) : pick<R, 3, MHY_LIM_SUPERBEE>(xf, dt);
 }
 template <class R>
-SweepBatchFn<R> dualBothBatchKernel(int lim, int m, bool xf) {
+SweepBatchFn<R> dualBothBatchKernel(int lim, int m, bool xf, int rows) {
+  const bool dt = dualBothDt(rows);
   const bool mm = lim == MHY_LIM_MINMOD;
-  if (m == 1) return mm ? pickBatch<R, 1, MHY_LIM_MINMOD>(xf) : pickBatch<R, 1, MHY_LIM_SUPERBEE>(xf);
-  if (m == 2) return mm ? pickBatch<R, 2, MHY_LIM_MINMOD>(xf) : pickBatch<R, 2, MHY_LIM_SUPERBEE>(xf);
-  return mm ? pickBatch<R, 3, MHY_LIM_MINMOD>(xf) : pickBatch<R, 3, MHY_LIM_SUPERBEE>(xf);
+  if (m == 1) return mm ? pickBatch<R, 1, MHY_LIM_MINMOD>(xf, dt) : pickBatch<R, 1, MHY_LIM_SUPERBEE>(xf, dt);
+  if (m == 2) return mm ? pickBatch<R, 2, MHY_LIM_MINMOD>(xf, dt) : pickBatch<R, 2, MHY_LIM_SUPERBEE>(xf, dt);
+  return mm ? pickBatch<R, 3, MHY_LIM_MINMOD>(xf, dt) : pickBatch<R, 3, MHY_LIM_SUPERBEE>(xf, dt);
 }
-template SweepFn<double> dualBothKernel<double>(int, int, bool);
-template SweepFn<float> dualBothKernel<float>(int, int, bool);
-template SweepBatchFn<double> dualBothBatchKernel<double>(int, int, bool);
-template SweepBatchFn<float> dualBothBatchKernel<float>(int, int, bool);
+template SweepFn<double> dualBothKernel<double>(int, int, bool, int);
+template SweepFn<float> dualBothKernel<float>(int, int, bool, int);
+template SweepBatchFn<double> dualBothBatchKernel<double>(int, int, bool, int);
+template SweepBatchFn<float> dualBothBatchKernel<float>(int, int, bool, int);
 
 }  // namespace mhy

@@ -25,6 +25,10 @@ __global__ void k_dt_reduce(KPT<R> kp);
 template <class R>
 __global__ void k_dt_finalize(KPT<R> kp);
 template <class R>
+__global__ void k_cfl_volume(KPT<R> kp);
+template <class R>
+__global__ void k_dt_reset(KPT<R> kp);
+template <class R>
 __global__ void k_dt_hold(KPT<R> kp);
 template <class R>
 __global__ void k_lagrange_node(KPT<R> kp);
@@ -108,11 +112,12 @@ unsigned dualWaveBlock(bool xd, bool mixed);
 // fixedLimiter), on bands of dualBothRows(waves at 2 rows) node
 // rows; dualBothItems: waves in all
 template <class R>
-SweepFn<R> dualBothKernel(int lim, int m, bool xfirst);
+SweepFn<R> dualBothKernel(int lim, int m, bool xfirst, int rows);
 template <class R>
-SweepBatchFn<R> dualBothBatchKernel(int lim, int m, bool xfirst);
+SweepBatchFn<R> dualBothBatchKernel(int lim, int m, bool xfirst, int rows);
 int dualBothItems(long nx, long ny, int rows, bool xfirst);
 int dualBothRows(long waves2);
+bool dualBothDt(int rows);  // the kernel also reduces the next step's dt
 template <class R, int M>
 __global__ void k_remap_final(KPT<R> kp);
 template <class R>

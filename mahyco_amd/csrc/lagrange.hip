@@ -62,7 +62,9 @@ __device__ __forceinline__ void dtReduceBody(const KPT<R>& kp, unsigned b, unsig
       const double a = ux[nd[s]], b = uy[nd[s]];
       uc += sqrt(a * a + b * b) * 0.25;
     }
-    const double v = o.cfl * sqrt(f.vol[kp.cur][c]) / (o.cfl_euler * uc + (double)f.c[kp.cur][c]);
+    // (the numerator of the fixed cells is formed once, at set-up)
+    const double cv = f.cvol ? f.cvol[c] : o.cfl * sqrt(f.vol[kp.cur][c]);
+    const double v = cv / (o.cfl_euler * uc + (double)f.c[kp.cur][c]);
     vmin = smin(vmin, v);
     const double pc = f.p[kp.cur][c];
     pm = (pc > pm) ? pc : pm;
@@ -126,6 +128,21 @@ __device__ __forceinline__ double dtForNodes(const KPT<R>& kp, bool first) {
   const DtNow d = dtFold(kp.f, kp.cur);
   if (first) dtStore(kp.f, kp.cur, kp.nxt, d);
   return d.dt1;
+}
+
+// cfl sqrt(vol) of the fixed Euler cells (set-up)
+template <class R>
+__global__ __launch_bounds__(256) void k_cfl_volume(KPT<R> kp) {
+  const long c = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (c < kp.ncell) kp.f.cvol[c] = kp.o.cfl * sqrt(kp.f.vol[0][c]);
+}
+// empties the accumulators of the current parity
+template <class R>
+__global__ void k_dt_reset(KPT<R> kp) {
+  if (threadIdx.x < kDtSlots && blockIdx.x == 0) {
+    kp.f.keys->k[kp.cur][threadIdx.x][0] = dkeyPos(DBL_MAX);
+    kp.f.keys->k[kp.cur][threadIdx.x][1] = dkeySigned(-DBL_MAX);
+  }
 }
 
 template <class R>
@@ -376,6 +393,8 @@ __global__ __launch_bounds__(256) void k_lagrange_cell_batch(BatchLaunchT<R> bl)
 #define MHY_LAGRANGE_INST(R)                                                 \
   template __global__ void k_dt_reduce<R>(KPT<R>);                           \
   template __global__ void k_dt_finalize<R>(KPT<R>);                         \
+  template __global__ void k_cfl_volume<R>(KPT<R>);                          \
+  template __global__ void k_dt_reset<R>(KPT<R>);                            \
   template __global__ void k_dt_hold<R>(KPT<R>);                             \
   template __global__ void k_lagrange_node<R>(KPT<R>);                       \
   template __global__ void k_lagrange_node_euler<R>(KPT<R>);                 \
