@@ -131,6 +131,7 @@ struct mhy_ctx {
   // face fluxes in buffers of their own.
   bool dualBoth = false;
   int dualRows = 32;  // node rows per band
+  int nodeRows = 1;   // node rows per band of the node update
   // nodal remap along y on LDS tiles of 16 node columns x dualTileRows
   // rows: 48 (MAHYCO_DUAL_Y=tile), 32 or 64 (tile32, tile64)
   bool dualTileY = false;
@@ -269,6 +270,7 @@ KP makeKP(const mhy_ctx* x) {
   kp.nnode = x->nnode;
   setLagrangeVelocity(kp);
   kp.dualRows = x->dualRows;
+  kp.nodeRows = x->nodeRows;
   return kp;
 }
 
@@ -526,13 +528,10 @@ bool lagFused(const mhy_ctx* x) { return x->fuseLag && (x->x_then_y_n || x->fuse
 int phaseLagrange(mhy_ctx* x) {
   if (x->euc) return phaseEucLagrange(x);
   KP kp = makeKP(x);
-  // interior rows, then enough rows of blocks for the boundary nodes (a
-  // grid's y dimension holds at most 65535)
-  const long gx = (x->o.nx - 1 + kBlock - 1) / kBlock, nedge = 2L * (x->o.nx + 1) + 2L * (x->o.ny - 1);
-  const long rows = x->o.ny - 1 + (nedge + gx * kBlock - 1) / std::max(gx * kBlock, 1L);
-  if (x->o.mode == MODE_FULL && x->o.nx >= 2 && x->o.ny >= 2 && rows <= 65535 && x->splitNode) {
+  if (x->o.mode == MODE_FULL && x->splitNode) {
+    const int items = nodeWalkItems(x->o.nx, x->o.ny, x->nodeRows);
     timed(x, K_NODE, [&] {
-      launchR(x, k_lagrange_node_euler<double>, k_lagrange_node_euler<float>, dim3((unsigned)gx, (unsigned)rows),
+      launchR(x, k_lagrange_node_walk<double>, k_lagrange_node_walk<float>, dim3((unsigned)((items + 3) / 4)),
               dim3(kBlock), kp);
     });
   } else {
@@ -1179,6 +1178,7 @@ static int createContext(const mhy_config* cfg, mhy_ctx** out, bool batchMember)
   x->fixLim = pickFixed(o);
   x->dualBoth = x->fixLim != 0 && x->sweepWave && !std::getenv("MAHYCO_DUAL_Y");
   x->dualRows = pickDualRows(dualBothItems(c.nx, c.ny, 2, true));
+  x->nodeRows = nodeWalkRows(nodeWalkItems(c.nx, c.ny, 1));
   if (x->dualBoth && x->tune.on) {  // no choice left at that site
     x->tune.ncand[0] = 0;
     x->tune.steps = 2 * mhy_ctx::kTuneRounds * (x->tune.ncand[1] + x->tune.ncand[2]);
@@ -1886,6 +1886,7 @@ struct mhy_batch {
   int fixLim = 0;         // limited slopes: every problem has this fixed limiter (fixedLimiter), or 0
   int dualLim = 0;        // the same with PenteBorne too: nodal remap of both sweeps in one kernel
   int dualRows = 32;      // node rows per band of that kernel
+  int nodeRows = 1;       // node rows per band of the node update
   void* dTable = nullptr;  // KPT<double> or KPT<float> entries
   unsigned* dStart = nullptr;  // BK_COUNT x (n+1)
   unsigned* dGx = nullptr;     // BK_COUNT x n
@@ -1937,7 +1938,7 @@ int batchEnqueueStepR(mhy_batch* b, int cur, bool xty, bool timing, bool reduce)
   };
   // (the nodal remap of both sweeps leaves the next step's accumulators)
   if (reduce) launch(BK_DT, k_dt_reduce_batch<R, false>, k_dt_reduce_batch<R, true>, cur);
-  launch(BK_NODE, k_lagrange_node_batch<R, false>, k_lagrange_node_batch<R, true>, cur);
+  launch(BK_NODE, nullptr, k_lagrange_node_batch<R>, cur);
   static const Fn cellLoop[3] = {k_lagrange_cell_batch<R, 1, false>, k_lagrange_cell_batch<R, 2, false>,
                                  k_lagrange_cell_batch<R, 3, false>};
   static const Fn cellOne[3] = {k_lagrange_cell_batch<R, 1, true>, k_lagrange_cell_batch<R, 2, true>,
@@ -2058,6 +2059,9 @@ int mhy_batch_create(const mhy_config* cfgs, int n, mhy_batch** out) {
   long waves2 = 0;
   for (const mhy_ctx* x : b->ctx) waves2 += dualBothItems(x->o.nx, x->o.ny, 2, true);
   b->dualRows = pickDualRows(waves2);
+  long waves1 = 0;
+  for (const mhy_ctx* x : b->ctx) waves1 += nodeWalkItems(x->o.nx, x->o.ny, 1);
+  b->nodeRows = nodeWalkRows(waves1);
   for (int v = 0; v < kVariants; ++v)
     for (int i = 0; i < n; ++i) {
       KP kp = makeKP(b->ctx[i]);
@@ -2069,6 +2073,7 @@ int mhy_batch_create(const mhy_config* cfgs, int n, mhy_batch** out) {
       kp.dtFold = 1;
       setLagrangeVelocity(kp);
       kp.dualRows = b->dualRows;
+      kp.nodeRows = b->nodeRows;
       table[(size_t)v * n + i] = kp;
     }
   // virtual-block layout of every kernel
@@ -2083,7 +2088,7 @@ int mhy_batch_create(const mhy_config* cfgs, int n, mhy_batch** out) {
         case BK_DT:  // a few cells per thread: fewer, longer virtual blocks
           g = dim3((unsigned)std::min<long>(kReduceBlocks, (x->ncell + 4 * kBlock - 1) / (4 * kBlock)));
           break;
-        case BK_NODE: g = gridFor(x->nnode); break;
+        case BK_NODE: g = dim3((unsigned)((nodeWalkItems(nx, ny, b->nodeRows) + 3) / 4)); break;
         case BK_CELL: g = gridFor(x->ncell); break;
         case BK_SWX: g = b->o3 ? sweepO3Grid(true, nx, ny) : sweepWaveGrid(true, nx, ny, b->mixed, b->pp); break;
         case BK_SWY:

@@ -32,15 +32,18 @@ template <class R>
 __global__ void k_dt_hold(KPT<R> kp);
 template <class R>
 __global__ void k_lagrange_node(KPT<R> kp);
-// the same node update on the fixed Euler grid, laid out by node row
+// the same node update on the fixed Euler grid, in bands of nodeWalkRows(waves
+// at one row) node rows; nodeWalkItems: waves in all
 template <class R>
-__global__ void k_lagrange_node_euler(KPT<R> kp);
+__global__ void k_lagrange_node_walk(KPT<R> kp);
+template <class R>
+__global__ void k_lagrange_node_batch(BatchLaunchT<R> bl);
+int nodeWalkItems(long nx, long ny, int rows);
+int nodeWalkRows(long waves1);
 template <class R, int M>
 __global__ void k_lagrange_cell(KPT<R> kp);
 template <class R, bool ONE>
 __global__ void k_dt_reduce_batch(BatchLaunchT<R> bl);
-template <class R, bool ONE>
-__global__ void k_lagrange_node_batch(BatchLaunchT<R> bl);
 template <class R, int M, bool ONE>
 __global__ void k_lagrange_cell_batch(BatchLaunchT<R> bl);
 template <class R, int M, bool PP, bool XD, bool ONE, class P>

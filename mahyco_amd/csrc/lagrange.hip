@@ -249,50 +249,15 @@ __device__ __forceinline__ void lagrangeNodeAt(const KPT<R>& kp, double dt1, lon
   }
 }
 
-// Interior node (j, i) of the fixed Euler grid (MODE_FULL): the four cells
-// exist and the corner normals are the raw half-edge sums.  The same operands
-// in the same order as lagrangeNodeAt, so the results are bitwise its own.
-template <class R>
-__device__ __forceinline__ void lagrangeNodeInner(const KPT<R>& kp, double dt1, int j, int i) {
-  const Opts& o = kp.o;
-  const auto& f = kp.f;
-  const int nx = o.nx;
-  const int p = j * (nx + 1) + i;
-  const int c0 = j * nx + i;  // cells (j, i), (j, i-1), (j-1, i), (j-1, i-1)
-  const int cc[4] = {c0, c0 - 1, c0 - nx, c0 - nx - 1};
-  double msum = 0.0;
-#pragma unroll
-  for (int q = 0; q < 4; ++q) msum = msum + f.M[cc[q]];
-  const double Mp = msum / 4.0;
-  f.Mp[p] = Mp;
-  const double uxn = (double)f.ux[kp.cur][p], uyn = (double)f.uy[kp.cur][p];
-  const double dt = 0.5 * (dt1 + f.sc->dt[kp.cur]);
-  const D2 X0 = eulerNode(o, j, i);
-  const D2 Cn[4] = {lpcNpcAxis(X0, eulerNode(o, j, i + 1), eulerNode(o, j + 1, i)),
-                    lpcNpcAxis(X0, eulerNode(o, j + 1, i), eulerNode(o, j, i - 1)),
-                    lpcNpcAxis(X0, eulerNode(o, j - 1, i), eulerNode(o, j, i + 1)),
-                    lpcNpcAxis(X0, eulerNode(o, j, i - 1), eulerNode(o, j - 1, i))};
-  D2 r = {0.0, 0.0};
-#pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    const double pq = (double)f.p[kp.cur][cc[q]] + (double)f.q[kp.cur][cc[q]];
-    r = d2add(r, d2mul(Cn[q], pq));
-  }
-  const D2 u1 = d2add(D2{uxn, uyn}, d2mul(r, dt / Mp));
-  kp.ul[p] = u1.x;
-  kp.vl[p] = u1.y;
-}
-
 // One thread per node, any mode (b: block index inside the problem).
 template <class R>
 __device__ __forceinline__ void lagrangeNodeBody(const KPT<R>& kp, unsigned b) {
   const double dt1 = dtForNodes(kp, b == 0 && threadIdx.x == 0);
   const long p = (long)b * blockDim.x + threadIdx.x;
   if (p >= kp.nnode) return;
-  const long nx = kp.o.nx, ny = kp.o.ny;
+  const long nx = kp.o.nx;
   const long j = (long)((unsigned)p / (unsigned)(nx + 1)), i = p - j * (nx + 1);
-  if (kp.o.mode == MODE_FULL && i > 0 && j > 0 && i < nx && j < ny) lagrangeNodeInner(kp, dt1, (int)j, (int)i);
-  else lagrangeNodeAt(kp, dt1, p, j, i);
+  lagrangeNodeAt(kp, dt1, p, j, i);
 }
 
 template <class R>
@@ -300,39 +265,110 @@ __global__ __launch_bounds__(256) void k_lagrange_node(KPT<R> kp) {
   lagrangeNodeBody(kp, blockIdx.x);
 }
 
-// The node update on the fixed Euler grid, laid out by position: blockIdx.y
-// < ny - 1 is one row of interior nodes (no index division, one test per
-// thread); the rows of blocks after them share the boundary nodes (bottom
-// row, top row, then the left and right columns without their corners), which
-// run the general body with its conditions.  One launch for both: as kernels of
-// their own the boundary nodes took 5 to 7 us on any mesh, and the time-step
-// finalize another 2 to 5 us; folded in here they overlap the interior rows
-// (one step of 256^2 cells 60.8 -> 55.8 us, of 500 x 333 cells with PenteBorne
-// 112 -> 103 us, the accumulators in lines of their own included).
+// The node update on the fixed Euler grid (MODE_FULL).  A wave takes 64 interior
+// node columns and walks up a band of kp.nodeRows node rows: each row's cell
+// masses and pressures are read once and serve the node rows below and above
+// it; the waves after the last band take 64 boundary nodes each (bottom row,
+// top row, then the left and right columns without their corners) through the
+// general body with its conditions.  Interior nodes have four cells, and the
+// corner normals are the raw half-edge sums; operands and order are those of
+// lagrangeNodeAt, so the results are bitwise its own.
+//
+// Bound by memory on large meshes (8 array passes in FP64) and by the latency of
+// the chain keys -> dt -> update on small ones; the cell loads come before the
+// fold so that the two overlap.  One launch does the whole of it: a finalize
+// kernel (2 to 5 us) and a boundary-node kernel (5 to 7 us) of their own cost
+// 4.9 us of a 256^2 step; one thread per interior node reading its four cells took
+// 27 us on 1531x1021 cells and 244 us in the 64-problem mixed ensemble, whose steps
+// went from 220 to 215 us and from 2945 to 2855 us.
 template <class R>
-__global__ __launch_bounds__(256) void k_lagrange_node_euler(KPT<R> kp) {
-  const int nx = kp.o.nx, ny = kp.o.ny;
-  const double dt1 = dtForNodes(kp, blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0);
-  if ((int)blockIdx.y < ny - 1) {
-    const int i = 1 + (int)(blockIdx.x * blockDim.x + threadIdx.x);
-    if (i < nx) lagrangeNodeInner(kp, dt1, 1 + (int)blockIdx.y, i);
+__device__ __forceinline__ void lagrangeNodeWalk(const KPT<R>& kp, int item) {
+  const Opts& o = kp.o;
+  const auto& f = kp.f;
+  const int nx = o.nx, ny = o.ny, rows = kp.nodeRows;
+  const int lane = threadIdx.x & 63;
+  const int groups = (nx - 1 + 63) / 64, bands = (ny - 1 + rows - 1) / rows;
+  const bool first = (item == 0 && lane == 0);
+  if (item >= groups * bands) {
+    const int e = (item - groups * bands) * 64 + lane;
+    const double dt1 = dtForNodes(kp, first);
+    int j, i;
+    if (e < nx + 1) {
+      j = 0, i = e;
+    } else if (e < 2 * (nx + 1)) {
+      j = ny, i = e - (nx + 1);
+    } else if (e < 2 * (nx + 1) + (ny - 1)) {
+      j = 1 + (e - 2 * (nx + 1)), i = 0;
+    } else if (e < 2 * (nx + 1) + 2 * (ny - 1)) {
+      j = 1 + (e - 2 * (nx + 1) - (ny - 1)), i = nx;
+    } else {
+      return;
+    }
+    lagrangeNodeAt(kp, dt1, (long)j * (nx + 1) + i, j, i);
     return;
   }
-  const int e = (((int)blockIdx.y - (ny - 1)) * (int)gridDim.x + (int)blockIdx.x) * 256 + (int)threadIdx.x;
-  int j, i;
-  if (e < nx + 1) {
-    j = 0, i = e;
-  } else if (e < 2 * (nx + 1)) {
-    j = ny, i = e - (nx + 1);
-  } else if (e < 2 * (nx + 1) + (ny - 1)) {
-    j = 1 + (e - 2 * (nx + 1)), i = 0;
-  } else if (e < 2 * (nx + 1) + 2 * (ny - 1)) {
-    j = 1 + (e - 2 * (nx + 1) - (ny - 1)), i = nx;
-  } else {
-    return;
+  const int i = 1 + (item % groups) * 64 + lane;
+  const int ic = i < nx ? i : nx - 1;  // lanes past the last column repeat it
+  const int j0 = 1 + (item / groups) * rows;
+  const int j1 = (j0 + rows - 1 < ny - 1) ? j0 + rows - 1 : ny - 1;
+  // cells (j, i) and (j, i-1) of a row: mass and pressure + pseudo
+  struct Cells {
+    double m0, m1, p0, p1;
+  };
+  auto loadCells = [&](int j) {
+    const int c = j * nx + ic;
+    Cells w;
+    w.m0 = at(f.M, c), w.m1 = at(f.M - 1, c);
+    w.p0 = (double)at(f.p[kp.cur], c) + (double)at(f.q[kp.cur], c);
+    w.p1 = (double)at(f.p[kp.cur] - 1, c) + (double)at(f.q[kp.cur] - 1, c);
+    return w;
+  };
+  Cells lo = loadCells(j0 - 1), hi = loadCells(j0);
+  const double dt1 = dtForNodes(kp, first);
+  const double dt = 0.5 * (dt1 + f.sc->dt[kp.cur]);
+  for (int j = j0; j <= j1; ++j) {
+    const int p = j * (nx + 1) + ic;
+    const double uxn = (double)at(f.ux[kp.cur], p), uyn = (double)at(f.uy[kp.cur], p);
+    const Cells next = (j < j1) ? loadCells(j + 1) : hi;
+    const double Mp = ((((0.0 + hi.m0) + hi.m1) + lo.m0) + lo.m1) / 4.0;
+    const D2 X0 = eulerNode(o, j, ic);
+    const D2 Cn[4] = {lpcNpcAxis(X0, eulerNode(o, j, ic + 1), eulerNode(o, j + 1, ic)),
+                      lpcNpcAxis(X0, eulerNode(o, j + 1, ic), eulerNode(o, j, ic - 1)),
+                      lpcNpcAxis(X0, eulerNode(o, j - 1, ic), eulerNode(o, j, ic + 1)),
+                      lpcNpcAxis(X0, eulerNode(o, j, ic - 1), eulerNode(o, j - 1, ic))};
+    D2 r = {0.0, 0.0};
+    r = d2add(r, d2mul(Cn[0], hi.p0));
+    r = d2add(r, d2mul(Cn[1], hi.p1));
+    r = d2add(r, d2mul(Cn[2], lo.p0));
+    r = d2add(r, d2mul(Cn[3], lo.p1));
+    const D2 u1 = d2add(D2{uxn, uyn}, d2mul(r, dt / Mp));
+    if (i < nx) {
+      at(f.Mp, p) = Mp;
+      at(kp.ul, p) = u1.x;
+      at(kp.vl, p) = u1.y;
+    }
+    lo = hi, hi = next;
   }
-  lagrangeNodeAt(kp, dt1, (long)j * (nx + 1) + i, j, i);
 }
+
+template <class R>
+__global__ __launch_bounds__(256) void k_lagrange_node_walk(KPT<R> kp) {
+  const int item = (int)(blockIdx.x * 4) + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  lagrangeNodeWalk(kp, item);
+}
+
+// waves of the kernel: bands of interior nodes, then 64 boundary nodes each
+int nodeWalkItems(long nx, long ny, int rows) {
+  const long nedge = 2 * (nx + 1) + 2 * (ny - 1);
+  return (int)((nx - 1 + 63) / 64 * ((ny - 1 + rows - 1) / rows) + (nedge + 63) / 64);
+}
+
+// Node rows per band, from the waves that one row each leaves: 4 rows where that
+// still leaves 512, else one.  us per step by rows: 256^2 (1020 waves) 1: 42.4, 4:
+// 42.6; 500x333 PenteBorne 1: 76.3, 4: 75.5; 1173x391 1: 161.5, 2: 157.8, 4: 158.7;
+// 1531x1021 1: 221, 4: 215, 8: 216; 2048^2 mixed 1: 450, 2: 432, 4: 435, 16: 436; 4096^2
+// 1: 1831, 4: 1764, 16: 1797; 64-problem mixed ensemble 1: 2957, 4: 2860, 8: 2853.
+int nodeWalkRows(long waves1) { return waves1 >= 2048 ? 4 : 1; }
 
 // Cell kernel: the cell part of the Lagrange phase (lagrangeCellCompute,
 // lagrange_cell.hpp) with the remap vector, the Lagrange volume and centroid
@@ -375,9 +411,11 @@ __global__ __launch_bounds__(256) void k_dt_reduce_batch(BatchLaunchT<R> bl) {
     __syncthreads();  // the shared scratch is reused by the next virtual block
   });
 }
-template <class R, bool ONE>
+template <class R>
 __global__ __launch_bounds__(256) void k_lagrange_node_batch(BatchLaunchT<R> bl) {
-  batchRun<ONE>(bl, [&](const KPT<R>& kp, unsigned b, unsigned, unsigned) { lagrangeNodeBody(kp, b); });
+  batchRun<true>(bl, [&](const KPT<R>& kp, unsigned local, unsigned, unsigned) {
+    lagrangeNodeWalk(kp, (int)(local * 4) + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)));
+  });
 }
 template <class R, int M, bool ONE>
 __global__ __launch_bounds__(256) void k_lagrange_cell_batch(BatchLaunchT<R> bl) {
@@ -386,7 +424,6 @@ __global__ __launch_bounds__(256) void k_lagrange_cell_batch(BatchLaunchT<R> bl)
 
 #define MHY_LAGRANGE_INST_ONE(R, ONE)                                        \
   template __global__ void k_dt_reduce_batch<R, ONE>(BatchLaunchT<R>);       \
-  template __global__ void k_lagrange_node_batch<R, ONE>(BatchLaunchT<R>);   \
   template __global__ void k_lagrange_cell_batch<R, 1, ONE>(BatchLaunchT<R>); \
   template __global__ void k_lagrange_cell_batch<R, 2, ONE>(BatchLaunchT<R>); \
   template __global__ void k_lagrange_cell_batch<R, 3, ONE>(BatchLaunchT<R>);
@@ -397,7 +434,8 @@ __global__ __launch_bounds__(256) void k_lagrange_cell_batch(BatchLaunchT<R> bl)
   template __global__ void k_dt_reset<R>(KPT<R>);                            \
   template __global__ void k_dt_hold<R>(KPT<R>);                             \
   template __global__ void k_lagrange_node<R>(KPT<R>);                       \
-  template __global__ void k_lagrange_node_euler<R>(KPT<R>);                 \
+  template __global__ void k_lagrange_node_walk<R>(KPT<R>);                  \
+  template __global__ void k_lagrange_node_batch<R>(BatchLaunchT<R>);        \
   template __global__ void k_lagrange_cell<R, 1>(KPT<R>);                    \
   template __global__ void k_lagrange_cell<R, 2>(KPT<R>);                    \
   template __global__ void k_lagrange_cell<R, 3>(KPT<R>);                    \
