@@ -148,6 +148,9 @@ struct mhy_ctx {
   bool useGraph = true;
   hipGraphExec_t graph[4] = {nullptr, nullptr, nullptr, nullptr};
   int status = MHY_OK;
+  // FP64 copy of one field on its way from or to the host (max(cells, nodes)
+  // values, allocated when first needed, freed with the context)
+  double* staging = nullptr;
   // this device's copy of the scratch array (mhy_conservation_noalloc)
   double* scratch = nullptr;
   long ncell = 0, nnode = 0, nface = 0;
@@ -777,6 +780,37 @@ int uploadR(mhy_ctx* x, double* dst, const std::vector<double>& src) {
   if (!x->mixed) return upload(x, dst, src);
   std::vector<float> h(src.begin(), src.end());
   HIPCHK(x, hipMemcpy(dst, h.data(), sizeof(float) * h.size(), hipMemcpyHostToDevice));
+  return MHY_OK;
+}
+
+// the staging array, or null when the device has no room for it
+double* stagingArray(mhy_ctx* x) {
+  if (!x->staging) {
+    void* p = nullptr;
+    if (hipMalloc(&p, sizeof(double) * (size_t)std::max(x->ncell, x->nnode)) != hipSuccess) {
+      (void)hipGetLastError();
+      return nullptr;
+    }
+    x->staging = static_cast<double*>(p);
+    x->allocs.push_back(p);
+  }
+  return x->staging;
+}
+
+// n values of a device array of type V to out as FP64: widened on the device,
+// or on the host when there is no staging array
+template <class V>
+int readWidened(mhy_ctx* x, const V* src, double* out, long n) {
+  if (double* st = stagingArray(x)) {
+    hipLaunchKernelGGL(k_widen<V>, gridFor(n), dim3(kBlock), 0, x->stream, src, st, n);
+    HIPCHK(x, hipGetLastError());
+    HIPCHK(x, hipMemcpyAsync(out, st, sizeof(double) * n, hipMemcpyDeviceToHost, x->stream));
+    HIPCHK(x, hipStreamSynchronize(x->stream));
+    return MHY_OK;
+  }
+  std::vector<V> h(n);
+  HIPCHK(x, hipMemcpy(h.data(), src, sizeof(V) * n, hipMemcpyDeviceToHost));
+  for (long i = 0; i < n; ++i) out[i] = h[i];
   return MHY_OK;
 }
 
@@ -1491,11 +1525,7 @@ int mhy_get_field(mhy_ctx* x, int field, double* out, long long n) {
   HIPCHK(x, hipStreamSynchronize(x->stream));
   if (field == MHY_CELL_MIXTE || field == MHY_CELL_PURE) {
     if (n != x->ncell) return fail(x, MHY_ERR_ARG, "size");
-    std::vector<int> v(x->ncell);
-    HIPCHK(x, hipMemcpy(v.data(), field == MHY_CELL_MIXTE ? x->f.mixte : x->f.pure, sizeof(int) * x->ncell,
-                        hipMemcpyDeviceToHost));
-    for (long c = 0; c < x->ncell; ++c) out[c] = v[c];
-    return MHY_OK;
+    return readWidened(x, field == MHY_CELL_MIXTE ? x->f.mixte : x->f.pure, out, x->ncell);
   }
   if (field == MHY_NODE_MASS) {
     if (x->euc) return fail(x, MHY_ERR_ARG, "the Eucclhyd scheme has no node mass");
@@ -1514,12 +1544,7 @@ int mhy_get_field(mhy_ctx* x, int field, double* out, long long n) {
   double* p = fieldPtr(x, field, len);
   if (!p) return fail(x, MHY_ERR_ARG, "unknown field " + std::to_string(field));
   if (n != len) return fail(x, MHY_ERR_ARG, "size");
-  if (x->mixed && isBulkField(field)) {
-    std::vector<float> h(len);
-    HIPCHK(x, hipMemcpy(h.data(), p, sizeof(float) * len, hipMemcpyDeviceToHost));
-    for (long i = 0; i < len; ++i) out[i] = h[i];
-    return MHY_OK;
-  }
+  if (x->mixed && isBulkField(field)) return readWidened(x, reinterpret_cast<const float*>(p), out, len);
   HIPCHK(x, hipMemcpy(out, p, sizeof(double) * len, hipMemcpyDeviceToHost));
   return MHY_OK;
 }
@@ -1541,6 +1566,13 @@ int mhy_set_field(mhy_ctx* x, int field, const double* in, long long n) {
   }
   HIPCHK(x, hipStreamSynchronize(x->stream));
   if (x->mixed && isBulkField(field)) {
+    if (double* stage = stagingArray(x)) {
+      HIPCHK(x, hipMemcpyAsync(stage, in, sizeof(double) * len, hipMemcpyHostToDevice, x->stream));
+      hipLaunchKernelGGL(k_narrow, gridFor(len), dim3(kBlock), 0, x->stream, stage, reinterpret_cast<float*>(p), len);
+      HIPCHK(x, hipGetLastError());
+      HIPCHK(x, hipStreamSynchronize(x->stream));
+      return MHY_OK;
+    }
     std::vector<float> h(in, in + len);
     HIPCHK(x, hipMemcpy(p, h.data(), sizeof(float) * len, hipMemcpyHostToDevice));
     return MHY_OK;
