@@ -205,6 +205,7 @@ struct KPT {
   int dtFold;    // the node update forms dt_{n+1} from the accumulators (whole steps);
                  // 0: it reads the dt a finalize kernel left (phase-level calls)
   R *ul, *vl;    // the step's Lagrange node velocity: uxl, uyl, or the n+1 buffers in place
+  int walkRows;  // rows per band of the column-walking y sweeps
   int nodeRows;  // node rows per band of the node update
   int dualRows;  // node rows per band of the nodal remap of both sweeps
   long ncell, nnode;

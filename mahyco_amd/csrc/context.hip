@@ -142,6 +142,7 @@ struct mhy_ctx {
   // material and limited slopes on meshes of at least 4096 walking waves,
   // where it measured faster.  MAHYCO_SWEEP_Y=walk / wave forces either.
   bool walkY = false;
+  int walkRows = 32;  // rows per band (MAHYCO_WALK_ROWS forces 4, 8, 16, 32 or 64)
   // mhy_run replays each step as a captured HIP graph, one per step parity
   // and sweep order (index 2 * cur + x_then_y_n); MAHYCO_GRAPH=0 launches
   // eagerly
@@ -274,6 +275,7 @@ KP makeKP(const mhy_ctx* x) {
   setLagrangeVelocity(kp);
   kp.dualRows = x->dualRows;
   kp.nodeRows = x->nodeRows;
+  kp.walkRows = x->walkRows;
   return kp;
 }
 
@@ -643,7 +645,7 @@ int phaseSweepStage(mhy_ctx* x, int sweep, int stage) {
       timed(x, kid, [&] { launchR(x, fd ? fd : runD, ff ? ff : runF, g, b, kp); });
     };
     if (walk) {
-      launchForm(walkKernel<double>(m, pp), walkKernel<float>(m, pp), sweepWalkGrid(x->o.nx, x->o.ny), dim3(kBlock));
+      launchForm(walkKernel<double>(m, pp), walkKernel<float>(m, pp), sweepWalkGrid(x->o.nx, x->o.ny, x->walkRows), dim3(kBlock));
     } else if (o3) {  // third order: LDS-tile kernel, no PenteBorne (checked at creation)
       static const KernelFn kd[2][3] = {
           {k_sweep_o3<double, 1, false>, k_sweep_o3<double, 2, false>, k_sweep_o3<double, 3, false>},
@@ -1108,7 +1110,7 @@ static int createContext(const mhy_config* cfg, mhy_ctx** out, bool batchMember)
     return bail(fail(x, MHY_ERR_ARG, "precision must be 0 (FP64) or 1 (mixed FP32 / FP64)"));
   x->mixed = (c.precision == 1);
   if (x->mixed) x->sweepWave = true;  // the per-cell stencil sweeps are FP64 only
-  x->walkY = x->mixed && c.nbmat == 1 && c.pp != 1 && (long)sweepWalkGrid(c.nx, c.ny).x * 4 >= 4096;
+  x->walkY = x->mixed && c.nbmat == 1 && c.pp != 1 && (long)sweepWalkGrid(c.nx, c.ny, 32).x * 4 >= 4096;
   x->dualWalkY = x->mixed && (long)dualWalkGrid(c.nx, c.ny).x * 4 >= 8192;
   // FP64: the LDS-tile kernel (4096^2 point explosion: 0.42 ms against 0.45 ms
   // for the wave strip)
@@ -1123,6 +1125,11 @@ static int createContext(const mhy_config* cfg, mhy_ctx** out, bool batchMember)
   if (const char* wy = std::getenv("MAHYCO_SWEEP_Y")) {
     if (std::string(wy) == "walk") x->walkY = true;
     if (std::string(wy) == "wave") x->walkY = false;
+  }
+  x->walkRows = sweepWalkRows(c.nx, c.ny);
+  if (const char* wr = std::getenv("MAHYCO_WALK_ROWS")) {
+    const int rows = std::atoi(wr);
+    if (rows == 4 || rows == 8 || rows == 16 || rows == 32 || rows == 64) x->walkRows = rows;
   }
   if (const char* g = std::getenv("MAHYCO_GRAPH")) x->useGraph = (std::string(g) != "0");
   // the fused first sweep needs the wave kernels for both sweep directions
@@ -1919,6 +1926,7 @@ struct mhy_batch {
   int dualLim = 0;        // the same with PenteBorne too: nodal remap of both sweeps in one kernel
   int dualRows = 32;      // node rows per band of that kernel
   int nodeRows = 1;       // node rows per band of the node update
+  int walkRows = 32;      // rows per band of the column-walking y sweeps
   void* dTable = nullptr;  // KPT<double> or KPT<float> entries
   unsigned* dStart = nullptr;  // BK_COUNT x (n+1)
   unsigned* dGx = nullptr;     // BK_COUNT x n
@@ -1975,7 +1983,11 @@ int batchEnqueueStepR(mhy_batch* b, int cur, bool xty, bool timing, bool reduce)
                                  k_lagrange_cell_batch<R, 3, false>};
   static const Fn cellOne[3] = {k_lagrange_cell_batch<R, 1, true>, k_lagrange_cell_batch<R, 2, true>,
                                 k_lagrange_cell_batch<R, 3, true>};
-  launch(BK_CELL, cellLoop[b->m - 1], cellOne[b->m - 1], cur);
+  // (fixed options, x first: the Lagrange update runs inside the first sweep, 64
+  // mixed problems 2855 -> 2605 us per step; y first the strips recompute a third
+  // of it as halo)
+  const bool lagX = b->fixLim && xty;
+  if (!lagX) launch(BK_CELL, cellLoop[b->m - 1], cellOne[b->m - 1], cur);
   for (int sweep = 1; sweep <= 2; ++sweep) {
     const bool xd = (sweep == 1) ? xty : !xty;
     const int fuse = (sweep == 2) ? 1 : 0;
@@ -1984,7 +1996,8 @@ int batchEnqueueStepR(mhy_batch* b, int cur, bool xty, bool timing, bool reduce)
       launch(xd ? BK_SWX : BK_SWY, o3BatchKernel<R, false>(xd, b->m), o3BatchKernel<R, true>(xd, b->m), v + 8 * fuse);
     else if (b->fixLim && !(!xd && b->walkY))
       launch(xd ? BK_SWX : BK_SWY, nullptr,
-             xd ? sweepFixedXBatch<R>(b->fixLim, b->m, sweep) : sweepFixedYBatch<R>(b->fixLim, b->m, sweep),
+             xd ? sweepFixedXBatch<R>(b->fixLim, b->m, (lagX && sweep == 1) ? 0 : sweep)
+                : sweepFixedYBatch<R>(b->fixLim, b->m, sweep),
              v + 8 * fuse, sweepWaveBlock(xd, b->mixed, b->pp));
     else if (!xd && b->walkY)
       launch(BK_SWY, walkBatchKernel<R, false>(b->m, b->pp), walkBatchKernel<R, true>(b->m, b->pp), v + 8 * fuse);
@@ -2106,6 +2119,7 @@ int mhy_batch_create(const mhy_config* cfgs, int n, mhy_batch** out) {
       setLagrangeVelocity(kp);
       kp.dualRows = b->dualRows;
       kp.nodeRows = b->nodeRows;
+      kp.walkRows = b->walkRows;
       table[(size_t)v * n + i] = kp;
     }
   // virtual-block layout of every kernel
@@ -2125,7 +2139,7 @@ int mhy_batch_create(const mhy_config* cfgs, int n, mhy_batch** out) {
         case BK_SWX: g = b->o3 ? sweepO3Grid(true, nx, ny) : sweepWaveGrid(true, nx, ny, b->mixed, b->pp); break;
         case BK_SWY:
           g = b->o3      ? sweepO3Grid(false, nx, ny)
-              : b->walkY ? sweepWalkGrid(nx, ny)
+              : b->walkY ? sweepWalkGrid(nx, ny, b->walkRows)
                          : sweepWaveGrid(false, nx, ny, b->mixed, b->pp);
           break;
         case BK_DUX: g = dualWaveGrid(true, nx, ny, b->mixed); break;

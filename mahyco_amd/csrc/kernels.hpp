@@ -95,7 +95,8 @@ template <class R, int M, bool PP, class P>
 __global__ void k_sweep_walk(KPT<R> kp);
 template <class R, int M, bool PP, bool ONE>
 __global__ void k_sweep_walk_batch(BatchLaunchT<R> bl);
-dim3 sweepWalkGrid(long nx, long ny);
+dim3 sweepWalkGrid(long nx, long ny, int rows);
+int sweepWalkRows(long nx, long ny);
 template <class R, bool XD>
 __global__ void k_dual(KPT<R> kp);
 template <class R, bool XD>

@@ -15,6 +15,7 @@ SweepFn<R> pick(int kind) {
 }
 template <class R, int M, int LIM>
 SweepBatchFn<R> pickBatch(int kind) {
+  if (kind == 0) return k_sweep_wave_lag_batch<R, M, true, FixOpts<LIM, 1>>;
   if (kind == 1) return k_sweep_wave_batch<R, M, false, true, true, FixOpts<LIM, 1>>;
   return k_sweep_wave_batch<R, M, false, true, true, FixOpts<LIM, 2>>;
 }

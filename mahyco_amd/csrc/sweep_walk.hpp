@@ -2,8 +2,8 @@
 // computeGradPhi, computeUpwindFaceQuantitiesForProjection, computeUremap of
 // the y direction; remap/PhaseRemap1.cc, remap/PhaseRemap2.cc).
 //
-// A wave covers 64 consecutive columns and walks down a band of kWalkRows
-// rows, plus two halo rows above and below.  Every row access of the wave
+// A wave covers 64 consecutive columns and walks down a band of
+// kp.walkRows rows, plus two halo rows above and below.  Every row access of the wave
 // is a whole 64-cell row segment.  Each iteration loads one new row and
 // keeps the two before it in registers: the divided difference at the new
 // row's minus face, the slope (or the PenteBorne fluxes) of the row before,
@@ -24,8 +24,6 @@ namespace mhy {
 using namespace sw;
 
 namespace {
-
-constexpr int kWalkRows = 32;  // rows updated per band
 
 // end-of-Lagrange node position (updatePosition, PhaseLagrange.cc:203-208)
 template <class R>
@@ -61,7 +59,8 @@ __device__ __forceinline__ void sweepWalkYBody(const KPT<R>& kp, unsigned b) {
   const long ngx = (nx + 63) / 64;
   const long g = (long)b * 4 + wave;
   const long i0 = (g % ngx) * 64 + lane;
-  const long a0 = (g / ngx) * kWalkRows;
+  const int rows = kp.walkRows;
+  const long a0 = (g / ngx) * rows;
 
   double* const* Uin = (P::sweep(kp) == 1) ? f.UL : f.U1;
   const double dtn = f.sc->dt[kp.cur], dt1 = f.sc->dt[kp.nxt];
@@ -81,7 +80,7 @@ __device__ __forceinline__ void sweepWalkYBody(const KPT<R>& kp, unsigned b) {
   T HA = T(0.0), HB = T(0.0);
   int flA = 0, flB = 0;
 
-  for (int k = 0; k < kWalkRows + 4; ++k) {
+  for (int k = 0; k < rows + 4; ++k) {
     // the column and what derives from it (addresses, Euler coordinates) are
     // formed again for every row from an opaque copy of the index: hoisted
     // out of the loop they would hold registers through every row
@@ -176,7 +175,7 @@ __device__ __forceinline__ void sweepWalkYBody(const KPT<R>& kp, unsigned b) {
     }
 
     // update of row A: minus face faceA, plus face faceB
-    if (inT && rA >= a0 && rA < a0 + kWalkRows && rA < ny) {
+    if (inT && rA >= a0 && rA < a0 + rows && rA < ny) {
       const long c = rA * nx + i;
       const bool hasM = (rA >= 1), hasP = (rA + 1 < ny);
       // Euler length of a face (Init.cc:528-533): the norm of an edge along one

@@ -452,6 +452,15 @@ __attribute__((amdgpu_waves_per_eu(kMinWavesLag<R, M, XD, P>))) void k_sweep_wav
   sweepWaveBody<R, M, false, XD, true, P>(kp, XD ? blockIdx.x : xcdBlock());
 }
 
+// all problems of an ensemble in one launch, one workgroup per virtual block:
+// the first sweep with the Lagrange update
+template <class R, int M, bool XD, class P>
+__global__ __launch_bounds__((XD ? 256 : 64 * kYWaves<R, false>))
+__attribute__((amdgpu_waves_per_eu(kMinWavesLag<R, M, XD, P>))) void k_sweep_wave_lag_batch(BatchLaunchT<R> bl) {
+  batchRun<true>(bl, [&](const KPT<R>& kp, unsigned local, unsigned, unsigned) {
+    sweepWaveBody<R, M, false, XD, true, P>(kp, local);
+  });
+}
 // all problems of an ensemble in one launch (BatchLaunchT, common.hpp)
 template <class R, int M, bool PP, bool XD, bool ONE, class P>
 __global__ __launch_bounds__((XD ? 256 : 64 * kYWaves<R, PP>))
