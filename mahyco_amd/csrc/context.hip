@@ -1675,6 +1675,9 @@ int mhy_kernel_bytes(const mhy_ctx* x, int k, double* bytes) {
   const int m = x->o.nbmat, nc = x->o.nc;
   const bool pp = x->o.pp == 1;
   const int meth = x->o.methode;
+  // bulk material fields the Lagrange update reads: mu, rho_k, e_k, p_k, and
+  // q_k for the centred pseudo
+  const int bulkIn = (x->o.pseudo_centree == 1 ? 5 : 4) * m;
   const double r = x->mixed ? 4.0 : 8.0, d = 8.0, i4 = 4.0;
   // cell part of the final remap: U2 in registers or read; writes rho, e, q,
   // p, c, mu_k, rho_k, e_k, p_k, c_k (bulk) and M, f_k, M_k, flags
@@ -1714,7 +1717,7 @@ int mhy_kernel_bytes(const mhy_ctx* x, int k, double* bytes) {
     case K_CELL:
       // u_n+1 ; f, M_k, vol (FP64), mu, rho_k, e_k, p_k, q_k + rho, divu, c ;
       // writes UL, VL, XcL, YcL (+ rL, qL) (FP64), divu, q_k
-      w = N * 2 * r + C * ((2 * m + 1) * d + (5 * m + 3) * r) + C * d * (nc + 3 + (meth == 1) + pp) + C * r * (1 + m);
+      w = N * 2 * r + C * ((2 * m + 1) * d + (bulkIn + 3) * r) + C * d * (nc + 3 + (meth == 1) + pp) + C * r * (1 + m);
       break;
     case K_SWEEP_X:
     case K_SWEEP_Y: {
@@ -1740,7 +1743,7 @@ int mhy_kernel_bytes(const mhy_ctx* x, int k, double* bytes) {
       // the Lagrange cell update's inputs (u_n+1 ; f, M_k, vol (FP64), mu,
       // rho_k, e_k, p_k, q_k + rho, divu, c) and outputs that outlive the
       // step (divu, q_k ; rL, qL), then sweep 1's outputs: U_1, face fluxes
-      const double lagIn = N * 2 * r + C * ((2 * m + 1) * d + (5 * m + 3) * r);
+      const double lagIn = N * 2 * r + C * ((2 * m + 1) * d + (bulkIn + 3) * r);
       const double lagOut = C * r * (1 + m) + C * d * ((meth == 1) + pp);
       const double fl = (meth == 2 ? C * m : F * m) * d;
       w = lagIn + lagOut + C * nc * d + fl;

@@ -114,17 +114,21 @@ __device__ __forceinline__ bool lagrangeCellCompute(const KPT<R>& kp, long c, lo
   // mass, density, energy and pressure those of the cell, unless the final
   // remap stored them (envx)
   const bool derived = (m == 1) && o.compact1 && !at(f.envx, c);
+  // (the step-start material pseudo enters the centred form of the energy
+  // update only; read always, and with both centroid coordinates stored where the
+  // second sweep reads one, a 4096^2 step took 8 % longer)
+  const bool centred = o.pseudo_centree == 1;
+#pragma unroll
+  for (int k = 0; k < m; ++k) qk0[k] = centred ? (double)at(f.q_k[cur][k], c) : 0.0;
   if (derived) {
     fk[0] = 1.0, mu0[0] = 1.0, Mk0[0] = Mc0, rk0[0] = rhoS;
     ek0[0] = (double)at(f.e[cur], c), pk0[0] = (double)at(f.p[cur], c);
-    qk0[0] = (double)at(f.q_k[cur][0], c);
   } else {
 #pragma unroll
     for (int k = 0; k < m; ++k) {
       fk[k] = at(f.f_k[k], c);
       Mk0[k] = at(f.M_k[k], c);
       rk0[k] = (double)at(f.rho_k[cur][k], c);
-      qk0[k] = (double)at(f.q_k[cur][k], c);
       ek0[k] = (double)at(f.e_k[cur][k], c);
       pk0[k] = (double)at(f.p_k[cur][k], c);
       mu0[k] = (double)at(f.mu_k[k], c);
@@ -180,7 +184,7 @@ __device__ __forceinline__ bool lagrangeCellCompute(const KPT<R>& kp, long c, lo
       if ((r1 > o.threshold) && (r0 > o.threshold)) {
         const double qn = qk0[k];
         double pseudo = 0.0;
-        if ((o.pseudo_centree == 1) && ((qk1[k] + qn) * (1.0 / r1 - 1.0 / r0) > 0.)) pseudo = 0.5 * (qk1[k] + qn);
+        if (centred && ((qk1[k] + qn) * (1.0 / r1 - 1.0 / r0) > 0.)) pseudo = 0.5 * (qk1[k] + qn);
         if (o.pseudo_centree == 0) pseudo = qk1[k];
         const double den = 1 + 0.5 * (o.gammap[k] - 1.0) * r1 * (1.0 / r1 - 1.0 / r0);
         const double num = ek0[k] - (0.5 * pk0[k] + pseudo) * (1.0 / r1 - 1.0 / r0);

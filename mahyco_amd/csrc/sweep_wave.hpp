@@ -240,7 +240,12 @@ __device__ __forceinline__ void sweepWaveBody(const KPT<R>& kp, unsigned b) {
       x = XD ? lc.xc.x : lc.xc.y;
       if (output && P::methode(o) == 1) at(f.rL, cb) = lc.rho;  // A2 dual fluxes
       if (output && PP) at(f.qL, cb) = lc.q;                // PenteBorne Phi of the second sweep
-      if (output && P::geomLoad(kp)) at(f.VL, cb) = lc.V, at(f.XcL, cb) = lc.xc.x, at(f.YcL, cb) = lc.xc.y;
+      // what the second sweep reads: the volume, and the centroid along its axis
+      if (output && P::geomLoad(kp)) {
+        at(f.VL, cb) = lc.V;
+        if (XD) at(f.YcL, cb) = lc.xc.y;
+        else at(f.XcL, cb) = lc.xc.x;
+      }
     } else {
       // (the VNR PenteBorne Phi takes the pseudo from q_L, not from U)
       const int nload = (PP && !kEuc<L>) ? 3 * M : NC;
