@@ -174,7 +174,7 @@ struct FieldsT {
   double *f_k[NMAT];
   R *mu_k[NMAT];
   double *M, *M_k[NMAT];
-  int *mixte, *pure;
+  unsigned char* flags;  // mixed / pure-material flags of a cell (packCellFlags)
   R *Mp, *outvx, *outvy;
   R *rho0, *e0, *rho_k0[NMAT], *e_k0[NMAT];  // t=0 fields (periodic cells)
   // per-step intermediates
@@ -244,6 +244,12 @@ template <class V>
 __device__ __forceinline__ const V& at(const V* base, long idx) {
   return *reinterpret_cast<const V*>(reinterpret_cast<const char*>(base) + (unsigned)idx * (unsigned)sizeof(V));
 }
+
+// A cell's mixed flag and its pure material (-1 to 2) in one byte.
+constexpr unsigned kMixedBit = 0x80;
+MHY_HD unsigned char packCellFlags(int mixte, int pure) { return (unsigned char)((mixte ? kMixedBit : 0) | (pure + 1)); }
+MHY_HD int cellMixed(unsigned char b) { return (b & kMixedBit) ? 1 : 0; }
+MHY_HD int cellPure(unsigned char b) { return (int)(b & 0x7f) - 1; }
 
 // bitwise equality (distinguishes signed zeros, never true for a NaN pattern
 // compared with another)

@@ -240,15 +240,22 @@ double* allocR(mhy_ctx* x, long n, hipError_t& e) {
   return static_cast<double*>(p);
 }
 
-int* allocI(mhy_ctx* x, long n, hipError_t& e) {
+unsigned char* allocB(mhy_ctx* x, long n, hipError_t& e) {
   if (e != hipSuccess) return nullptr;
   void* p = nullptr;
-  e = hipMalloc(&p, sizeof(int) * (size_t)std::max(n, 1L));
+  e = hipMalloc(&p, (size_t)std::max(n, 1L));
   if (e == hipSuccess) {
     x->allocs.push_back(p);
-    e = hipMemset(p, 0, sizeof(int) * (size_t)std::max(n, 1L));
+    e = hipMemset(p, 0, (size_t)std::max(n, 1L));
   }
-  return static_cast<int*>(p);
+  return static_cast<unsigned char*>(p);
+}
+
+// the initial mixed / pure flags
+hipError_t uploadFlags(unsigned char* dst, const HostInit& h, long n) {
+  std::vector<unsigned char> b(n);
+  for (long c = 0; c < n; ++c) b[c] = packCellFlags(h.mixte[c], h.pure[c]);
+  return hipMemcpy(dst, b.data(), (size_t)n, hipMemcpyHostToDevice);
 }
 
 // the Lagrange node velocity of the step with kp's parity
@@ -799,19 +806,18 @@ double* stagingArray(mhy_ctx* x) {
   return x->staging;
 }
 
-// n values of a device array of type V to out as FP64: widened on the device,
-// or on the host when there is no staging array
-template <class V>
-int readWidened(mhy_ctx* x, const V* src, double* out, long n) {
+// n FP32 values of a device array to out as FP64: widened on the device, or on
+// the host when there is no staging array
+int readWidened(mhy_ctx* x, const float* src, double* out, long n) {
   if (double* st = stagingArray(x)) {
-    hipLaunchKernelGGL(k_widen<V>, gridFor(n), dim3(kBlock), 0, x->stream, src, st, n);
+    hipLaunchKernelGGL(k_widen, gridFor(n), dim3(kBlock), 0, x->stream, src, st, n);
     HIPCHK(x, hipGetLastError());
     HIPCHK(x, hipMemcpyAsync(out, st, sizeof(double) * n, hipMemcpyDeviceToHost, x->stream));
     HIPCHK(x, hipStreamSynchronize(x->stream));
     return MHY_OK;
   }
-  std::vector<V> h(n);
-  HIPCHK(x, hipMemcpy(h.data(), src, sizeof(V) * n, hipMemcpyDeviceToHost));
+  std::vector<float> h(n);
+  HIPCHK(x, hipMemcpy(h.data(), src, sizeof(float) * n, hipMemcpyDeviceToHost));
   for (long i = 0; i < n; ++i) out[i] = h[i];
   return MHY_OK;
 }
@@ -1008,8 +1014,7 @@ static int setupEucclhyd(mhy_ctx* x, const mhy_config& c, bool batchMember) {
     AD(ef.fsx[k], C), AD(ef.fsy[k], C), AD(ef.pmin[k], N), AD(ef.pmax[k], N);
   }
   AD(f.M, C);
-  f.mixte = allocI(x, C, e);
-  f.pure = allocI(x, C, e);
+  f.flags = allocB(x, C, e);
   for (int q = 0; q < 4; ++q) AD(ef.gv[q], C);
   for (int d = 0; d < 2; ++d) AD(ef.vmin[d], N), AD(ef.vmax[d], N);
   AD(ef.perim, C), AD(ef.outvx, C), AD(ef.outvy, C);
@@ -1053,8 +1058,7 @@ static int setupEucclhyd(mhy_ctx* x, const mhy_config& c, bool batchMember) {
     up(f.X[0], X), up(f.Y[0], Y);
   }
   if (ok != MHY_OK) return ok;
-  if (hipMemcpy(f.mixte, h.mixte.data(), sizeof(int) * C, hipMemcpyHostToDevice) != hipSuccess ||
-      hipMemcpy(f.pure, h.pure.data(), sizeof(int) * C, hipMemcpyHostToDevice) != hipSuccess)
+  if (uploadFlags(f.flags, h, C) != hipSuccess)
     return fail(x, MHY_ERR_DEVICE, "upload flags");
   Scalars s0;
   std::memset(&s0, 0, sizeof(s0));
@@ -1258,8 +1262,7 @@ static int createContext(const mhy_config* cfg, mhy_ctx** out, bool batchMember)
   }
   for (int k = 0; k < m; ++k) AD(f.f_k[k], C), AR(f.mu_k[k], C), AD(f.M_k[k], C);
   AD(f.M, C);
-  f.mixte = allocI(x, C, e);
-  f.pure = allocI(x, C, e);
+  f.flags = allocB(x, C, e);
   if (o.compact1 && e == hipSuccess) {
     void* p = nullptr;
     if ((e = hipMalloc(&p, C)) == hipSuccess) x->allocs.push_back(p);
@@ -1335,8 +1338,7 @@ static int createContext(const mhy_config* cfg, mhy_ctx** out, bool batchMember)
     for (int k = 0; k < m; ++k) upR(f.rho_k0[k], h.rho_k[k]), upR(f.e_k0[k], h.e_k[k]);
   }
   if (u != MHY_OK) return bail(u);
-  if (hipMemcpy(f.mixte, h.mixte.data(), sizeof(int) * C, hipMemcpyHostToDevice) != hipSuccess ||
-      hipMemcpy(f.pure, h.pure.data(), sizeof(int) * C, hipMemcpyHostToDevice) != hipSuccess)
+  if (uploadFlags(f.flags, h, C) != hipSuccess)
     return bail(fail(x, MHY_ERR_DEVICE, "upload flags"));
   // the initial material fields are stored: every cell reads them
   if (o.compact1 && hipMemset(f.envx, 1, C) != hipSuccess) return bail(fail(x, MHY_ERR_DEVICE, "material flags"));
@@ -1532,7 +1534,10 @@ int mhy_get_field(mhy_ctx* x, int field, double* out, long long n) {
   HIPCHK(x, hipStreamSynchronize(x->stream));
   if (field == MHY_CELL_MIXTE || field == MHY_CELL_PURE) {
     if (n != x->ncell) return fail(x, MHY_ERR_ARG, "size");
-    return readWidened(x, field == MHY_CELL_MIXTE ? x->f.mixte : x->f.pure, out, x->ncell);
+    std::vector<unsigned char> b(x->ncell);
+    HIPCHK(x, hipMemcpy(b.data(), x->f.flags, (size_t)x->ncell, hipMemcpyDeviceToHost));
+    for (long c = 0; c < x->ncell; ++c) out[c] = (field == MHY_CELL_MIXTE) ? cellMixed(b[c]) : cellPure(b[c]);
+    return MHY_OK;
   }
   if (field == MHY_NODE_MASS) {
     if (x->euc) return fail(x, MHY_ERR_ARG, "the Eucclhyd scheme has no node mass");
@@ -1668,7 +1673,7 @@ const char* mhy_kernel_name(const mhy_ctx*, int k) { return (k >= 0 && k < K_COU
 // Algorithmic bytes of one launch: every input word the kernel must read
 // from HBM once and every output word it must write once (neighbour reuse
 // through the caches counted once).  Bulk fields count 4 bytes in the mixed
-// form, everything else 8 (flags 4).
+// form, everything else 8 (the flags one byte).
 int mhy_kernel_bytes(const mhy_ctx* x, int k, double* bytes) {
   if (!x || !bytes || k < 0 || k >= K_COUNT) return MHY_ERR_ARG;
   const double C = (double)x->ncell, N = (double)x->nnode, F = (double)x->nface;
@@ -1678,10 +1683,10 @@ int mhy_kernel_bytes(const mhy_ctx* x, int k, double* bytes) {
   // bulk material fields the Lagrange update reads: mu, rho_k, e_k, p_k, and
   // q_k for the centred pseudo
   const int bulkIn = (x->o.pseudo_centree == 1 ? 5 : 4) * m;
-  const double r = x->mixed ? 4.0 : 8.0, d = 8.0, i4 = 4.0;
+  const double r = x->mixed ? 4.0 : 8.0, d = 8.0, i1 = 1.0;
   // cell part of the final remap: U2 in registers or read; writes rho, e, q,
   // p, c, mu_k, rho_k, e_k, p_k, c_k (bulk) and M, f_k, M_k, flags
-  const double finalWrites = C * r * (5 + 5 * m) + C * d * (1 + 2 * m) + C * i4 * 2;
+  const double finalWrites = C * r * (5 + 5 * m) + C * d * (1 + 2 * m) + C * i1;
   double w = 0;
   if (x->euc) {  // Eucclhyd kernels (FP64)
     const bool o2 = x->o.space_order == 2, lag = x->o.mode == MODE_LAGRANGE;
@@ -1701,10 +1706,10 @@ int mhy_kernel_bytes(const mhy_ctx* x, int k, double* bytes) {
         break;
       case K_SWEEP_X:
       case K_SWEEP_Y:  // U_in, V_L and centroid, node velocities (+ flags) ; U_out
-        w = C * d * nc + C * d * 2 + N * 2 * d + C * i4 * 2 * (pp && x->o.pp_mixte) + C * d * nc;
+        w = C * d * nc + C * d * 2 + N * 2 * d + C * i1 * (pp && x->o.pp_mixte) + C * d * nc;
         break;
       case K_FINAL:  // U_2, volume ; rho, e, velocity, f_k, mu_k, rho_k, e_k, outputs, flags
-        w = C * d * (nc + 1) + C * d * (2 + 2 + 4 * m + 2) + C * i4 * 2;
+        w = C * d * (nc + 1) + C * d * (2 + 2 + 4 * m + 2) + C * i1;
         break;
       default: w = 0.0; break;
     }
@@ -1725,7 +1730,7 @@ int mhy_kernel_bytes(const mhy_ctx* x, int k, double* bytes) {
       // form V_L and the centroid from the node positions; the other kernels
       // read them) ; writes U_out, face fluxes (or PB)
       const double geo = x->sweepWave && x->o.order != 3 ? 0.0 : C * d * 2;
-      const double in = C * d * nc + geo + C * d * pp + C * i4 * 2 * (pp && x->o.pp_mixte) + N * 2 * r;
+      const double in = C * d * nc + geo + C * d * pp + C * i1 * (pp && x->o.pp_mixte) + N * 2 * r;
       const double fl = (meth == 2 ? C * m : F * m) * d;
       const double s1 = in + C * nc * d + fl;
       // sweep 2 with the final remap fused: no U2 store, the final outputs

@@ -577,8 +577,7 @@ __global__ __launch_bounds__(256) void k_euc_final(KP kp, EucFields e) {
 #pragma unroll
   for (int k = 0; k < M; ++k)
     if (fr[k] > 0.) matcell++, imatpure = k;
-  at(f.mixte, c) = (matcell > 1) ? 1 : 0;
-  at(f.pure, c) = (matcell > 1) ? -1 : imatpure;
+  at(f.flags, c) = packCellFlags(matcell > 1, (matcell > 1) ? -1 : imatpure);
   double mf[M], fm = 0.;
 #pragma unroll
   for (int k = 0; k < M; ++k) mf[k] = U[M + k] / masset;

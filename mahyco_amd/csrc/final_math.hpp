@@ -15,7 +15,7 @@ __device__ __forceinline__ void raiseErr(Scalars* sc, int code) { atomicCAS(&sc-
 template <class R, int M>
 struct FinalOut {
   R rho, e, q, p, c;
-  int mixte, pure;
+  int flags;  // packCellFlags
   double Mc;
   double fr[M], Mk[M];
   R mu[M], rk[M], ek[M], pk[M], ck[M];
@@ -61,8 +61,6 @@ __device__ __forceinline__ void finalCompute(const KPT<R>& kp, long c, const dou
 #pragma unroll
   for (int k = 0; k < M; ++k)
     if (fr[k] > 0.) matcell++, imatpure = k;
-  const int mixte = (matcell > 1) ? 1 : 0;
-  const int pure = (matcell > 1) ? -1 : imatpure;
 #pragma unroll
   for (int k = 0; k < M; ++k) mu[k] = U[M + k] / masset;
   double fm = 0.;
@@ -145,8 +143,7 @@ __device__ __forceinline__ void finalCompute(const KPT<R>& kp, long c, const dou
   out.p = (R)p1;
   out.c = (R)c1;
   out.Mc = Mc;
-  out.mixte = mixte;
-  out.pure = pure;
+  out.flags = packCellFlags(matcell > 1, (matcell > 1) ? -1 : imatpure);
 #pragma unroll
   for (int k = 0; k < M; ++k) {
     out.fr[k] = fr[k];
@@ -169,8 +166,7 @@ __device__ __forceinline__ void finalStore(const KPT<R>& kp, long c, const Final
   at(f.p[nxt], c) = out.p;
   at(f.c[nxt], c) = out.c;
   at(f.M, c) = out.Mc;
-  at(f.mixte, c) = out.mixte;
-  at(f.pure, c) = out.pure;
+  at(f.flags, c) = (unsigned char)out.flags;
   if constexpr (M == 1) {
     if (kp.o.compact1) {
       // the material fields equal 1, 1 and the mean fields bit for bit in

@@ -130,8 +130,7 @@ template <class R>
 __global__ void k_conservation(KPT<R> kp, double* out);
 template <class R>
 __global__ void k_env_expand(KPT<R> kp);
-template <class V>
-__global__ void k_widen(const V* in, double* out, long n);
+__global__ void k_widen(const float* in, double* out, long n);
 __global__ void k_narrow(const double* in, float* out, long n);
 
 }  // namespace mhy

@@ -800,12 +800,11 @@ __global__ __launch_bounds__(256) void k_conservation(KPT<R> kp, double* out) {
   }
 }
 
-// Field access: FP32 (or int) device arrays to FP64 and back, so that the host
+// Field access: FP32 device arrays to FP64 and back, so that the host
 // copies FP64 values only.  Bound by memory (12 bytes per value); converted on
 // the host by one thread, the four fields of a 2048^2 mixed state took 9.0 ms, so
 // about 2 ms (50 steps and the four fields 31.5 -> 24.1 ms).
-template <class V>
-__global__ __launch_bounds__(256) void k_widen(const V* in, double* out, long n) {
+__global__ __launch_bounds__(256) void k_widen(const float* in, double* out, long n) {
   const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) out[i] = (double)in[i];
 }
@@ -813,8 +812,6 @@ __global__ __launch_bounds__(256) void k_narrow(const double* in, float* out, lo
   const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) out[i] = (float)in[i];
 }
-template __global__ void k_widen<float>(const float*, double*, long);
-template __global__ void k_widen<int>(const int*, double*, long);
 
 #define MHY_REMAP_INST(R)                                              \
   template __global__ void k_dual<R, true>(KPT<R>);                    \

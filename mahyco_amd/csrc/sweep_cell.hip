@@ -197,7 +197,7 @@ __global__ __launch_bounds__(256) void k_sweep_cell(KP kp) {
     s[d].xc = XD ? f.XcL[cd] : f.YcL[cd];
     s[d].H = needH ? widthCell<XD>(kp, dt1, XD ? j : b, XD ? b : i) : 0.0;
     s[d].fl = 0;
-    if (mixteOpt) s[d].fl = (kp.sweep == 1) ? packFlags(f.mixte[cd], f.pure[cd]) : packedFlags<M, double>(s[d].phi);
+    if (mixteOpt) s[d].fl = (kp.sweep == 1) ? packFlags(cellMixed(f.flags[cd]), cellPure(f.flags[cd])) : packedFlags<M, double>(s[d].phi);
   }
   // a missing neighbour takes the values of the cell it neighbours
   // (PhaseRemap1.cc:157-158)

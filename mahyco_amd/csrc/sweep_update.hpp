@@ -180,7 +180,7 @@ __device__ __forceinline__ void visitCellOut(CellOut<R, L>& out, bool withG, boo
   constexpr int M = kMat<L>;
   if constexpr (FUSE) {
     FinalOut<R, M>& fo = out.fin;
-    fn(fo.rho), fn(fo.e), fn(fo.q), fn(fo.p), fn(fo.c), fn(fo.mixte), fn(fo.pure), fn(fo.Mc);
+    fn(fo.rho), fn(fo.e), fn(fo.q), fn(fo.p), fn(fo.c), fn(fo.flags), fn(fo.Mc);
 #pragma unroll
     for (int k = 0; k < M; ++k) fn(fo.fr[k]), fn(fo.Mk[k]), fn(fo.mu[k]), fn(fo.rk[k]), fn(fo.ek[k]), fn(fo.pk[k]), fn(fo.ck[k]);
   } else {
@@ -201,7 +201,7 @@ __device__ __forceinline__ void visitCellOut(CellOut<R, L>& out, bool withG, boo
 template <class R, int M>
 constexpr int kFuse8 = 1 + 2 * M + (sizeof(R) == 8 ? 5 + 5 * M : 0);
 template <class R, int M>
-constexpr int kFuse4 = 2 + (sizeof(R) == 4 ? 5 + 5 * M : 0);
+constexpr int kFuse4 = 1 + (sizeof(R) == 4 ? 5 + 5 * M : 0);
 // LDS bytes per staged cell: the larger of the two layouts (final fields or
 // remap vector), each followed by G and DF
 template <class R, int L, bool PP>

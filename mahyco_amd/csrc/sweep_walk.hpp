@@ -99,7 +99,7 @@ __device__ __forceinline__ void sweepWalkYBody(const KPT<R>& kp, unsigned b) {
       x = at(f.YcL, cb);
       h = needH ? T(widthY(kp, dt1, r, i)) : T(0.0);
       flg = 0;
-      if (mixteOpt) flg = (P::sweep(kp) == 1) ? packFlags(at(f.mixte, cb), at(f.pure, cb)) : packedFlags<M, T>(ph);
+      if (mixteOpt) flg = (P::sweep(kp) == 1) ? packFlags(cellMixed(at(f.flags, cb)), cellPure(at(f.flags, cb))) : packedFlags<M, T>(ph);
     };
     // normal velocity of face r, between rows r-1 and r (PrepareRemap.cc:50-62)
     auto fnv = [&](long r) {

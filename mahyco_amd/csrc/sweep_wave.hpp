@@ -267,7 +267,7 @@ __device__ __forceinline__ void sweepWaveBody(const KPT<R>& kp, unsigned b) {
     cellPhi<L, PP, T>(u, PP ? 1.0 : V, qv, ph);
     h = needH ? T(widthW<XD>(kp, dt1, jb, ib)) : T(0.0);
     flg = 0;
-    if (mixteOpt) flg = (P::sweep(kp) == 1) ? packFlags(at(f.mixte, cb), at(f.pure, cb)) : packedFlags<L, T>(ph);
+    if (mixteOpt) flg = (P::sweep(kp) == 1) ? packFlags(cellMixed(at(f.flags, cb)), cellPure(at(f.flags, cb))) : packedFlags<L, T>(ph);
   };
   T phi[NC], H = T(0.0);
   double xc = 0.0;

@@ -1,5 +1,5 @@
-"""Field access of the mixed form and of the integer flags, which the device
-widens to FP64 and narrows: every value is exactly the FP32 rounding of what
+"""Field access of the mixed form, whose values the device widens to FP64 and
+narrows, and of the mixed / pure flags, kept in one byte: every value is exactly the FP32 rounding of what
 was written, the flags equal the oracle's.  Lengths around a block of 256."""
 import numpy as np
 import pytest
