@@ -578,10 +578,10 @@ SweepFn<R> sweepWaveKernel(bool xd, int m, bool pp) {
 template <class R>
 SweepFn<R> lagSweepKernel(bool xd, int m) {
   static const SweepFn<R> kl[2][3] = {
-      {k_sweep_wave_lag<R, 1, false, RunOpts>, k_sweep_wave_lag<R, 2, false, RunOpts>,
-       k_sweep_wave_lag<R, 3, false, RunOpts>},
-      {k_sweep_wave_lag<R, 1, true, RunOpts>, k_sweep_wave_lag<R, 2, true, RunOpts>,
-       k_sweep_wave_lag<R, 3, true, RunOpts>}};
+      {k_sweep_wave_lag<R, 1, false, false, RunOpts>, k_sweep_wave_lag<R, 2, false, false, RunOpts>,
+       k_sweep_wave_lag<R, 3, false, false, RunOpts>},
+      {k_sweep_wave_lag<R, 1, false, true, RunOpts>, k_sweep_wave_lag<R, 2, false, true, RunOpts>,
+       k_sweep_wave_lag<R, 3, false, true, RunOpts>}};
   return kl[xd ? 1 : 0][m - 1];
 }
 // column-walking y sweep
@@ -1221,6 +1221,14 @@ static int createContext(const mhy_config* cfg, mhy_ctx** out, bool batchMember)
   o.flux_left = b.flux_left, o.flux_right = b.flux_right, o.flux_bottom = b.flux_bottom, o.flux_top = b.flux_top;
   o.flux_any = (b.flux_left + b.flux_right + b.flux_bottom + b.flux_top) > 0;
   x->fixLim = pickFixed(o);
+  // PenteBorne with fixed options (FP64, no mixte): the Lagrange update inside the
+  // first sweep of the x-first steps (110 VGPRs for two materials; 1280^2: 86 + 70
+  // us as two kernels, a step 415 -> 396 us).  Along y the strips recompute a
+  // third of it as halo, and with run-time options the sweep is bound by its
+  // arithmetic and registers: there it stays its own kernel.
+  if (c.pp == 1 && x->fixLim != 0 && !x->mixed && c.pp_mixte != 1 && x->sweepWave && !batchMember && x->geomStored &&
+      !std::getenv("MAHYCO_FUSE_LAGRANGE"))
+    x->fuseLag = true, x->fuseLagY = false;
   x->dualBoth = x->fixLim != 0 && x->sweepWave && !std::getenv("MAHYCO_DUAL_Y");
   x->dualRows = pickDualRows(dualBothItems(c.nx, c.ny, 2, true));
   x->nodeRows = nodeWalkRows(nodeWalkItems(c.nx, c.ny, 1));

@@ -64,8 +64,9 @@ dim3 sweepO3Grid(bool xd, long nx, long ny);
 // P: where the options come from (RunOpts, or FixOpts for the common sets)
 template <class R, int M, bool PP, bool XD, class P>
 __global__ void k_sweep_wave(KPT<R> kp);
-// the first sweep with the cell part of the Lagrange phase fused in (limited slopes)
-template <class R, int M, bool XD, class P>
+// the first sweep with the cell part of the Lagrange phase fused in (limited
+// slopes; PenteBorne with fixed options along x)
+template <class R, int M, bool PP, bool XD, class P>
 __global__ void k_sweep_wave_lag(KPT<R> kp);
 // the sweeps with fixed options for a limiter (fixedLimiter), m materials;
 // kind: 0 fused Lagrange sweep, 1 first sweep, 2 second sweep with the final

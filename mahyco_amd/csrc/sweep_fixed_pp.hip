@@ -9,6 +9,9 @@ namespace mhy {
 namespace {
 template <int M, bool XD, int LIM>
 SweepFn<double> pickPP(int sweep) {
+  if constexpr (XD) {
+    if (sweep == 0) return k_sweep_wave_lag<double, M, true, XD, FixOpts<LIM, 1>>;
+  }
   if (sweep == 1) return k_sweep_wave<double, M, true, XD, FixOpts<LIM, 1>>;
   return k_sweep_wave<double, M, true, XD, FixOpts<LIM, 2>>;
 }

@@ -9,7 +9,7 @@ namespace mhy {
 namespace {
 template <class R, int M, int LIM>
 SweepFn<R> pick(int kind) {
-  if (kind == 0) return k_sweep_wave_lag<R, M, true, FixOpts<LIM, 1>>;
+  if (kind == 0) return k_sweep_wave_lag<R, M, false, true, FixOpts<LIM, 1>>;
   if (kind == 1) return k_sweep_wave<R, M, false, true, FixOpts<LIM, 1>>;
   return k_sweep_wave<R, M, false, true, FixOpts<LIM, 2>>;
 }

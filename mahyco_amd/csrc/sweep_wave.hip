@@ -12,8 +12,8 @@ namespace mhy {
   template __global__ void k_sweep_wave_batch<R, M, PP, true, true, RunOpts>(BatchLaunchT<R>); \
   template __global__ void k_sweep_wave_batch<R, M, PP, false, true, RunOpts>(BatchLaunchT<R>);
 #define MHY_SWEEP_WAVE_LAG(R, M) \
-  template __global__ void k_sweep_wave_lag<R, M, true, RunOpts>(KPT<R>); \
-  template __global__ void k_sweep_wave_lag<R, M, false, RunOpts>(KPT<R>);
+  template __global__ void k_sweep_wave_lag<R, M, false, true, RunOpts>(KPT<R>); \
+  template __global__ void k_sweep_wave_lag<R, M, false, false, RunOpts>(KPT<R>);
 #define MHY_SWEEP_WAVE_INST_R(R) \
   MHY_SWEEP_WAVE_LAG(R, 1) \
   MHY_SWEEP_WAVE_LAG(R, 2) \

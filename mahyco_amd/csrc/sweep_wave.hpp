@@ -440,8 +440,8 @@ constexpr int kMinWavesBatch = (M < 3) ? kMinWaves<R, PP, XD> : 1;
 // costs no spill.  (With fixed options they take 79, 6 waves.)
 template <class R, int L, bool PP, bool XD, class P>
 constexpr int kMinWavesPlain = (!kMixed<R> && L == 1 && !PP) ? 5 : kMinWaves<R, PP, XD>;
-template <class R, int L, bool XD, class P>
-constexpr int kMinWavesLag = kParkLag<R, L, false> ? 5 : kMinWaves<R, false, XD>;
+template <class R, int L, bool PP, bool XD, class P>
+constexpr int kMinWavesLag = kParkLag<R, L, PP> ? 5 : kMinWaves<R, PP, XD>;
 
 template <class R, int M, bool PP, bool XD, class P>
 __global__ __launch_bounds__((XD ? 256 : 64 * kYWaves<R, PP>))
@@ -450,18 +450,17 @@ __attribute__((amdgpu_waves_per_eu(kMinWavesPlain<R, M, PP, XD, P>))) void k_swe
 }
 
 // the first sweep of a step with the cell part of the Lagrange phase
-// (limited slopes: with PenteBorne the update runs better as its own kernel)
-template <class R, int M, bool XD, class P>
-__global__ __launch_bounds__((XD ? 256 : 64 * kYWaves<R, false>))
-__attribute__((amdgpu_waves_per_eu(kMinWavesLag<R, M, XD, P>))) void k_sweep_wave_lag(KPT<R> kp) {
-  sweepWaveBody<R, M, false, XD, true, P>(kp, XD ? blockIdx.x : xcdBlock());
+template <class R, int M, bool PP, bool XD, class P>
+__global__ __launch_bounds__((XD ? 256 : 64 * kYWaves<R, PP>))
+__attribute__((amdgpu_waves_per_eu(kMinWavesLag<R, M, PP, XD, P>))) void k_sweep_wave_lag(KPT<R> kp) {
+  sweepWaveBody<R, M, PP, XD, true, P>(kp, XD ? blockIdx.x : xcdBlock());
 }
 
 // all problems of an ensemble in one launch, one workgroup per virtual block:
 // the first sweep with the Lagrange update
 template <class R, int M, bool XD, class P>
 __global__ __launch_bounds__((XD ? 256 : 64 * kYWaves<R, false>))
-__attribute__((amdgpu_waves_per_eu(kMinWavesLag<R, M, XD, P>))) void k_sweep_wave_lag_batch(BatchLaunchT<R> bl) {
+__attribute__((amdgpu_waves_per_eu(kMinWavesLag<R, M, false, XD, P>))) void k_sweep_wave_lag_batch(BatchLaunchT<R> bl) {
   batchRun<true>(bl, [&](const KPT<R>& kp, unsigned local, unsigned, unsigned) {
     sweepWaveBody<R, M, false, XD, true, P>(kp, local);
   });
