@@ -481,7 +481,7 @@ int phaseEucFinal(mhy_ctx* x) {
 // tile kernel for the third order.
 template <int L>
 EucSweepFn eucSweepFor(bool xd, bool pp, bool o3) {
-  if (o3) return xd ? k_sweep_o3<double, L, true> : k_sweep_o3<double, L, false>;
+  if (o3) return xd ? k_sweep_o3<double, L, true, RunOpts> : k_sweep_o3<double, L, false, RunOpts>;
   if (pp) return xd ? k_sweep_wave<double, L, true, true, RunOpts> : k_sweep_wave<double, L, true, false, RunOpts>;
   return xd ? k_sweep_wave<double, L, false, true, RunOpts> : k_sweep_wave<double, L, false, false, RunOpts>;
 }
@@ -506,7 +506,7 @@ int phaseEucSweep(mhy_ctx* x, int sweep, int stage) {
   const dim3 grid = o3 ? sweepO3Grid(xd, x->o.nx, x->o.ny) : sweepWaveGrid(xd, x->o.nx, x->o.ny, false, pp);
   const dim3 block(o3 ? kBlock : sweepWaveBlock(xd, false, pp));
   const Opts& o = x->o;
-  const bool fixedForm = x->fixLim == MHY_LIM_SUPERBEE && pp && o.conservative == 0 &&
+  const bool fixedForm = x->fixLim == MHY_LIM_SUPERBEE && pp && o.order == 2 && o.conservative == 0 &&
                          (o.pp_mixte != 1 || o.limiter_pure == MHY_LIM_ARITHMETICG);
   const EucSweepFn k = fixedForm ? sweepFixedEuc(xd, o.nbmat, o.pp_mixte == 1, sweep)
                                  : eucSweepKernel(xd, o.nbmat, pp, o.conservative == 1, o3);
@@ -592,6 +592,14 @@ SweepFn<R> walkKernel(int m, bool pp) {
                                       {k_sweep_walk<R, 3, false, RunOpts>, k_sweep_walk<R, 3, true, RunOpts>}};
   return kk[m - 1][pp ? 1 : 0];
 }
+// third-order sweep
+template <class R>
+SweepFn<R> o3Kernel(bool xd, int m) {
+  static const SweepFn<R> ko[2][3] = {
+      {k_sweep_o3<R, 1, false, RunOpts>, k_sweep_o3<R, 2, false, RunOpts>, k_sweep_o3<R, 3, false, RunOpts>},
+      {k_sweep_o3<R, 1, true, RunOpts>, k_sweep_o3<R, 2, true, RunOpts>, k_sweep_o3<R, 3, true, RunOpts>}};
+  return ko[xd ? 1 : 0][m - 1];
+}
 // the sweep compiled for a limiter's fixed options (lim from fixedLimiter), or
 // null where there is none: mixed-form PenteBorne, the PenteBorne mixte
 // option, walking PenteBorne sweeps, and a second sweep without the final
@@ -601,6 +609,7 @@ SweepFn<R> fixedKernel(const mhy_ctx* x, const KP& kp, bool xd, bool lag, bool w
   const int lim = x->fixLim, m = x->o.nbmat;
   if (lim == 0 || !kp.geomLoad || (kp.sweep == 2 && !kp.fuseFinal)) return nullptr;
   const int kind = lag ? 0 : kp.sweep;
+  if (x->o.order == 3) return sweepFixedO3<R>(xd, m, kind);
   if (x->o.pp == 1) {
     if constexpr (kMixed<R>) return nullptr;
     else return (x->o.pp_mixte == 1 || walk) ? nullptr : sweepFixedPP(xd, lim, m, kind);
@@ -654,14 +663,7 @@ int phaseSweepStage(mhy_ctx* x, int sweep, int stage) {
     if (walk) {
       launchForm(walkKernel<double>(m, pp), walkKernel<float>(m, pp), sweepWalkGrid(x->o.nx, x->o.ny, x->walkRows), dim3(kBlock));
     } else if (o3) {  // third order: LDS-tile kernel, no PenteBorne (checked at creation)
-      static const KernelFn kd[2][3] = {
-          {k_sweep_o3<double, 1, false>, k_sweep_o3<double, 2, false>, k_sweep_o3<double, 3, false>},
-          {k_sweep_o3<double, 1, true>, k_sweep_o3<double, 2, true>, k_sweep_o3<double, 3, true>}};
-      static const KernelFnF kf[2][3] = {
-          {k_sweep_o3<float, 1, false>, k_sweep_o3<float, 2, false>, k_sweep_o3<float, 3, false>},
-          {k_sweep_o3<float, 1, true>, k_sweep_o3<float, 2, true>, k_sweep_o3<float, 3, true>}};
-      const int di = xd ? 1 : 0, mi = x->o.nbmat - 1;
-      timed(x, xd ? K_SWEEP_X : K_SWEEP_Y, [&] { launchR(x, kd[di][mi], kf[di][mi], grid, block, kp); });
+      launchForm(o3Kernel<double>(xd, m), o3Kernel<float>(xd, m), grid, block);
     } else if (lagSweep) {  // with the cell part of the Lagrange phase
       launchForm(lagSweepKernel<double>(xd, m), lagSweepKernel<float>(xd, m), grid, block);
     } else if (wave) {
@@ -710,8 +712,8 @@ int phaseDualBoth(mhy_ctx* x) {
   const bool xfirst = x->x_then_y_n;
   const int items = dualBothItems(x->o.nx, x->o.ny, x->dualRows, xfirst);
   timed(x, K_DUAL, [&] {
-    launchR(x, dualBothKernel<double>(x->fixLim, x->o.nbmat, xfirst, x->dualRows),
-            dualBothKernel<float>(x->fixLim, x->o.nbmat, xfirst, x->dualRows), dim3((unsigned)((items + 3) / 4)), dim3(kBlock), kp);
+    launchR(x, dualBothKernel<double>(x->fixLim, x->o.nbmat, xfirst, x->dualRows, x->o.order),
+            dualBothKernel<float>(x->fixLim, x->o.nbmat, xfirst, x->dualRows, x->o.order), dim3((unsigned)((items + 3) / 4)), dim3(kBlock), kp);
   });
   x->keysNext = dualBothDt(x->dualRows);
   return checkLaunch(x, "dual");
@@ -2105,7 +2107,7 @@ int mhy_batch_create(const mhy_config* cfgs, int n, mhy_batch** out) {
     // (kind 1 and 2 of the limited-slope sweeps, one limiter for all)
     const int lim = (b->pp || b->o3) ? 0 : b->ctx[i]->fixLim;
     b->fixLim = (i == 0 || b->fixLim == lim) ? lim : 0;
-    const int dual = b->ctx[i]->dualBoth ? b->ctx[i]->fixLim : 0;
+    const int dual = (b->ctx[i]->dualBoth && !b->o3) ? b->ctx[i]->fixLim : 0;
     b->dualLim = (i == 0 || b->dualLim == dual) ? dual : 0;
   }
   b->cur0 = b->cur = b->ctx[0]->cur;

@@ -1,6 +1,6 @@
 // Nodal momentum remap of both sweeps in one kernel (remap/DualPhaseRemap1.cc,
 // remap/DualPhaseRemap2.cc), after both cell sweeps, for the options the
-// fixed sweeps take (second order, a classic limiter, mass fluxes).
+// fixed sweeps take (second or third order, a classic limiter, mass fluxes).
 //
 // One sweep at a time the nodal remap is bound by memory: it stores the nodal
 // momentum and mass and the Lagrange coordinate of the second axis for the
@@ -73,8 +73,8 @@ struct Nodal {
 
 // Upwind velocity through the dual face between the node before (pm, gm) and
 // this node (p, g): along velocity uN / u0, distance h, mass flux `flux`
-// (UtilesDualRemap.cc:234-397, second order).
-template <class T>
+// (UtilesDualRemap.cc:234-397; the gradient term times ORD - 1).
+template <int ORD, class T>
 __device__ __forceinline__ Vel<double> upwindFace(Vel<T> pm, Vel<T> gm, Vel<T> p, Vel<T> g, T uN, T u0, T h, T dtn,
                                                   double flux) {
   const T u = T(0.5) * (uN + u0);
@@ -82,7 +82,8 @@ __device__ __forceinline__ Vel<double> upwindFace(Vel<T> pm, Vel<T> gm, Vel<T> p
   const T s = T(sign) * h - dtn * u;
   const bool nb = flux > 0;
   const T bx = nb ? pm.x : p.x, by = nb ? pm.y : p.y, gx = nb ? gm.x : g.x, gy = nb ? gm.y : g.y;
-  return {(double)(bx + T(0.5) * gx * s), (double)(by + T(0.5) * gy * s)};
+  if constexpr (ORD == 2) return {(double)(bx + T(0.5) * gx * s), (double)(by + T(0.5) * gy * s)};
+  else return {(double)(bx + T(ORD - 1) * (T(0.5) * gx * s)), (double)(by + T(ORD - 1) * (T(0.5) * gy * s))};
 }
 
 // the nodal update from the fluxes through its two faces
@@ -100,7 +101,7 @@ __device__ __forceinline__ T slope(T gp, T gm) {
 }  // namespace
 
 // item: column group and band of this wave (kp.dualRows node rows per band)
-template <class R, int M, int LIM, bool XFIRST, bool DT>
+template <class R, int M, int LIM, bool XFIRST, bool DT, int ORD>
 __device__ __forceinline__ void dualBothBody(const KPT<R>& kp, int item) {
   using T = typename std::conditional<kMixed<R>, float, double>::type;
   const Opts& o = kp.o;
@@ -198,7 +199,7 @@ __device__ __forceinline__ void dualBothBody(const KPT<R>& kp, int item) {
     const Vel<T> dp = {after(d.x), after(d.y)};
     const Vel<T> g = {intX ? slope<LIM>(dp.x, d.x) : T(0), intX ? slope<LIM>(dp.y, d.y) : T(0)};
     const Vel<T> gm = {before(g.x), before(g.y)};
-    const Vel<double> um = upwindFace<T>(pm, gm, ph, g, pm.x, ph.x, h, dtnT, flux);
+    const Vel<double> um = upwindFace<ORD, T>(pm, gm, ph, g, pm.x, ph.x, h, dtnT, flux);
     const Vel<double> up = {after(um.x), after(um.y)};
     return updateNode(U, flux, after(flux), um, up, intX);
   };
@@ -237,7 +238,7 @@ __device__ __forceinline__ void dualBothBody(const KPT<R>& kp, int item) {
       fluxB += ((t >= 1 && t <= nx - 1) ? cm + c : (t >= 1 ? cm : c)) * wy;
       gyP[k] = w.gy[k];
     }
-    const Vel<double> upB = upwindFace<T>(phA, gA, phB, gB, phA.y, phB.y, T(ylB - ylA), dtnT, fluxB);
+    const Vel<double> upB = upwindFace<ORD, T>(phA, gA, phB, gB, phA.y, phB.y, T(ylB - ylA), dtnT, fluxB);
     const int a = r - 2;
     Nodal V = updateNode(UA, fluxA, fluxB, upA, upB, a >= 1 && a <= ny - 1);
     if constexpr (!XFIRST) {
@@ -288,15 +289,15 @@ __device__ __forceinline__ void dualBothBody(const KPT<R>& kp, int item) {
 }
 
 // (a wave past the last band leaves at once: the kernel has no barrier)
-template <class R, int M, int LIM, bool XFIRST, bool DT>
+template <class R, int M, int LIM, bool XFIRST, bool DT, int ORD>
 __global__ __launch_bounds__(256) void k_dual_both(KPT<R> kp) {
-  dualBothBody<R, M, LIM, XFIRST, DT>(kp, (int)(blockIdx.x * 4 + (threadIdx.x >> 6)));
+  dualBothBody<R, M, LIM, XFIRST, DT, ORD>(kp, (int)(blockIdx.x * 4 + (threadIdx.x >> 6)));
 }
 // all problems of an ensemble in one launch, one workgroup per virtual block
-template <class R, int M, int LIM, bool XFIRST, bool DT>
+template <class R, int M, int LIM, bool XFIRST, bool DT, int ORD>
 __global__ __launch_bounds__(256) void k_dual_both_batch(BatchLaunchT<R> bl) {
   batchRun<true>(bl, [&](const KPT<R>& kp, unsigned local, unsigned, unsigned) {
-    dualBothBody<R, M, LIM, XFIRST, DT>(kp, (int)(local * 4 + (threadIdx.x >> 6)));
+    dualBothBody<R, M, LIM, XFIRST, DT, ORD>(kp, (int)(local * 4 + (threadIdx.x >> 6)));
   });
 }
 
@@ -330,24 +331,27 @@ int dualBothRows(long waves2) {
 }
 
 namespace {
-template <class R, int M, int LIM>
+template <class R, int M, int LIM, int ORD>
 SweepFn<R> pick(bool xfirst, bool dt) {
-  if (dt) return xfirst ? k_dual_both<R, M, LIM, true, true> : k_dual_both<R, M, LIM, false, true>;
-  return xfirst ? k_dual_both<R, M, LIM, true, false> : k_dual_both<R, M, LIM, false, false>;
+  if (dt) return xfirst ? k_dual_both<R, M, LIM, true, true, ORD> : k_dual_both<R, M, LIM, false, true, ORD>;
+  return xfirst ? k_dual_both<R, M, LIM, true, false, ORD> : k_dual_both<R, M, LIM, false, false, ORD>;
 }
 template <class R, int M, int LIM>
 SweepBatchFn<R> pickBatch(bool xfirst, bool dt) {
-  if (dt) return xfirst ? k_dual_both_batch<R, M, LIM, true, true> : k_dual_both_batch<R, M, LIM, false, true>;
-  return xfirst ? k_dual_both_batch<R, M, LIM, true, false> : k_dual_both_batch<R, M, LIM, false, false>;
+  if (dt) return xfirst ? k_dual_both_batch<R, M, LIM, true, true, 2> : k_dual_both_batch<R, M, LIM, false, true, 2>;
+  return xfirst ? k_dual_both_batch<R, M, LIM, true, false, 2> : k_dual_both_batch<R, M, LIM, false, false, 2>;
+}
+template <class R, int M>
+SweepFn<R> pickLim(int lim, bool xf, bool dt, int order) {
+  if (order == 3)
+    return lim == MHY_LIM_MINMOD ? pick<R, M, MHY_LIM_MINMOD, 3>(xf, dt) : pick<R, M, MHY_LIM_SUPERBEE, 3>(xf, dt);
+  return lim == MHY_LIM_MINMOD ? pick<R, M, MHY_LIM_MINMOD, 2>(xf, dt) : pick<R, M, MHY_LIM_SUPERBEE, 2>(xf, dt);
 }
 }  // namespace
 template <class R>
-SweepFn<R> dualBothKernel(int lim, int m, bool xf, int rows) {
+SweepFn<R> dualBothKernel(int lim, int m, bool xf, int rows, int order) {
   const bool dt = dualBothDt(rows);
-  const bool mm = lim == MHY_LIM_MINMOD;
-  if (m == 1) return mm ? pick<R, 1, MHY_LIM_MINMOD>(xf, dt) : pick<R, 1, MHY_LIM_SUPERBEE>(xf, dt);
-  if (m == 2) return mm ? pick<R, 2, MHY_LIM_MINMOD>(xf, dt) : pick<R, 2, MHY_LIM_SUPERBEE>(xf, dt);
-  return mm ? pick<R, 3, MHY_LIM_MINMOD>(xf, dt) : pick<R, 3, MHY_LIM_SUPERBEE>(xf, dt);
+  return m == 1 ? pickLim<R, 1>(lim, xf, dt, order) : m == 2 ? pickLim<R, 2>(lim, xf, dt, order) : pickLim<R, 3>(lim, xf, dt, order);
 }
 template <class R>
 SweepBatchFn<R> dualBothBatchKernel(int lim, int m, bool xf, int rows) {
@@ -357,8 +361,8 @@ SweepBatchFn<R> dualBothBatchKernel(int lim, int m, bool xf, int rows) {
   if (m == 2) return mm ? pickBatch<R, 2, MHY_LIM_MINMOD>(xf, dt) : pickBatch<R, 2, MHY_LIM_SUPERBEE>(xf, dt);
   return mm ? pickBatch<R, 3, MHY_LIM_MINMOD>(xf, dt) : pickBatch<R, 3, MHY_LIM_SUPERBEE>(xf, dt);
 }
-template SweepFn<double> dualBothKernel<double>(int, int, bool, int);
-template SweepFn<float> dualBothKernel<float>(int, int, bool, int);
+template SweepFn<double> dualBothKernel<double>(int, int, bool, int, int);
+template SweepFn<float> dualBothKernel<float>(int, int, bool, int, int);
 template SweepBatchFn<double> dualBothBatchKernel<double>(int, int, bool, int);
 template SweepBatchFn<float> dualBothBatchKernel<float>(int, int, bool, int);
 

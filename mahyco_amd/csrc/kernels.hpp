@@ -7,6 +7,11 @@
 
 namespace mhy {
 
+template <class R>
+using SweepFn = void (*)(KPT<R>);
+template <class R>
+using SweepBatchFn = void (*)(BatchLaunchT<R>);
+
 // Eucclhyd Lagrange phase and final remap (eucclhyd.hip); M: materials
 template <int M>
 __global__ void k_euc_start(KP kp, EucFields e);
@@ -56,8 +61,10 @@ __global__ void k_dual_batch(BatchLaunchT<R> bl);
 template <int M, bool PP, bool XD>
 __global__ void k_sweep_cell(KP kp);
 // third-order sweep on LDS tiles (256-thread blocks)
-template <class R, int M, bool XD>
+template <class R, int M, bool XD, class P>
 __global__ void k_sweep_o3(KPT<R> kp);
+template <class R>
+SweepFn<R> sweepFixedO3(bool xd, int m, int kind);
 template <class R, int M, bool XD, bool ONE>
 __global__ void k_sweep_o3_batch(BatchLaunchT<R> bl);
 dim3 sweepO3Grid(bool xd, long nx, long ny);
@@ -71,10 +78,6 @@ __global__ void k_sweep_wave_lag(KPT<R> kp);
 // the sweeps with fixed options for a limiter (fixedLimiter), m materials;
 // kind: 0 fused Lagrange sweep, 1 first sweep, 2 second sweep with the final
 // remap
-template <class R>
-using SweepFn = void (*)(KPT<R>);
-template <class R>
-using SweepBatchFn = void (*)(BatchLaunchT<R>);
 template <class R>
 SweepFn<R> sweepFixedX(int lim, int m, int kind);
 template <class R>
@@ -117,7 +120,7 @@ unsigned dualWaveBlock(bool xd, bool mixed);
 // fixedLimiter), on bands of dualBothRows(waves at 2 rows) node
 // rows; dualBothItems: waves in all
 template <class R>
-SweepFn<R> dualBothKernel(int lim, int m, bool xfirst, int rows);
+SweepFn<R> dualBothKernel(int lim, int m, bool xfirst, int rows, int order);
 template <class R>
 SweepBatchFn<R> dualBothBatchKernel(int lim, int m, bool xfirst, int rows);
 int dualBothItems(long nx, long ny, int rows, bool xfirst);

@@ -77,10 +77,11 @@ struct FixOpts {
 };
 
 // The limiter of the fixed form these options have, or 0: they run the
-// run-time form.
+// run-time form.  Third order has it too (its own sweeps; the limiter is the
+// nodal remap's).
 inline int fixedLimiter(const Opts& o) {
   const bool classic = o.limiter == MHY_LIM_MINMOD || o.limiter == MHY_LIM_SUPERBEE;
-  bool ok = classic && o.order == 2 && o.mode == MODE_FULL && !o.flux_any && !o.periodic_right &&
+  bool ok = classic && (o.order == 2 || o.order == 3) && o.mode == MODE_FULL && !o.flux_any && !o.periodic_right &&
             (o.methode == 0 || o.euc) && !(o.pp == 1 && o.pp_complet == 1);
   for (int k = 0; k < o.nbmat; ++k) ok = ok && o.eos[k] == MHY_EOS_PERFECT_GAS;
   return ok ? o.limiter : 0;

@@ -10,8 +10,8 @@
 // so FP64 results are bitwise those of the CPU path.  The face fluxes are
 // also written per face for the nodal (dual) momentum remap.
 //
-// The file also holds the third-order sweep (projectionOrder 3), which reads
-// cells a-3 .. a+3 from an LDS tile (k_sweep_o3).
+// The file also holds the third-order sweep (projectionOrder 3) on LDS tiles
+// (k_sweep_o3).
 #include "final_math.hpp"
 #include "kernels.hpp"
 #include "sweep_math.hpp"
@@ -345,12 +345,19 @@ __global__ __launch_bounds__(256) void k_sweep_cell(KP kp) {
   }
 }
 
-// Third-order sweep on an LDS tile: each thread loads one cell (its means
-// U/V_L and its width), the block then forms the faces of its inner cells
-// from LDS.  Along x a block is 256 cells of a row, 250 updated; along y
-// 8 columns x 32 rows, 26 rows updated.  Slots past the domain edge load the
-// edge cell, which is what the reference's neighbour lookups return
-// (remap/UtilesMesh.cc:5-51).  Arithmetic order follows the reference.
+// Third-order sweep on an LDS tile, one cell per thread: along x a block is 256
+// cells of a row, 250 updated; along y 8 columns x 32 rows, 26 rows updated.
+// Slots past the domain edge load the edge cell, which is what the reference's
+// neighbour lookups return (remap/UtilesMesh.cc:5-51).
+//
+// Bound by FP64 arithmetic: a cell's two faces take the gradients of 5 cells,
+// 4 edge values and two fluxes, 51 quotients of widths among them.  Each is
+// formed once per tile slot, by the slot's own thread, and passed on through LDS:
+// its means, the gradient of its cell, the value at its minus edge, the flux
+// through its minus face.  The same functions of the same operands, so the
+// results are bitwise those of forming them for every cell, which took 136
+// VGPRs instead of 74 and 70 us per sweep of a 1024^2 one-material mesh (a step,
+// with the nodal remap of both sweeps in one kernel, 266 -> 188 us).
 namespace {
 constexpr int kO3Block = 256;
 constexpr int kO3XOut = kO3Block - 6;
@@ -359,74 +366,19 @@ constexpr int kO3YRows = kO3Block / kO3YCols;
 constexpr int kO3YOut = kO3YRows - 6;
 }  // namespace
 
-// the faces and the update of the inner cell at along index a, across
-// index t, whose tile slot is tid (sY: NC planes of kO3Block means)
-template <class R, int L, bool XD>
-__device__ __forceinline__ void sweepO3Cell(const KPT<R>& kp, const double* sY, const double* sH, int tid, long a,
-                                            long t, long na) {
-  constexpr int NC = kNC<L>;
-  constexpr int S = XD ? 1 : kO3YCols;  // thread distance of the along-sweep neighbour
-  const Opts& o = kp.o;
-  const auto& f = kp.f;
-  const long nx = o.nx;
-  const double dtn = f.sc->dt[kp.cur];
-  const long j = XD ? t : a, i = XD ? a : t;
-  const long c = j * nx + i;
-  // face normal velocity of face b, between along-cells b-1 and b
-  // (PrepareRemap.cc:50-62)
-  auto fnv = [&](long b) {
-    long n1, n2;
-    if (XD) n1 = j * (nx + 1) + b, n2 = (j + 1) * (nx + 1) + b;
-    else n1 = b * (nx + 1) + i, n2 = b * (nx + 1) + i + 1;
-    const R* u = XD ? kp.ul : kp.vl;
-    return 0.0 + ((0.0 + (double)u[n1]) + (double)u[n2]) * 0.5;
-  };
-  // Euler length of face b (Init.cc:528-533)
-  auto faceLen = [&](long b) {
-    D2 e1, e2;
-    if (XD) e1 = eulerNode(o, j, b), e2 = eulerNode(o, j + 1, b);
-    else e1 = eulerNode(o, b, i), e2 = eulerNode(o, b, i + 1);
-    return d2norm(d2sub(e2, e1));
-  };
-  const bool hasM = (a >= 1), hasP = (a + 1 < na);
-  const double Lm = faceLen(a), Lp = faceLen(a + 1);
-  const double vm = fnv(a), vp = fnv(a + 1);
-  double H[7];
-#pragma unroll
-  for (int k = 0; k < 7; ++k) H[k] = sH[tid + (k - 3) * S];
-  O3Grad gk[5];
-  O3Edge ek[4];
-#pragma unroll
-  for (int k = 1; k <= 5; ++k) gk[k - 1] = o3GradCoef(H[k - 1], H[k], H[k + 1]);
-#pragma unroll
-  for (int k = 1; k <= 4; ++k) ek[k - 1] = o3EdgeCoef(H[k - 1], H[k], H[k + 1], H[k + 2]);
-  const O3Sweep swM = o3SweepCoef(vm * dtn, H[2], H[3]), swP = o3SweepCoef(vp * dtn, H[3], H[4]);
-  double phiM[NC], phiP[NC];
-#pragma unroll
-  for (int q = 0; q < NC; ++q) {
-    double y[7], g[5], e[4];
-#pragma unroll
-    for (int k = 0; k < 7; ++k) y[k] = sY[q * kO3Block + tid + (k - 3) * S];
-#pragma unroll
-    for (int k = 1; k <= 5; ++k) g[k - 1] = o3Grad(gk[k - 1], y[k - 1], y[k], y[k + 1]);
-#pragma unroll
-    for (int k = 1; k <= 4; ++k) e[k - 1] = o3Edge(ek[k - 1], y[k], y[k + 1], g[k - 1], g[k]);
-    phiM[q] = hasM ? o3Flux(swM, y, e[0], e[1], e[2]) : 0.0;
-    phiP[q] = hasP ? o3Flux(swP, y + 1, e[1], e[2], e[3]) : 0.0;
-  }
-  sweepUpdateCell<R, L, false, XD, RunOpts, double>(kp, c, i, j, a, hasM, hasP, vm, vp, Lm, Lp, phiM, phiP);
-}
-
 // One tile; blk: its linear block index.  R: bulk storage type.  The face
 // values are FP64 in both forms (the remap vectors, V_L and the fluxes are
 // FP64; the mixed form stores the node velocities the widths come from in
-// FP32).  Every thread of the block reaches both barriers (no early
+// FP32).  Every thread of the block reaches every barrier (no early
 // return), so the ensemble kernels can run several tiles in one workgroup.
 // L: the remap-vector layout (kNC; VNR or Eucclhyd).
-template <class R, int L, bool XD>
+template <class R, int L, bool XD, class P>
 __device__ __forceinline__ void sweepO3Body(const KPT<R>& kp, unsigned blk) {
   constexpr int NC = kNC<L>;
+  constexpr int S = XD ? 1 : kO3YCols;  // thread distance of the along-sweep neighbour
   __shared__ double sY[NC][kO3Block];
+  __shared__ double sG[NC][kO3Block];  // gradients, then face fluxes
+  __shared__ double sE[NC][kO3Block];  // minus-edge values
   __shared__ double sH[kO3Block];
   const Opts& o = kp.o;
   const auto& f = kp.f;
@@ -450,33 +402,100 @@ __device__ __forceinline__ void sweepO3Body(const KPT<R>& kp, unsigned blk) {
     na = ny, nt = nx;
   }
   const bool inT = (t < nt);
-  double* const* Uin = (kp.sweep == 1) ? f.UL : f.U1;
+  double* const* Uin = (P::sweep(kp) == 1) ? f.UL : f.U1;
   // the time step of the end-of-Lagrange node positions (VNR: dt^{n+1};
   // Eucclhyd: dt^n, eucclhyd_remap/PhaseLagrange.cc:573-583)
-  const double dt1 = f.sc->dt[kEuc<L> ? kp.cur : kp.nxt];
+  const double dtn = f.sc->dt[kp.cur], dt1 = f.sc->dt[kEuc<L> ? kp.cur : kp.nxt];
+  double y0[NC], H0 = 0.0;
+#pragma unroll
+  for (int q = 0; q < NC; ++q) y0[q] = 0.0;
   if (inT) {
     const long b = min(max(a, 0L), na - 1);
     const long j = XD ? t : b, i = XD ? b : t;
     const long cb = j * nx + i;
     const double V = f.VL[cb];
 #pragma unroll
-    for (int q = 0; q < NC; ++q) sY[q][tid] = Uin[q][cb] / V;
-    sH[tid] = widthCell<XD>(kp, dt1, j, i);
+    for (int q = 0; q < NC; ++q) y0[q] = Uin[q][cb] / V;
+    H0 = widthCell<XD>(kp, dt1, j, i);
+  }
+#pragma unroll
+  for (int q = 0; q < NC; ++q) sY[q][tid] = y0[q];
+  sH[tid] = H0;
+  __syncthreads();
+  // gradient of this slot's cell (the first and last slot have no neighbour)
+  const bool g1 = slot >= 1 && slot <= last - 1;
+  double Hm = 0.0, Hp = 0.0;
+  if (g1) {
+    Hm = sH[tid - S], Hp = sH[tid + S];
+    const O3Grad gk = o3GradCoef(Hm, H0, Hp);
+#pragma unroll
+    for (int q = 0; q < NC; ++q) sG[q][tid] = o3Grad(gk, sY[q][tid - S], y0[q], sY[q][tid + S]);
   }
   __syncthreads();
-  if (inT && a >= 0 && a < na && slot >= 3 && slot <= last - 3) sweepO3Cell<R, L, XD>(kp, sY[0], sH, tid, a, t, na);
+  // value at the edge towards the slot before
+  double e0[NC];
+#pragma unroll
+  for (int q = 0; q < NC; ++q) e0[q] = 0.0;
+  if (g1 && slot >= 2) {
+    const O3Edge ek = o3EdgeCoef(sH[tid - 2 * S], Hm, H0, Hp);
+#pragma unroll
+    for (int q = 0; q < NC; ++q) {
+      e0[q] = o3Edge(ek, sY[q][tid - S], y0[q], sG[q][tid - S], sG[q][tid]);
+      sE[q][tid] = e0[q];
+    }
+  }
+  __syncthreads();
+  const long j = XD ? t : a, i = XD ? a : t;
+  // face normal velocity of face b, between along-cells b-1 and b
+  // (PrepareRemap.cc:50-62)
+  auto fnv = [&](long b) {
+    long n1, n2;
+    if (XD) n1 = j * (nx + 1) + b, n2 = (j + 1) * (nx + 1) + b;
+    else n1 = b * (nx + 1) + i, n2 = b * (nx + 1) + i + 1;
+    const R* u = XD ? kp.ul : kp.vl;
+    return 0.0 + ((0.0 + (double)u[n1]) + (double)u[n2]) * 0.5;
+  };
+  // flux value of the face towards the slot before, where that face is inside
+  // the domain (the gradients in sG are no longer needed)
+  const bool inner = inT && a >= 1 && a < na;
+  const double vm = (inT && a >= 0 && a <= na) ? fnv(a) : 0.0;
+  double phiM[NC];
+#pragma unroll
+  for (int q = 0; q < NC; ++q) phiM[q] = 0.0;
+  if (inner && slot >= 3 && slot <= last - 2) {
+    const O3Sweep sw = o3SweepCoef(vm * dtn, Hm, H0);
+#pragma unroll
+    for (int q = 0; q < NC; ++q) {
+      // means of the cells a-2 .. a+1 in their places of the six around the face
+      const double y[6] = {0.0, sY[q][tid - 2 * S], sY[q][tid - S], y0[q], sY[q][tid + S], 0.0};
+      phiM[q] = o3Flux(sw, y, sE[q][tid - S], e0[q], sE[q][tid + S]);
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < NC; ++q) sG[q][tid] = phiM[q];
+  __syncthreads();
+  if (inT && a >= 0 && a < na && slot >= 3 && slot <= last - 3) {
+    const bool hasM = (a >= 1), hasP = (a + 1 < na);
+    const double vp = fnv(a + 1);
+    double phiP[NC];
+#pragma unroll
+    for (int q = 0; q < NC; ++q) phiP[q] = hasP ? sG[q][tid + S] : 0.0;
+    // Euler face length (Init.cc:528-533): sqrt(fl(w w)) = |w|, the same for both faces
+    const double w = XD ? fabs(o.dy * (double)(j + 1) - o.dy * (double)j) : fabs(o.dx * (double)(i + 1) - o.dx * (double)i);
+    sweepUpdateCell<R, L, false, XD, P, double>(kp, j * nx + i, i, j, a, hasM, hasP, vm, vp, w, w, phiM, phiP);
+  }
   __syncthreads();  // the ensemble kernels reuse the tile for their next block
 }
 
-template <class R, int M, bool XD>
+template <class R, int M, bool XD, class P>
 __global__ __launch_bounds__(kO3Block) void k_sweep_o3(KPT<R> kp) {
-  sweepO3Body<R, M, XD>(kp, blockIdx.x);
+  sweepO3Body<R, M, XD, P>(kp, blockIdx.x);
 }
 
 // all problems of an ensemble in one launch (BatchLaunchT, common.hpp)
 template <class R, int M, bool XD, bool ONE>
 __global__ __launch_bounds__(kO3Block) void k_sweep_o3_batch(BatchLaunchT<R> bl) {
-  batchRun<ONE>(bl, [&](const KPT<R>& kp, unsigned local, unsigned, unsigned) { sweepO3Body<R, M, XD>(kp, local); });
+  batchRun<ONE>(bl, [&](const KPT<R>& kp, unsigned local, unsigned, unsigned) { sweepO3Body<R, M, XD, RunOpts>(kp, local); });
 }
 
 dim3 sweepO3Grid(bool xd, long nx, long ny) {
@@ -485,8 +504,8 @@ dim3 sweepO3Grid(bool xd, long nx, long ny) {
 }
 
 #define MHY_SWEEP_O3_INST(R, M)                                                \
-  template __global__ void k_sweep_o3<R, M, true>(KPT<R>);                       \
-  template __global__ void k_sweep_o3<R, M, false>(KPT<R>);                      \
+  template __global__ void k_sweep_o3<R, M, true, RunOpts>(KPT<R>);              \
+  template __global__ void k_sweep_o3<R, M, false, RunOpts>(KPT<R>);             \
   template __global__ void k_sweep_o3_batch<R, M, true, false>(BatchLaunchT<R>);  \
   template __global__ void k_sweep_o3_batch<R, M, false, false>(BatchLaunchT<R>); \
   template __global__ void k_sweep_o3_batch<R, M, true, true>(BatchLaunchT<R>);   \
@@ -501,8 +520,8 @@ MHY_SWEEP_O3_INST(float, 3)
 
 // the Eucclhyd layouts (FP64 only, no ensembles)
 #define MHY_SWEEP_O3_EUC(L)                                  \
-  template __global__ void k_sweep_o3<double, L, true>(KP); \
-  template __global__ void k_sweep_o3<double, L, false>(KP);
+  template __global__ void k_sweep_o3<double, L, true, RunOpts>(KP); \
+  template __global__ void k_sweep_o3<double, L, false, RunOpts>(KP);
 MHY_SWEEP_O3_EUC(5)
 MHY_SWEEP_O3_EUC(6)
 MHY_SWEEP_O3_EUC(7)
@@ -510,6 +529,23 @@ MHY_SWEEP_O3_EUC(9)
 MHY_SWEEP_O3_EUC(10)
 MHY_SWEEP_O3_EUC(11)
 #undef MHY_SWEEP_O3_EUC
+
+// The third-order sweeps with the options their update takes fixed (perfect
+// gases, mass fluxes, the sweep order; the limiter is the nodal remap's only)
+namespace {
+template <class R, int M, bool XD>
+SweepFn<R> pickO3(int sweep) {
+  return sweep == 1 ? k_sweep_o3<R, M, XD, FixOpts<MHY_LIM_MINMOD, 1>> : k_sweep_o3<R, M, XD, FixOpts<MHY_LIM_MINMOD, 2>>;
+}
+}  // namespace
+template <class R>
+SweepFn<R> sweepFixedO3(bool xd, int m, int sweep) {
+  if (m == 1) return xd ? pickO3<R, 1, true>(sweep) : pickO3<R, 1, false>(sweep);
+  if (m == 2) return xd ? pickO3<R, 2, true>(sweep) : pickO3<R, 2, false>(sweep);
+  return xd ? pickO3<R, 3, true>(sweep) : pickO3<R, 3, false>(sweep);
+}
+template SweepFn<double> sweepFixedO3<double>(bool, int, int);
+template SweepFn<float> sweepFixedO3<float>(bool, int, int);
 
 #define MHY_SWEEP_CELL_INST(M, PP)                       \
   template __global__ void k_sweep_cell<M, PP, true>(KP); \

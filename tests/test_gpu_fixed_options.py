@@ -10,7 +10,9 @@ import pytest
 import mahyco_amd
 from mahyco_amd import abi, configs
 
-from gpu_helpers import MAT, field_names, log
+from oracle import refcpu
+
+from gpu_helpers import MAT, compare_state, field_names, log
 from test_gpu_variants import env
 
 pytestmark = pytest.mark.gpu
@@ -75,6 +77,27 @@ def test_penteborne(m, nx, ny, limiter):
     cfg = problem(m, nx, ny, limiter, pp=1)
     log(f"[fixed] PenteBorne m={m} {nx}x{ny} {limiter}")
     assert_equal_runs(lambda: mahyco_amd.Context(cfg), field_names(cfg), chunks=(1, 2, 60))
+
+
+@pytest.mark.parametrize("precision", [0, 1], ids=["fp64", "mixed"])
+@pytest.mark.parametrize("m,nx,ny", [(1, 2, 2), (1, 250, 26), (2, 251, 27), (3, 253, 3), (1, 8, 55), (2, 9, 29)])
+def test_third_order(m, nx, ny, precision):
+    """Tiles of 250 columns and of 8 columns x 26 rows; FP64 also against the oracle."""
+    cfg = problem(m, max(nx, 8), ny, "superBee", precision)
+    cfg.nx, cfg.projection_order = nx, 3
+    log(f"[fixed] order 3 m={m} {nx}x{ny} precision={precision}")
+    assert_equal_runs(lambda: mahyco_amd.Context(cfg), field_names(cfg))
+    if precision == 0:
+        ctx, orc = mahyco_amd.Context(cfg), refcpu.Oracle(cfg)
+        try:
+            for n in (1, 2, 9):
+                ctx.run(n)
+                orc.step(n)
+                _, name, bitwise = compare_state(ctx, orc, cfg)
+                assert bitwise, name
+        finally:
+            ctx.close()
+            orc.close()
 
 
 @pytest.mark.parametrize("mixte", [0, 1])
