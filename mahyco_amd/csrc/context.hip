@@ -108,8 +108,10 @@ struct mhy_ctx {
   bool fuseLag = true;
   // ... also on steps whose first sweep runs along y (the tuner may turn it
   // off there: the y strips recompute a third of their cells as halo)
-  // (MAHYCO_LAG_Y=fused / separate forces either)
+  // (MAHYCO_LAG_Y=fused / separate / walk forces one)
   bool fuseLagY = true;
+  // ... there on walking bands instead of strips (fixed options only)
+  bool lagWalkY = false;
   // with the fused first sweep: that sweep stores the Lagrange volume and
   // centroid for the second (environment MAHYCO_SWEEP_GEOM=load), or the
   // second sweep forms them again from the node velocities (=recompute)
@@ -290,10 +292,10 @@ KP makeKP(const mhy_ctx* x) {
 // nodal remap along y (TD_BOTH: of both sweeps, in one kernel)
 enum { TD_TILE = 0, TD_WAVE = 1, TD_WALK = 2, TD_TILE32 = 3, TD_TILE64 = 4, TD_BOTH = 5 };
 enum { TS_WAVE = 0, TS_WALK = 1 };               // cell sweep along y
-enum { TL_FUSED = 0, TL_SEPARATE = 1 };          // Lagrange cell update of y-first steps
+enum { TL_FUSED = 0, TL_SEPARATE = 1, TL_WALK = 2 };  // Lagrange cell update of y-first steps
 const char* kDualNames[6] = {"tile", "wave", "walk", "tile32", "tile64", "both"};
 const char* kSweepNames[2] = {"wave", "walk"};
-const char* kLagNames[2] = {"fused", "separate"};
+const char* kLagNames[3] = {"fused", "separate", "walk"};
 
 void setDualY(mhy_ctx* x, int c) {
   x->dualTileY = (c == TD_TILE || c == TD_TILE32 || c == TD_TILE64);
@@ -302,12 +304,17 @@ void setDualY(mhy_ctx* x, int c) {
   x->dualWaveY = true;
 }
 
+void setLagY(mhy_ctx* x, int c) {
+  x->fuseLagY = (c != TL_SEPARATE);
+  x->lagWalkY = (c == TL_WALK);
+}
+
 // Applies candidate index ci of a site.
 void tuneApply(mhy_ctx* x, int site, int ci) {
   const int id = x->tune.cand[site][ci];
   if (site == 0) setDualY(x, id);
   else if (site == 1) x->walkY = (id == TS_WALK);
-  else x->fuseLagY = (id == TL_FUSED);
+  else setLagY(x, id);
 }
 
 // The site, round and candidate index of tuning step k (sites one after the
@@ -650,7 +657,7 @@ int phaseSweepStage(mhy_ctx* x, int sweep, int stage) {
                            : gridFor(x->ncell);
     const dim3 block(wave ? sweepWaveBlock(xd, x->mixed, x->o.pp == 1) : kBlock);
     const bool lagSweep = (sweep == 1 && lagFused(x));
-    const bool walk = !xd && wave && x->walkY && !lagSweep;
+    const bool walk = !xd && wave && (lagSweep ? x->lagWalkY && fixedKernel<double>(x, kp, false, true, true) : x->walkY);
     const KernelId kid = lagSweep ? (xd ? K_LAGSWEEP_X : K_LAGSWEEP_Y) : (xd ? K_SWEEP_X : K_SWEEP_Y);
     const int m = x->o.nbmat;
     const bool pp = x->o.pp == 1;
@@ -1151,8 +1158,9 @@ static int createContext(const mhy_config* cfg, mhy_ctx** out, bool batchMember)
   if (const char* fl = std::getenv("MAHYCO_FUSE_LAGRANGE"))
     if (std::string(fl) == "0") x->fuseLag = false;
   if (const char* ly = std::getenv("MAHYCO_LAG_Y")) {
-    x->fuseLagY = (std::string(ly) != "separate");
-    x->tune.forcedLag = kLagNames[x->fuseLagY ? TL_FUSED : TL_SEPARATE];
+    const int c = std::string(ly) == "separate" ? TL_SEPARATE : std::string(ly) == "walk" ? TL_WALK : TL_FUSED;
+    setLagY(x, c);
+    x->tune.forcedLag = kLagNames[c];
     x->tune.choice = "lagrange_y=" + x->tune.forcedLag;
   }
   if (const char* sn = std::getenv("MAHYCO_SPLIT_NODE")) x->splitNode = (std::string(sn) != "0");
@@ -1231,6 +1239,13 @@ static int createContext(const mhy_config* cfg, mhy_ctx** out, bool batchMember)
   if (c.pp == 1 && x->fixLim != 0 && !x->mixed && c.pp_mixte != 1 && x->sweepWave && !batchMember && x->geomStored &&
       !std::getenv("MAHYCO_FUSE_LAGRANGE"))
     x->fuseLag = true, x->fuseLagY = false;
+  // y-first steps of the fixed options: the fused Lagrange update on strips or on
+  // walking bands, which recompute 4 rows a band of up to 32 instead of 4 of 12 but hold
+  // 2-3 waves per SIMD.  us per step, separate kernel / strips / bands: 3 materials
+  // FP64 3072x2048 1526 / 1551 / 1415, mixed 1151 / 1136 / 1057; one material
+  // FP64 4096^2 1713 / 1667 / 1630, 2048^2 478 / 464 / 473, 1280x1024 190 / 178 / 181:
+  // the separate kernel is the best of none, so it is not tried there.
+  if (x->fixLim != 0 && x->geomStored && x->tune.ncand[2] == 2) x->tune.cand[2][1] = TL_WALK;
   x->dualBoth = x->fixLim != 0 && x->sweepWave && !std::getenv("MAHYCO_DUAL_Y");
   x->dualRows = pickDualRows(dualBothItems(c.nx, c.ny, 2, true));
   x->nodeRows = nodeWalkRows(nodeWalkItems(c.nx, c.ny, 1));

@@ -4,11 +4,12 @@
 
 namespace mhy {
 
-// the walkers with their options fixed: sweep 1 (after the separate Lagrange
-// kernel) or 2 (with the final remap)
+// the walkers with their options fixed: sweep 1 with the Lagrange update (0) or after
+// the separate Lagrange kernel (1), sweep 2 with the final remap (2)
 namespace {
 template <class R, int M, int LIM>
 SweepFn<R> pickWalk(int sweep) {
+  if (sweep == 0) return k_sweep_walk_lag<R, M, FixOpts<LIM, 1>>;
   return sweep == 1 ? k_sweep_walk<R, M, false, FixOpts<LIM, 1>> : k_sweep_walk<R, M, false, FixOpts<LIM, 2>>;
 }
 }  // namespace

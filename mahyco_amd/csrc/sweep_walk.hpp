@@ -10,12 +10,17 @@
 // the face value between the two rows before, and the update of the row
 // two back.  Operation order is that of the wave-strip sweeps (and of the
 // reference), so FP64 results are bitwise the same.
+//
+// LAG: the first sweep of a step with the cell part of the Lagrange phase, as the
+// strips have it: a row's remap vector waits two iterations in a ring of three slots per
+// thread in LDS, and only the band's own rows store what outlives the step.
 #pragma once
 
 #include <type_traits>
 
 #include "final_math.hpp"
 #include "kernels.hpp"
+#include "lagrange_cell.hpp"
 #include "sweep_math.hpp"
 #include "sweep_update.hpp"
 
@@ -47,7 +52,7 @@ __device__ __forceinline__ double widthY(const KPT<R>& kp, double dt1, long j, l
 
 // b: linear block index; the waves of all bands are numbered column-group
 // first, 4 per block.
-template <class R, int M, bool PP, class P>
+template <class R, int M, bool PP, class P, bool LAG = false>
 __device__ __forceinline__ void sweepWalkYBody(const KPT<R>& kp, unsigned b) {
   using T = typename std::conditional<kMixed<R> && !PP, float, double>::type;
   constexpr int NC = 3 * M + 1;
@@ -80,6 +85,10 @@ __device__ __forceinline__ void sweepWalkYBody(const KPT<R>& kp, unsigned b) {
   T HA = T(0.0), HB = T(0.0);
   int flA = 0, flB = 0;
 
+  // LAG: the remap vectors of the last three rows, each thread its own slots
+  __shared__ double uRing[LAG ? 3 : 1][LAG ? NC : 1][LAG ? 256 : 1];
+  int slot = 0;  // ring slot of the new row
+
   for (int k = 0; k < rows + 4; ++k) {
     // the column and what derives from it (addresses, Euler coordinates) are
     // formed again for every row from an opaque copy of the index: hoisted
@@ -92,6 +101,20 @@ __device__ __forceinline__ void sweepWalkYBody(const KPT<R>& kp, unsigned b) {
     auto loadRow = [&](long r, T* ph, double& x, T& h, int& flg) {
       const long cb = r * nx + i;
       double u[NC];
+      if constexpr (LAG) {
+        // the Lagrange update of the cell; a band's own rows store what outlives the step
+        const bool own = r >= a0 && r < a0 + rows;
+        LagCell<M> lc;
+        lagrangeCellCompute<R, M, P>(kp, cb, r, i, own, lc);
+#pragma unroll
+        for (int q = 0; q < NC; ++q) u[q] = lc.U[q], uRing[slot][q][threadIdx.x] = lc.U[q];
+        cellPhi<M, PP, T>(u, lc.V, lc.q, ph);
+        x = lc.xc.y;
+        if (own) at(f.VL, cb) = lc.V, at(f.XcL, cb) = lc.xc.x;
+        h = needH ? T(widthY(kp, dt1, r, i)) : T(0.0);
+        flg = 0;
+        return;
+      }
       const int nload = PP ? 3 * M : NC;
 #pragma unroll
       for (int q = 0; q < NC; ++q) u[q] = (q < nload) ? at(Uin[q], cb) : 0.0;
@@ -192,7 +215,13 @@ __device__ __forceinline__ void sweepWalkYBody(const KPT<R>& kp, unsigned b) {
 #pragma unroll
         for (int k2 = 0; k2 < M; ++k2) at(f.DF[k2], c) = formed ? (double)dualA[k2] * w : 0.0;
       }
-      sweepUpdateCell<R, M, PP, false, P, T>(kp, c, i, rA, rA, hasM, hasP, vA, vB, Lm, Lp, phiM, phiP);
+      double uOwn[LAG ? NC : 1];
+      if constexpr (LAG) {
+        const int sA = slot == 2 ? 0 : slot + 1;  // two rows ago
+#pragma unroll
+        for (int q = 0; q < NC; ++q) uOwn[q] = uRing[sA][q][threadIdx.x];
+      }
+      sweepUpdateCell<R, M, PP, false, P, T>(kp, c, i, rA, rA, hasM, hasP, vA, vB, Lm, Lp, phiM, phiP, LAG ? uOwn : nullptr);
     }
 
     // rotate: B becomes A, N becomes B
@@ -210,6 +239,7 @@ __device__ __forceinline__ void sweepWalkYBody(const KPT<R>& kp, unsigned b) {
     HA = HB, HB = HN;
     flA = flB, flB = flN;
     vA = vB, vB = vN;
+    if constexpr (LAG) slot = slot == 2 ? 0 : slot + 1;
   }
 }
 
@@ -222,6 +252,14 @@ template <class R, int M, bool PP, class P>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWalkWaves<R, M, PP>))) void k_sweep_walk(
     KPT<R> kp) {
   sweepWalkYBody<R, M, PP, P>(kp, blockIdx.x);
+}
+
+// the first sweep of a step with the cell part of the Lagrange phase.  FP64: 166 VGPRs
+// (3 waves per SIMD), 207, 253 for 1, 2, 3 materials; mixed 138, 165, 191.  Held to 4
+// waves it spills: 4096^2 1630 -> 2105 us a step, 2048^2 mixed 402 -> 409.
+template <class R, int M, class P>
+__global__ __launch_bounds__(256) void k_sweep_walk_lag(KPT<R> kp) {
+  sweepWalkYBody<R, M, false, P, true>(kp, blockIdx.x);
 }
 
 template <class R, int M, bool PP, bool ONE>
