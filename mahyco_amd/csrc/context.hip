@@ -106,8 +106,8 @@ struct mhy_ctx {
   // sweep 1 runs the cell part of the Lagrange phase (wave sweeps only;
   // environment MAHYCO_FUSE_LAGRANGE=0 keeps it a separate kernel)
   bool fuseLag = true;
-  // ... also on steps whose first sweep runs along y (the tuner may turn it
-  // off there: the y strips recompute a third of their cells as halo)
+  // ... also on steps whose first sweep runs along y (the y strips recompute a
+  // third of their cells as halo: the tuner may turn it off, or into bands)
   // (MAHYCO_LAG_Y=fused / separate / walk forces one)
   bool fuseLagY = true;
   // ... there on walking bands instead of strips (fixed options only)
@@ -172,10 +172,11 @@ struct mhy_ctx {
   int launches[K_COUNT] = {0};
   // Launch-shape tuner.  The y-direction kernels come in interchangeable
   // variants with different tilings (results bitwise the same): the nodal
-  // remap as 16x64-node LDS tiles, 4x16-node wave strips or 64-column
-  // walking bands; the cell sweep as 4x16-cell wave strips or 64-column
+  // remap, where it is not one kernel for both sweeps, as LDS tiles, 4x16-node
+  // wave strips or 64-column walking bands; the cell sweep as 4x16-cell wave strips or 64-column
   // walking bands; and, on steps whose first sweep runs along y, the
-  // Lagrange cell update fused into that sweep or run as its own kernel.  On
+  // Lagrange cell update fused into that sweep on strips or on walking bands
+  // (fixed options), or on strips or run as its own kernel.  On
   // a large problem the first steps time whole steps, one site after the
   // other (the other sites keep their current choice): kTuneRounds rounds
   // over the site's candidates, two steps per candidate and round (one of
