@@ -13,6 +13,7 @@
 #include <string>
 #include <vector>
 
+#include "block_tuner.hpp"
 #include "common.hpp"
 #include "host/init.hpp"
 #include "host/output.hpp"
@@ -1974,8 +1975,7 @@ struct mhy_batch {
   long long cells = 0;
   bool tune = true, useGraph = true;
   int tuneStep = 0;
-  float tuneMs[BK_COUNT][kNCand] = {};
-  bool ran[BK_COUNT] = {};  // launched (and timed) in the last tuning step
+  BlockTuner<BK_COUNT, kNCand> tuner;
   hipEvent_t ev[2 * BK_COUNT] = {};
   hipGraphExec_t exec[2] = {nullptr, nullptr};
   std::string err;
@@ -2005,7 +2005,7 @@ int batchEnqueueStepR(mhy_batch* b, int cur, bool xty, bool timing, bool reduce)
     const bool one = !fnLoop || b->blocks[k] == 0 || b->blocks[k] >= b->total[k];
     const unsigned grid = one ? b->total[k] : b->blocks[k];
     const Fn fn = one ? fnOne : fnLoop;
-    b->ran[k] = true;
+    if (fnLoop) b->tuner.launched(k);
     if (timing) (void)hipEventRecord(b->ev[2 * k], b->stream);
     hipLaunchKernelGGL(fn, dim3(grid), dim3(block), 0, b->stream, bl);
     if (timing) (void)hipEventRecord(b->ev[2 * k + 1], b->stream);
@@ -2077,12 +2077,7 @@ int batchCapture(mhy_batch* b) {
 
 // picks, per kernel, the candidate workgroup count with the shortest time
 void batchPickBlocks(mhy_batch* b) {
-  for (int k = 0; k < BK_COUNT; ++k) {
-    int best = 0;
-    for (int c = 1; c < kNCand; ++c)
-      if (b->tuneMs[k][c] > 0.f && (b->tuneMs[k][best] <= 0.f || b->tuneMs[k][c] < b->tuneMs[k][best])) best = c;
-    b->blocks[k] = kCand[best];
-  }
+  for (int k = 0; k < BK_COUNT; ++k) b->blocks[k] = kCand[b->tuner.pick(k)];
 }
 
 }  // namespace
@@ -2253,13 +2248,14 @@ int mhy_batch_run(mhy_batch* b, int nsteps) {
       // at candidate tuneStep / 2, timed
       const int cand = b->tuneStep / 2;
       for (int k = 0; k < BK_COUNT; ++k) b->blocks[k] = kCand[cand];
+      b->tuner.begin();
       if ((st = batchEnqueueStep(b, b->cur, b->xty, true, reduce)) != MHY_OK) return st;
       if (hipStreamSynchronize(b->stream) != hipSuccess) return batchFail(b, MHY_ERR_DEVICE, "batch sync");
       const bool verbose = std::getenv("MAHYCO_BATCH_VERBOSE") != nullptr;
       for (int k = 0; k < BK_COUNT; ++k) {  // a kernel runs at most once per step
-        if (!b->ran[k]) continue;
+        if (!b->tuner.timed[k]) continue;
         float ms = 0.f;
-        if (hipEventElapsedTime(&ms, b->ev[2 * k], b->ev[2 * k + 1]) == hipSuccess) b->tuneMs[k][cand] += ms;
+        if (hipEventElapsedTime(&ms, b->ev[2 * k], b->ev[2 * k + 1]) == hipSuccess) b->tuner.add(k, cand, ms);
         if (verbose) std::fprintf(stderr, "[batch tune] kernel %d blocks %u: %.4f ms\n", k, kCand[cand], ms);
       }
       if (++b->tuneStep == kTuneSteps) {
