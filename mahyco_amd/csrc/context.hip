@@ -1453,9 +1453,11 @@ int captureStep(mhy_ctx* x) {
 // One step (without the n/n+1 swap): a replay of the captured step when
 // graphs is set, else eager launches.
 int stepOnce(mhy_ctx* x, bool graphs) {
-  // no graph is captured before the tuner has fixed the kernel variants
-  // nor from a state whose dt accumulators the reduction kernel has to fill first
-  if (!graphs || x->tune.on || (leavesDt(x) && !x->keysFull)) return runIteration(x);
+  // no graph is captured before the tuner has fixed the kernel variants, nor
+  // replayed from a state whose dt accumulators are not as this context's own steps leave
+  // them: empty after a field was written, or full after an ensemble's step in a
+  // problem whose bands are too short to fill them alone
+  if (!graphs || x->tune.on || leavesDt(x) != x->keysFull) return runIteration(x);
   hipGraphExec_t& g = x->graph[2 * x->cur + (x->x_then_y_n ? 1 : 0)];
   if (!g) {
     const int st = captureStep(x);
