@@ -526,6 +526,9 @@ int phaseEucSweep(mhy_ctx* x, int sweep, int stage) {
 int phaseDt(mhy_ctx* x) {
   if (x->euc) return phaseEucStart(x);
   tuneSelect(x);  // a step starts here
+  // (its dt empties the next step's accumulators, which the last step of a finished
+  // time loop, never swapped, may have left full)
+  x->keysNext = false;
   KP kp = makeKP(x);
   if (x->o.mode == MODE_ADVECTION) {
     timed(x, K_DT, [&] { launchR(x, k_dt_hold<double>, k_dt_hold<float>, dim3(1), dim3(64), kp); });
