@@ -517,8 +517,8 @@ int phaseEucSweep(mhy_ctx* x, int sweep, int stage) {
   const Opts& o = x->o;
   const bool fixedForm = x->fixLim == MHY_LIM_SUPERBEE && pp && o.order == 2 && o.conservative == 0 &&
                          (o.pp_mixte != 1 || o.limiter_pure == MHY_LIM_ARITHMETICG);
-  const EucSweepFn k = fixedForm ? sweepFixedEuc(xd, o.nbmat, o.pp_mixte == 1, sweep)
-                                 : eucSweepKernel(xd, o.nbmat, pp, o.conservative == 1, o3);
+  EucSweepFn k = fixedForm ? sweepFixedEuc(xd, o.nbmat, o.pp_mixte == 1, sweep) : nullptr;
+  if (!k) k = eucSweepKernel(xd, o.nbmat, pp, o.conservative == 1, o3);
   timed(x, xd ? K_SWEEP_X : K_SWEEP_Y, [&] { hipLaunchKernelGGL(k, grid, block, 0, x->stream, kp); });
   return checkLaunch(x, "eucclhyd sweep");
 }
@@ -586,9 +586,11 @@ SweepFn<R> sweepWaveKernel(bool xd, int m, bool pp) {
        {k_sweep_wave<R, 3, false, true, RunOpts>, k_sweep_wave<R, 3, true, true, RunOpts>}}};
   return kw[xd ? 1 : 0][m - 1][pp ? 1 : 0];
 }
-// the first sweep with the fused Lagrange update
+// the first sweep with the fused Lagrange update (limited slopes; PenteBorne has it
+// with fixed options only)
 template <class R>
-SweepFn<R> lagSweepKernel(bool xd, int m) {
+SweepFn<R> lagSweepKernel(bool xd, int m, bool pp) {
+  if (pp) return nullptr;
   static const SweepFn<R> kl[2][3] = {
       {k_sweep_wave_lag<R, 1, false, false, RunOpts>, k_sweep_wave_lag<R, 2, false, false, RunOpts>,
        k_sweep_wave_lag<R, 3, false, false, RunOpts>},
@@ -667,23 +669,28 @@ int phaseSweepStage(mhy_ctx* x, int sweep, int stage) {
     const int m = x->o.nbmat;
     const bool pp = x->o.pp == 1;
     // each form's kernel with fixed options, else the run-time one
+    bool missing = false;
     auto launchForm = [&](SweepFn<double> runD, SweepFn<float> runF, dim3 g, dim3 b) {
       const SweepFn<double> fd = x->mixed ? nullptr : fixedKernel<double>(x, kp, xd, lagSweep, walk);
       const SweepFn<float> ff = x->mixed ? fixedKernel<float>(x, kp, xd, lagSweep, walk) : nullptr;
-      timed(x, kid, [&] { launchR(x, fd ? fd : runD, ff ? ff : runF, g, b, kp); });
+      const SweepFn<double> kd = fd ? fd : runD;
+      const SweepFn<float> kf = ff ? ff : runF;
+      missing = x->mixed ? !kf : !kd;
+      if (!missing) timed(x, kid, [&] { launchR(x, kd, kf, g, b, kp); });
     };
     if (walk) {
       launchForm(walkKernel<double>(m, pp), walkKernel<float>(m, pp), sweepWalkGrid(x->o.nx, x->o.ny, x->walkRows), dim3(kBlock));
     } else if (o3) {  // third order: LDS-tile kernel, no PenteBorne (checked at creation)
       launchForm(o3Kernel<double>(xd, m), o3Kernel<float>(xd, m), grid, block);
     } else if (lagSweep) {  // with the cell part of the Lagrange phase
-      launchForm(lagSweepKernel<double>(xd, m), lagSweepKernel<float>(xd, m), grid, block);
+      launchForm(lagSweepKernel<double>(xd, m, pp), lagSweepKernel<float>(xd, m, pp), grid, block);
     } else if (wave) {
       launchForm(sweepWaveKernel<double>(xd, m, pp), sweepWaveKernel<float>(xd, m, pp), grid, block);
     } else {
       const KernelFn k = sweepKernel(xd, m, pp);
       timed(x, kid, [&] { hipLaunchKernelGGL(k, grid, block, 0, x->stream, kp); });
     }
+    if (missing) return fail(x, MHY_ERR_ARG, "no kernel of this cell sweep with these options");
   } else if (x->sweepWave && xd) {
     const dim3 grid = dualWaveGrid(true, x->o.nx, x->o.ny, x->mixed);
     timed(x, K_DUAL_X, [&] { launchR(x, k_dual_wave<double, true>, k_dual_wave<float, true>, grid, dim3(kBlock), kp); });
@@ -723,10 +730,10 @@ int phaseDualBoth(mhy_ctx* x) {
   const KP kp = makeKP(x);
   const bool xfirst = x->x_then_y_n;
   const int items = dualBothItems(x->o.nx, x->o.ny, x->dualRows, xfirst);
-  timed(x, K_DUAL, [&] {
-    launchR(x, dualBothKernel<double>(x->fixLim, x->o.nbmat, xfirst, x->dualRows, x->o.order),
-            dualBothKernel<float>(x->fixLim, x->o.nbmat, xfirst, x->dualRows, x->o.order), dim3((unsigned)((items + 3) / 4)), dim3(kBlock), kp);
-  });
+  const SweepFn<double> kd = dualBothKernel<double>(x->fixLim, x->o.nbmat, xfirst, x->dualRows, x->o.order);
+  const SweepFn<float> kf = dualBothKernel<float>(x->fixLim, x->o.nbmat, xfirst, x->dualRows, x->o.order);
+  if (!kd || !kf) return fail(x, MHY_ERR_ARG, "no nodal remap of both sweeps with these options");
+  timed(x, K_DUAL, [&] { launchR(x, kd, kf, dim3((unsigned)((items + 3) / 4)), dim3(kBlock), kp); });
   x->keysNext = dualBothDt(x->dualRows);
   return checkLaunch(x, "dual");
 }
@@ -2000,6 +2007,7 @@ bool batchLeavesDt(const mhy_batch* b) { return b->dualLim != 0 && dualBothDt(b-
 template <class R>
 int batchEnqueueStepR(mhy_batch* b, int cur, bool xty, bool timing, bool reduce) {
   const int n = (int)b->ctx.size();
+  bool missing = false;  // a picker has no kernel
   // fnLoop walks contiguous virtual-block ranges (blocks[k] workgroups);
   // fnOne runs one workgroup per virtual block (blocks[k] == 0)
   using Fn = void (*)(BatchLaunchT<R>);
@@ -2010,6 +2018,10 @@ int batchEnqueueStepR(mhy_batch* b, int cur, bool xty, bool timing, bool reduce)
     const bool one = !fnLoop || b->blocks[k] == 0 || b->blocks[k] >= b->total[k];
     const unsigned grid = one ? b->total[k] : b->blocks[k];
     const Fn fn = one ? fnOne : fnLoop;
+    if (!fn) {
+      missing = true;
+      return;
+    }
     if (fnLoop) b->tuner.launched(k);
     if (timing) (void)hipEventRecord(b->ev[2 * k], b->stream);
     hipLaunchKernelGGL(fn, dim3(grid), dim3(block), 0, b->stream, bl);
@@ -2051,6 +2063,7 @@ int batchEnqueueStepR(mhy_batch* b, int cur, bool xty, bool timing, bool reduce)
       launch(BK_DUY, k_dual_wave_batch<R, false, false>, k_dual_wave_batch<R, false, true>, v, dualWaveBlock(false, b->mixed));
     else launch(BK_DUY, k_dual_batch<R, false, false>, k_dual_batch<R, false, true>, v);
   }
+  if (missing) return batchFail(b, MHY_ERR_ARG, "no ensemble kernel of a sweep with these options");
   hipError_t e = hipGetLastError();
   return e == hipSuccess ? MHY_OK : batchFail(b, MHY_ERR_DEVICE, std::string("batch launch: ") + hipGetErrorString(e));
 }

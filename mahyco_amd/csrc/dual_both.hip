@@ -350,11 +350,13 @@ SweepFn<R> pickLim(int lim, bool xf, bool dt, int order) {
 }  // namespace
 template <class R>
 SweepFn<R> dualBothKernel(int lim, int m, bool xf, int rows, int order) {
+  if (!fixedExists(lim, 1, 1)) return nullptr;
   const bool dt = dualBothDt(rows);
   return m == 1 ? pickLim<R, 1>(lim, xf, dt, order) : m == 2 ? pickLim<R, 2>(lim, xf, dt, order) : pickLim<R, 3>(lim, xf, dt, order);
 }
 template <class R>
 SweepBatchFn<R> dualBothBatchKernel(int lim, int m, bool xf, int rows) {
+  if (!fixedExists(lim, 1, 1)) return nullptr;
   const bool dt = dualBothDt(rows);
   const bool mm = lim == MHY_LIM_MINMOD;
   if (m == 1) return mm ? pickBatch<R, 1, MHY_LIM_MINMOD>(xf, dt) : pickBatch<R, 1, MHY_LIM_SUPERBEE>(xf, dt);

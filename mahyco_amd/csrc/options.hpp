@@ -87,4 +87,11 @@ inline int fixedLimiter(const Opts& o) {
   return ok ? o.limiter : 0;
 }
 
+// The kernels with fixed options exist for these limiters and for the kinds of
+// sweep from firstKind on (0: first sweep with the Lagrange update, 1: first sweep, 2: second
+// sweep); their pickers return null for anything else.
+inline bool fixedExists(int lim, int kind, int firstKind) {
+  return (lim == MHY_LIM_MINMOD || lim == MHY_LIM_SUPERBEE) && kind >= firstKind && kind <= 2;
+}
+
 }  // namespace mhy

@@ -540,6 +540,7 @@ SweepFn<R> pickO3(int sweep) {
 }  // namespace
 template <class R>
 SweepFn<R> sweepFixedO3(bool xd, int m, int sweep) {
+  if (!fixedExists(MHY_LIM_MINMOD, sweep, 1)) return nullptr;
   if (m == 1) return xd ? pickO3<R, 1, true>(sweep) : pickO3<R, 1, false>(sweep);
   if (m == 2) return xd ? pickO3<R, 2, true>(sweep) : pickO3<R, 2, false>(sweep);
   return xd ? pickO3<R, 3, true>(sweep) : pickO3<R, 3, false>(sweep);

@@ -33,6 +33,7 @@ SweepFn<double> pickEucDir(bool xd, bool mixte, int sweep) {
 }  // namespace
 
 SweepFn<double> sweepFixedPP(bool xd, int lim, int m, int sweep) {
+  if (!fixedExists(lim, sweep, xd ? 0 : 1)) return nullptr;
   if (m == 1) return xd ? pickPPLim<1, true>(lim, sweep) : pickPPLim<1, false>(lim, sweep);
   if (m == 2) return xd ? pickPPLim<2, true>(lim, sweep) : pickPPLim<2, false>(lim, sweep);
   return xd ? pickPPLim<3, true>(lim, sweep) : pickPPLim<3, false>(lim, sweep);
@@ -40,6 +41,7 @@ SweepFn<double> sweepFixedPP(bool xd, int lim, int m, int sweep) {
 
 // superBee
 SweepFn<double> sweepFixedEuc(bool xd, int m, bool mixte, int sweep) {
+  if (!fixedExists(MHY_LIM_SUPERBEE, sweep, 1)) return nullptr;
   if (m == 1) return pickEucDir<5>(xd, mixte, sweep);
   if (m == 2) return pickEucDir<6>(xd, mixte, sweep);
   return pickEucDir<7>(xd, mixte, sweep);

@@ -15,6 +15,7 @@ SweepFn<R> pickWalk(int sweep) {
 }  // namespace
 template <class R>
 SweepFn<R> sweepFixedWalk(int lim, int m, int sweep) {
+  if (!fixedExists(lim, sweep, 0)) return nullptr;
   const bool mm = lim == MHY_LIM_MINMOD;
   if (m == 1) return mm ? pickWalk<R, 1, MHY_LIM_MINMOD>(sweep) : pickWalk<R, 1, MHY_LIM_SUPERBEE>(sweep);
   if (m == 2) return mm ? pickWalk<R, 2, MHY_LIM_MINMOD>(sweep) : pickWalk<R, 2, MHY_LIM_SUPERBEE>(sweep);

@@ -23,6 +23,7 @@ SweepBatchFn<R> pickBatch(int kind) {
 
 template <class R>
 SweepFn<R> sweepFixedX(int lim, int m, int kind) {
+  if (!fixedExists(lim, kind, 0)) return nullptr;
   const bool mm = lim == MHY_LIM_MINMOD;
   if (m == 1) return mm ? pick<R, 1, MHY_LIM_MINMOD>(kind) : pick<R, 1, MHY_LIM_SUPERBEE>(kind);
   if (m == 2) return mm ? pick<R, 2, MHY_LIM_MINMOD>(kind) : pick<R, 2, MHY_LIM_SUPERBEE>(kind);
@@ -30,6 +31,7 @@ SweepFn<R> sweepFixedX(int lim, int m, int kind) {
 }
 template <class R>
 SweepBatchFn<R> sweepFixedXBatch(int lim, int m, int kind) {
+  if (!fixedExists(lim, kind, 0)) return nullptr;
   const bool mm = lim == MHY_LIM_MINMOD;
   if (m == 1) return mm ? pickBatch<R, 1, MHY_LIM_MINMOD>(kind) : pickBatch<R, 1, MHY_LIM_SUPERBEE>(kind);
   if (m == 2) return mm ? pickBatch<R, 2, MHY_LIM_MINMOD>(kind) : pickBatch<R, 2, MHY_LIM_SUPERBEE>(kind);
