@@ -631,6 +631,16 @@ SweepFn<R> fixedKernel(const mhy_ctx* x, const KP& kp, bool xd, bool lag, bool w
   if (walk) return sweepFixedWalk<R>(lim, m, kind);
   return xd ? sweepFixedX<R>(lim, m, kind) : sweepFixedY<R>(lim, m, kind);
 }
+// y-first steps: the fused Lagrange update runs on walking bands
+bool lagWalks(const mhy_ctx* x) {
+  return x->lagWalkY && x->sweepWave && fixedKernel<double>(x, makeKP(x), false, true, true);
+}
+// the Lagrange cell update of y-first steps as it runs: a forced variant that these
+// options have no kernel for falls back to the strips or to the separate kernel
+int lagYVariant(const mhy_ctx* x) {
+  if (!x->fuseLag || !x->fuseLagY) return TL_SEPARATE;
+  return lagWalks(x) ? TL_WALK : TL_FUSED;
+}
 // the per-cell stencil kernels
 KernelFn sweepKernel(bool xd, int m, bool pp) {
   static const KernelFn kc[2][3][2] = {
@@ -664,7 +674,7 @@ int phaseSweepStage(mhy_ctx* x, int sweep, int stage) {
                            : gridFor(x->ncell);
     const dim3 block(wave ? sweepWaveBlock(xd, x->mixed, x->o.pp == 1) : kBlock);
     const bool lagSweep = (sweep == 1 && lagFused(x));
-    const bool walk = !xd && wave && (lagSweep ? x->lagWalkY && fixedKernel<double>(x, kp, false, true, true) : x->walkY);
+    const bool walk = !xd && wave && (lagSweep ? lagWalks(x) : x->walkY);
     const KernelId kid = lagSweep ? (xd ? K_LAGSWEEP_X : K_LAGSWEEP_Y) : (xd ? K_SWEEP_X : K_SWEEP_Y);
     const int m = x->o.nbmat;
     const bool pp = x->o.pp == 1;
@@ -1172,8 +1182,6 @@ static int createContext(const mhy_config* cfg, mhy_ctx** out, bool batchMember)
   if (const char* ly = std::getenv("MAHYCO_LAG_Y")) {
     const int c = std::string(ly) == "separate" ? TL_SEPARATE : std::string(ly) == "walk" ? TL_WALK : TL_FUSED;
     setLagY(x, c);
-    x->tune.forcedLag = kLagNames[c];
-    x->tune.choice = "lagrange_y=" + x->tune.forcedLag;
   }
   if (const char* sn = std::getenv("MAHYCO_SPLIT_NODE")) x->splitNode = (std::string(sn) != "0");
   // the tuner (MAHYCO_AUTOTUNE=0 disables it; a variant forced through the
@@ -1401,6 +1409,10 @@ static int createContext(const mhy_config* cfg, mhy_ctx** out, bool batchMember)
   x->cur = 0;
   x->x_then_y_n = true;
   x->iteration = 0;
+  if (std::getenv("MAHYCO_LAG_Y")) {
+    x->tune.forcedLag = kLagNames[lagYVariant(x)];
+    x->tune.choice = "lagrange_y=" + x->tune.forcedLag;
+  }
   *out = x;
   return MHY_OK;
 }
