@@ -1322,7 +1322,14 @@ static int createContext(const mhy_config* cfg, mhy_ctx** out, bool batchMember)
     // U_L, V_L and the centroid: the fused first sweep keeps U_L in
     // registers, but a step whose first sweep runs along y may run the
     // separate Lagrange kernel (the tuner's choice)
-    for (int q = 0; q < o.nc; ++q) AD(f.UL[q], C), AD(f.U1[q], C), AD(f.U2[q], C);
+    // U_2: only where the final remap is a kernel of its own.  (Its 3m + 1 arrays are
+    // more than the buffers of the nodal remap of both sweeps take, so the largest mesh
+    // that fits the card is no smaller for them.)
+    for (int q = 0; q < o.nc; ++q) {
+      AD(f.UL[q], C), AD(f.U1[q], C);
+      f.U2[q] = f.U1[q];
+      if (!x->fuseFinal) AD(f.U2[q], C);
+    }
     AD(f.VL, C), AD(f.XcL, C), AD(f.YcL, C);
     if (o.methode == 1) AD(f.rL, C);
     if (o.pp == 1) AD(f.qL, C);
