@@ -152,8 +152,8 @@ struct mhy_ctx {
   bool useGraph = true;
   hipGraphExec_t graph[4] = {nullptr, nullptr, nullptr, nullptr};
   int status = MHY_OK;
-  // FP64 copy of one field on its way from or to the host (max(cells, nodes)
-  // values, allocated when first needed, freed with the context)
+  // mixed form: FP64 copy of one field on its way from or to the host (a value
+  // per node), or null where the device had no room for it at set-up
   double* staging = nullptr;
   // this device's copy of the scratch array (mhy_conservation_noalloc)
   double* scratch = nullptr;
@@ -823,24 +823,22 @@ int uploadR(mhy_ctx* x, double* dst, const std::vector<double>& src) {
   return MHY_OK;
 }
 
-// the staging array, or null when the device has no room for it
-double* stagingArray(mhy_ctx* x) {
-  if (!x->staging) {
-    void* p = nullptr;
-    if (hipMalloc(&p, sizeof(double) * (size_t)std::max(x->ncell, x->nnode)) != hipSuccess) {
-      (void)hipGetLastError();
-      return nullptr;
-    }
-    x->staging = static_cast<double*>(p);
-    x->allocs.push_back(p);
+// the staging array, at set-up: field access allocates nothing.  Without room for
+// it the fields are converted on the host.
+void allocStaging(mhy_ctx* x) {
+  void* p = nullptr;
+  if (hipMalloc(&p, sizeof(double) * (size_t)x->nnode) != hipSuccess) {
+    (void)hipGetLastError();
+    return;
   }
-  return x->staging;
+  x->staging = static_cast<double*>(p);
+  x->allocs.push_back(p);
 }
 
 // n FP32 values of a device array to out as FP64: widened on the device, or on
 // the host when there is no staging array
 int readWidened(mhy_ctx* x, const float* src, double* out, long n) {
-  if (double* st = stagingArray(x)) {
+  if (double* st = x->staging) {
     hipLaunchKernelGGL(k_widen, gridFor(n), dim3(kBlock), 0, x->stream, src, st, n);
     HIPCHK(x, hipGetLastError());
     HIPCHK(x, hipMemcpyAsync(out, st, sizeof(double) * n, hipMemcpyDeviceToHost, x->stream));
@@ -1357,6 +1355,7 @@ static int createContext(const mhy_config* cfg, mhy_ctx** out, bool batchMember)
 #undef AR
 #undef AD
   if (e != hipSuccess) return bail(fail(x, MHY_ERR_DEVICE, std::string("device allocation: ") + hipGetErrorString(e)));
+  if (x->mixed) allocStaging(x);
 
   // initial state into the "n" slot 0 (setUpTimeLoopN, VnrRemap.cc:68-87)
   int u = MHY_OK;
@@ -1636,7 +1635,7 @@ int mhy_set_field(mhy_ctx* x, int field, const double* in, long long n) {
   }
   HIPCHK(x, hipStreamSynchronize(x->stream));
   if (x->mixed && isBulkField(field)) {
-    if (double* stage = stagingArray(x)) {
+    if (double* stage = x->staging) {
       HIPCHK(x, hipMemcpyAsync(stage, in, sizeof(double) * len, hipMemcpyHostToDevice, x->stream));
       hipLaunchKernelGGL(k_narrow, gridFor(len), dim3(kBlock), 0, x->stream, stage, reinterpret_cast<float*>(p), len);
       HIPCHK(x, hipGetLastError());

@@ -40,3 +40,20 @@ def test_context_is_no_larger(m, limiter, precision, pp):
         assert 0.8 * allowed < taken <= allowed
     finally:
         ctx.close()
+
+
+def test_field_access_allocates_nothing():
+    """Reading and writing fields leaves the device's free memory as it is, also in the
+    mixed form, whose values are widened and narrowed on the device."""
+    cfg = problem(1, 1500, 1500, "minmod", 1)
+    ctx = mahyco_amd.Context(cfg)
+    try:
+        ctx.run(1)
+        torch.cuda.synchronize()
+        free = torch.cuda.mem_get_info()[0]
+        rho = ctx.get("density")
+        ctx.set("density", rho)
+        ctx.get("velocity_x")
+        assert torch.cuda.mem_get_info()[0] == free
+    finally:
+        ctx.close()
