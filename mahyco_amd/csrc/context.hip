@@ -1741,9 +1741,18 @@ int mhy_kernel_bytes(const mhy_ctx* x, int k, double* bytes) {
   // q_k for the centred pseudo
   const int bulkIn = (x->o.pseudo_centree == 1 ? 5 : 4) * m;
   const double r = x->mixed ? 4.0 : 8.0, d = 8.0, i1 = 1.0;
+  // one material whose fields are stored where they differ from the means only:
+  // the material fields are neither read nor written (but q_k of the centred pseudo),
+  // one more flag is
+  const bool compact = x->o.compact1;
   // cell part of the final remap: U2 in registers or read; writes rho, e, q,
   // p, c, mu_k, rho_k, e_k, p_k, c_k (bulk) and M, f_k, M_k, flags
-  const double finalWrites = C * r * (5 + 5 * m) + C * d * (1 + 2 * m) + C * i1;
+  const double finalWrites =
+      compact ? C * r * 5 + C * d + C * i1 * 2 : C * r * (5 + 5 * m) + C * d * (1 + 2 * m) + C * i1;
+  // what the Lagrange update reads: u_n+1 ; f, M_k, vol (FP64), mu, rho_k, e_k,
+  // p_k, q_k + rho, divu, c ; compact: vol, M, rho, divu, c, e, p and the flag
+  const double lagIn = N * 2 * r + (compact ? C * (2 * d + (5 + (bulkIn - 4 * m)) * r + i1)
+                                            : C * ((2 * m + 1) * d + (bulkIn + 3) * r));
   double w = 0;
   if (x->euc) {  // Eucclhyd kernels (FP64)
     const bool o2 = x->o.space_order == 2, lag = x->o.mode == MODE_LAGRANGE;
@@ -1777,9 +1786,8 @@ int mhy_kernel_bytes(const mhy_ctx* x, int k, double* bytes) {
     case K_DT: w = C * (d + 2 * r) + N * 2 * r; break;  // vol ; c, p ; u
     case K_NODE: w = N * 2 * r + C * (2 * r + d) + N * 3 * r; break;  // u_n ; p, q ; M ; u_n+1, Mp
     case K_CELL:
-      // u_n+1 ; f, M_k, vol (FP64), mu, rho_k, e_k, p_k, q_k + rho, divu, c ;
       // writes UL, VL, XcL, YcL (+ rL, qL) (FP64), divu, q_k
-      w = N * 2 * r + C * ((2 * m + 1) * d + (bulkIn + 3) * r) + C * d * (nc + 3 + (meth == 1) + pp) + C * r * (1 + m);
+      w = lagIn + C * d * (nc + 3 + (meth == 1) + pp) + C * r * (1 + m);
       break;
     case K_SWEEP_X:
     case K_SWEEP_Y: {
@@ -1802,10 +1810,8 @@ int mhy_kernel_bytes(const mhy_ctx* x, int k, double* bytes) {
     }
     case K_LAGSWEEP_X:
     case K_LAGSWEEP_Y: {
-      // the Lagrange cell update's inputs (u_n+1 ; f, M_k, vol (FP64), mu,
-      // rho_k, e_k, p_k, q_k + rho, divu, c) and outputs that outlive the
-      // step (divu, q_k ; rL, qL), then sweep 1's outputs: U_1, face fluxes
-      const double lagIn = N * 2 * r + C * ((2 * m + 1) * d + (bulkIn + 3) * r);
+      // the Lagrange cell update's inputs and outputs that outlive the step
+      // (divu, q_k ; rL, qL), then sweep 1's outputs: U_1, face fluxes
       const double lagOut = C * r * (1 + m) + C * d * ((meth == 1) + pp);
       const double fl = (meth == 2 ? C * m : F * m) * d;
       w = lagIn + lagOut + C * nc * d + fl;
