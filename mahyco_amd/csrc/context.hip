@@ -1285,76 +1285,92 @@ static int createContext(const mhy_config* cfg, mhy_ctx** out, bool batchMember)
     return bail(fail(x, MHY_ERR_DEVICE, "hipGetSymbolAddress of the scratch array failed"));
   if ((e = hipStreamCreate(&x->stream)) != hipSuccess) return bail(fail(x, MHY_ERR_DEVICE, hipGetErrorString(e)));
   Fields& f = x->f;
-  std::memset(&f, 0, sizeof(f));
 #define AD(ptr, n) ((ptr) = allocD(x, (n), e))
 #define AR(ptr, n) ((ptr) = allocR(x, (n), e))
-  for (int s = 0; s < 2; ++s) {
-    AR(f.rho[s], C), AR(f.p[s], C), AR(f.q[s], C), AR(f.c[s], C), AR(f.divu[s], C), AR(f.e[s], C);
-    for (int k = 0; k < m; ++k) {
-      AR(f.rho_k[s][k], C), AR(f.p_k[s][k], C), AR(f.q_k[s][k], C), AR(f.c_k[s][k], C), AR(f.e_k[s][k], C);
-    }
-    AR(f.ux[s], N), AR(f.uy[s], N);
-  }
-  if (o.mode == MODE_LAGRANGE) {
-    for (int s = 0; s < 2; ++s) AD(f.X[s], N), AD(f.Y[s], N), AD(f.vol[s], C);
-    AR(f.outvx, N), AR(f.outvy, N);
-  } else {
-    AD(f.vol[0], C);
-    f.vol[1] = f.vol[0];  // Euler sub-volumes: constant
-    if (o.mode == MODE_FULL) AD(f.cvol, C);
-  }
-  for (int k = 0; k < m; ++k) AD(f.f_k[k], C), AR(f.mu_k[k], C), AD(f.M_k[k], C);
-  AD(f.M, C);
-  f.flags = allocB(x, C, e);
-  if (o.compact1 && e == hipSuccess) {
-    void* p = nullptr;
-    if ((e = hipMalloc(&p, C)) == hipSuccess) x->allocs.push_back(p);
-    f.envx = static_cast<unsigned char*>(p);
-  }
-  AR(f.Mp, N);
-  if (o.periodic_right) {
-    AR(f.rho0, C), AR(f.e0, C);
-    for (int k = 0; k < m; ++k) AR(f.rho_k0[k], C), AR(f.e_k0[k], C);
-  }
-  if (o.mode != MODE_LAGRANGE) {
-    // U_L, V_L and the centroid: the fused first sweep keeps U_L in
-    // registers, but a step whose first sweep runs along y may run the
-    // separate Lagrange kernel (the tuner's choice)
-    // U_2: only where the final remap is a kernel of its own.  (Its 3m + 1 arrays are
-    // more than the buffers of the nodal remap of both sweeps take, so the largest mesh
-    // that fits the card is no smaller for them.)
-    for (int q = 0; q < o.nc; ++q) {
-      AD(f.UL[q], C), AD(f.U1[q], C);
-      f.U2[q] = f.U1[q];
-      if (!x->fuseFinal) AD(f.U2[q], C);
-    }
-    AD(f.VL, C), AD(f.XcL, C), AD(f.YcL, C);
-    if (o.methode == 1) AD(f.rL, C);
-    if (o.pp == 1) AD(f.qL, C);
-    x->nface = std::max((long)(c.nx + 1) * c.ny, (long)c.nx * (c.ny + 1));
-    if (o.methode == 0 || o.methode == 1)
+  // every array; storeU2: U_2 too where the second sweep finishes its cells, which does
+  // not need it
+  auto allocArrays = [&](bool storeU2) {
+    std::memset(&f, 0, sizeof(f));
+    e = hipSuccess;
+    for (int s = 0; s < 2; ++s) {
+      AR(f.rho[s], C), AR(f.p[s], C), AR(f.q[s], C), AR(f.c[s], C), AR(f.divu[s], C), AR(f.e[s], C);
       for (int k = 0; k < m; ++k) {
-        AD(f.G[k], x->nface);
-        f.G2[k] = f.G[k];
-        if (x->dualBoth) AD(f.G2[k], x->nface);
+        AR(f.rho_k[s][k], C), AR(f.p_k[s][k], C), AR(f.q_k[s][k], C), AR(f.c_k[s][k], C), AR(f.e_k[s][k], C);
       }
-    if (x->dualBoth) AR(f.uxl, N), AR(f.uyl, N);
-    if (o.methode == 2)
-      for (int k = 0; k < m; ++k) AD(f.DF[k], C);
-    for (int d = 0; d < 3; ++d) AD(f.UD1[d], N);
-    AD(f.XL2, N);
-  }
-  if (e == hipSuccess) {
-    void* p = nullptr;
-    if ((e = hipMalloc(&p, sizeof(Scalars))) == hipSuccess) x->allocs.push_back(p);
-    f.sc = static_cast<Scalars*>(p);
-    p = nullptr;
-    if (e == hipSuccess && (e = hipMalloc(&p, sizeof(DtKeys))) == hipSuccess) x->allocs.push_back(p);
-    f.keys = static_cast<DtKeys*>(p);
-  }
+      AR(f.ux[s], N), AR(f.uy[s], N);
+    }
+    if (o.mode == MODE_LAGRANGE) {
+      for (int s = 0; s < 2; ++s) AD(f.X[s], N), AD(f.Y[s], N), AD(f.vol[s], C);
+      AR(f.outvx, N), AR(f.outvy, N);
+    } else {
+      AD(f.vol[0], C);
+      f.vol[1] = f.vol[0];  // Euler sub-volumes: constant
+      if (o.mode == MODE_FULL) AD(f.cvol, C);
+    }
+    for (int k = 0; k < m; ++k) AD(f.f_k[k], C), AR(f.mu_k[k], C), AD(f.M_k[k], C);
+    AD(f.M, C);
+    f.flags = allocB(x, C, e);
+    if (o.compact1 && e == hipSuccess) {
+      void* p = nullptr;
+      if ((e = hipMalloc(&p, C)) == hipSuccess) x->allocs.push_back(p);
+      f.envx = static_cast<unsigned char*>(p);
+    }
+    AR(f.Mp, N);
+    if (o.periodic_right) {
+      AR(f.rho0, C), AR(f.e0, C);
+      for (int k = 0; k < m; ++k) AR(f.rho_k0[k], C), AR(f.e_k0[k], C);
+    }
+    if (o.mode != MODE_LAGRANGE) {
+      // U_L, V_L and the centroid: the fused first sweep keeps U_L in
+      // registers, but a step whose first sweep runs along y may run the
+      // separate Lagrange kernel (the tuner's choice)
+      for (int q = 0; q < o.nc; ++q) {
+        AD(f.UL[q], C), AD(f.U1[q], C);
+        f.U2[q] = f.U1[q];
+        if (storeU2) AD(f.U2[q], C);
+      }
+      AD(f.VL, C), AD(f.XcL, C), AD(f.YcL, C);
+      if (o.methode == 1) AD(f.rL, C);
+      if (o.pp == 1) AD(f.qL, C);
+      x->nface = std::max((long)(c.nx + 1) * c.ny, (long)c.nx * (c.ny + 1));
+      if (o.methode == 0 || o.methode == 1)
+        for (int k = 0; k < m; ++k) {
+          AD(f.G[k], x->nface);
+          f.G2[k] = f.G[k];
+          if (x->dualBoth) AD(f.G2[k], x->nface);
+        }
+      if (x->dualBoth) AR(f.uxl, N), AR(f.uyl, N);
+      if (o.methode == 2)
+        for (int k = 0; k < m; ++k) AD(f.DF[k], C);
+      for (int d = 0; d < 3; ++d) AD(f.UD1[d], N);
+      AD(f.XL2, N);
+    }
+    if (e == hipSuccess) {
+      void* p = nullptr;
+      if ((e = hipMalloc(&p, sizeof(Scalars))) == hipSuccess) x->allocs.push_back(p);
+      f.sc = static_cast<Scalars*>(p);
+      p = nullptr;
+      if (e == hipSuccess && (e = hipMalloc(&p, sizeof(DtKeys))) == hipSuccess) x->allocs.push_back(p);
+      f.keys = static_cast<DtKeys*>(p);
+    }
+  };
 #undef AR
 #undef AD
-  if (e != hipSuccess) return bail(fail(x, MHY_ERR_DEVICE, std::string("device allocation: ") + hipGetErrorString(e)));
+  // A device without room for all of it gets the context without U_2, whose 3m + 1 arrays
+  // are more than the buffers of the nodal remap of both sweeps take.  (Always without it,
+  // other arrays lie elsewhere in the caches: three materials FP64 between -3.2 and
+  // +0.5 % by mesh, 0.7 % slower in the mean of 12.)
+  allocArrays(true);
+  if (e == hipErrorOutOfMemory && x->fuseFinal) {
+    (void)hipGetLastError();
+    for (void* p : x->allocs) (void)hipFree(p);
+    x->allocs.clear();
+    allocArrays(false);
+  }
+  if (e != hipSuccess) {
+    (void)hipGetLastError();  // (not another context's error)
+    return bail(fail(x, MHY_ERR_DEVICE, std::string("device allocation: ") + hipGetErrorString(e)));
+  }
   if (x->mixed) allocStaging(x);
 
   // initial state into the "n" slot 0 (setUpTimeLoopN, VnrRemap.cc:68-87)
