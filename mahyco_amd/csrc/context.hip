@@ -153,7 +153,7 @@ struct mhy_ctx {
   hipGraphExec_t graph[4] = {nullptr, nullptr, nullptr, nullptr};
   int status = MHY_OK;
   // mixed form: FP64 copy of one field on its way from or to the host (a value
-  // per node), or null where the device had no room for it at set-up
+  // per node), or null on small meshes and where the device had no room for it
   double* staging = nullptr;
   // this device's copy of the scratch array (mhy_conservation_noalloc)
   double* scratch = nullptr;
@@ -823,9 +823,29 @@ int uploadR(mhy_ctx* x, double* dst, const std::vector<double>& src) {
   return MHY_OK;
 }
 
-// the staging array, at set-up: field access allocates nothing.  Without room for
-// it the fields are converted on the host.
+// Mixed form: a field of n values is converted on the device, so that FP64 crosses to
+// or from the caller's buffer, or on the host.  The device conversion wins where the
+// copy runs at the link's rate, a pinned buffer, from about 10^5 values on (us, host / device
+// conversion, reading: 256^2 values 26 / 31, 400^2 52 / 44, 1024^2 381 / 172, 2048^2 2000 / 623); into
+// pageable memory twice the bytes cost more than the conversion saves until the fields
+// are large (reading 512^2 97 / 122, 1024^2 380 / 472, 2048^2 2000 / 1890, 4096^2 20100 / 7440; writing
+// 512^2 84 / 96, 1024^2 254 / 262, 1448^2 474 / 483, 2048^2 1490 / 940).
+constexpr long kConvertPinned = 1L << 17, kConvertRead = 1L << 22, kConvertWrite = 1L << 21;
+bool convertOnDevice(const mhy_ctx* x, const void* buffer, long n, bool read) {
+  if (!x->staging || n < kConvertPinned) return false;
+  if (n >= (read ? kConvertRead : kConvertWrite)) return true;
+  hipPointerAttribute_t a;
+  if (hipPointerGetAttributes(&a, buffer) != hipSuccess) {
+    (void)hipGetLastError();  // (ordinary host memory)
+    return false;
+  }
+  return a.type == hipMemoryTypeHost;
+}
+
+// the staging array of that conversion, at set-up: field access allocates nothing.
+// Without room for it the fields are converted on the host.
 void allocStaging(mhy_ctx* x) {
+  if (x->nnode < kConvertPinned) return;
   void* p = nullptr;
   if (hipMalloc(&p, sizeof(double) * (size_t)x->nnode) != hipSuccess) {
     (void)hipGetLastError();
@@ -835,10 +855,10 @@ void allocStaging(mhy_ctx* x) {
   x->allocs.push_back(p);
 }
 
-// n FP32 values of a device array to out as FP64: widened on the device, or on
-// the host when there is no staging array
+// n FP32 values of a device array to out as FP64
 int readWidened(mhy_ctx* x, const float* src, double* out, long n) {
-  if (double* st = x->staging) {
+  if (convertOnDevice(x, out, n, true)) {
+    double* st = x->staging;
     hipLaunchKernelGGL(k_widen, gridFor(n), dim3(kBlock), 0, x->stream, src, st, n);
     HIPCHK(x, hipGetLastError());
     HIPCHK(x, hipMemcpyAsync(out, st, sizeof(double) * n, hipMemcpyDeviceToHost, x->stream));
@@ -1651,7 +1671,8 @@ int mhy_set_field(mhy_ctx* x, int field, const double* in, long long n) {
   }
   HIPCHK(x, hipStreamSynchronize(x->stream));
   if (x->mixed && isBulkField(field)) {
-    if (double* stage = x->staging) {
+    if (convertOnDevice(x, in, len, false)) {
+      double* stage = x->staging;
       HIPCHK(x, hipMemcpyAsync(stage, in, sizeof(double) * len, hipMemcpyHostToDevice, x->stream));
       hipLaunchKernelGGL(k_narrow, gridFor(len), dim3(kBlock), 0, x->stream, stage, reinterpret_cast<float*>(p), len);
       HIPCHK(x, hipGetLastError());

@@ -802,8 +802,9 @@ __global__ __launch_bounds__(256) void k_conservation(KPT<R> kp, double* out) {
 
 // Field access: FP32 device arrays to FP64 and back, so that the host
 // copies FP64 values only.  Bound by memory (12 bytes per value); converted on
-// the host by one thread, the four fields of a 2048^2 mixed state took 9.0 ms, so
-// about 2 ms (50 steps and the four fields 31.5 -> 24.1 ms).
+// the host by one thread, the four fields of a 2048^2 mixed state took 9.0 ms into pinned
+// memory, so about 2 ms (50 steps and the four fields 31.5 -> 24.1 ms).  convertOnDevice
+// (context.hip) says which calls take it.
 __global__ __launch_bounds__(256) void k_widen(const float* in, double* out, long n) {
   const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) out[i] = (double)in[i];
