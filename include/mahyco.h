@@ -309,9 +309,10 @@ int mhy_kernel_count(const mhy_ctx* ctx);
  * first sweep on strips or on walking bands, or run as its own kernel;
  * results bitwise the same) and keep
  * the fastest before any graph is captured.  Returns the kept variants
- * ("dual_y=both sweep_y=walk lagrange_y=fused") and a Lagrange variant forced
- * through the environment (MAHYCO_LAG_Y), or "" while tuning or when the
- * tuner is off (MAHYCO_AUTOTUNE=0).  No counterpart in the reference. */
+ * ("dual_y=both sweep_y=walk lagrange_y=fused").  With a Lagrange variant forced
+ * through the environment (MAHYCO_LAG_Y), the one that runs with these options
+ * ("lagrange_y=separate" where they have no kernel for it).  "" while tuning or
+ * when the tuner is off (MAHYCO_AUTOTUNE=0).  No counterpart in the reference. */
 const char* mhy_tuned_kernels(const mhy_ctx* ctx);
 const char* mhy_kernel_name(const mhy_ctx* ctx, int k);
 int mhy_kernel_bytes(const mhy_ctx* ctx, int k, double* bytes_per_launch);

@@ -117,8 +117,9 @@ struct mhy_ctx {
   // centroid for the second (environment MAHYCO_SWEEP_GEOM=load), or the
   // second sweep forms them again from the node velocities (=recompute)
   bool geomStored = true;
-  // node update on the Euler grid as an interior kernel and a boundary
-  // kernel (MAHYCO_SPLIT_NODE=0: one kernel for all nodes)
+  // node update on the Euler grid as one launch of walking bands for the interior
+  // nodes and general threads for the boundary ones (MAHYCO_SPLIT_NODE=0: one general
+  // thread per node)
   bool splitNode = true;
   // nodal remap along y: the wave kernel (default) or the per-node stencil
   // kernel (environment MAHYCO_DUAL_Y=node)
@@ -1187,10 +1188,10 @@ static int createContext(const mhy_config* cfg, mhy_ctx** out, bool batchMember)
   if (const char* g = std::getenv("MAHYCO_GRAPH")) x->useGraph = (std::string(g) != "0");
   // the fused first sweep needs the wave kernels for both sweep directions
   // (the column walker and the third-order and per-cell kernels read the
-  // stored remap vector).  The PenteBorne sweeps are bound by their FP64
-  // arithmetic, not by memory: the Lagrange update runs better as its own
-  // streaming kernel there (2048^2 two-material case: 1.24 ms per step
-  // separate, 1.27 ms fused), so it is fused with the limited-slope sweeps only.
+  // stored remap vector).  PenteBorne sweeps with run-time options are bound by
+  // their FP64 arithmetic and registers, not by memory: the Lagrange update runs better
+  // as its own streaming kernel there (2048^2 two-material case: 1.24 ms per step
+  // separate, 1.27 ms fused).  With fixed options the x-first steps fuse it, set below.
   // (a column-walking second sweep reads the stored Lagrange geometry)
   if (const char* sg = std::getenv("MAHYCO_SWEEP_GEOM")) x->geomStored = (std::string(sg) != "recompute");
   x->fuseLag = x->sweepWave && c.projection_order != 3 && c.avec_projection == 1 && !batchMember && c.pp != 1 &&

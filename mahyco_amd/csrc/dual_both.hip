@@ -5,7 +5,8 @@
 // One sweep at a time the nodal remap is bound by memory: it stores the nodal
 // momentum and mass and the Lagrange coordinate of the second axis for the
 // next sweep to read back, 8 of the 15 array passes of the pair.  Here a wave
-// covers 64 node columns (59 or 58 updated) and walks down a band of node rows: the
+// covers 64 node columns (60 or 59 updated, x or y first; one less with DT) and walks
+// down a band of node rows: the
 // row-wise sweep works on one node row, its along-x neighbours being the
 // adjacent lanes (DPP moves), and the column-wise sweep on the rows the wave
 // keeps in registers.  A classic limiter's gradient needs one neighbour on

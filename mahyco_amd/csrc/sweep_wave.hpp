@@ -25,9 +25,10 @@
 // LAG: the first sweep of a step also runs the cell part of the Lagrange
 // phase (lagrangeCellCompute): each lane forms its cell's Lagrange update and
 // remap vector in registers, the halo lanes redundantly, and only the
-// updated cells store the words that outlive the step.  The remap vector,
-// the Lagrange volume and the centroid never go through memory; the second
-// sweep forms the volume and centroid again from the node velocities.
+// updated cells store the words that outlive the step.  The remap vector
+// never goes through memory; the Lagrange volume and the centroid along the second
+// sweep's axis are stored for that sweep, or formed again by it from the node
+// velocities (geomLoad 0).
 #pragma once
 
 #include <type_traits>
@@ -433,26 +434,26 @@ __device__ __forceinline__ void sweepWaveBody(const KPT<R>& kp, unsigned b) {
 template <class R, bool PP, bool XD>
 constexpr int kMinWaves = (!XD && kMixed<R> && !PP) ? 4 : 1;
 // the same for the ensemble kernels, whose three-material form would spill
-template <class R, int M, bool PP, bool XD, class P>
+template <class R, int M, bool PP, bool XD>
 constexpr int kMinWavesBatch = (M < 3) ? kMinWaves<R, PP, XD> : 1;
 // the plain sweeps of one material in FP64 with limited slopes need 98
 // VGPRs unbounded with run-time options; 96 (5 waves per SIMD instead of 4)
 // costs no spill.  (With fixed options they take 79, 6 waves.)
-template <class R, int L, bool PP, bool XD, class P>
+template <class R, int L, bool PP, bool XD>
 constexpr int kMinWavesPlain = (!kMixed<R> && L == 1 && !PP) ? 5 : kMinWaves<R, PP, XD>;
-template <class R, int L, bool PP, bool XD, class P>
+template <class R, int L, bool PP, bool XD>
 constexpr int kMinWavesLag = kParkLag<R, L, PP> ? 5 : kMinWaves<R, PP, XD>;
 
 template <class R, int M, bool PP, bool XD, class P>
 __global__ __launch_bounds__((XD ? 256 : 64 * kYWaves<R, PP>))
-__attribute__((amdgpu_waves_per_eu(kMinWavesPlain<R, M, PP, XD, P>))) void k_sweep_wave(KPT<R> kp) {
+__attribute__((amdgpu_waves_per_eu(kMinWavesPlain<R, M, PP, XD>))) void k_sweep_wave(KPT<R> kp) {
   sweepWaveBody<R, M, PP, XD, false, P>(kp, XD ? blockIdx.x : xcdBlock());
 }
 
 // the first sweep of a step with the cell part of the Lagrange phase
 template <class R, int M, bool PP, bool XD, class P>
 __global__ __launch_bounds__((XD ? 256 : 64 * kYWaves<R, PP>))
-__attribute__((amdgpu_waves_per_eu(kMinWavesLag<R, M, PP, XD, P>))) void k_sweep_wave_lag(KPT<R> kp) {
+__attribute__((amdgpu_waves_per_eu(kMinWavesLag<R, M, PP, XD>))) void k_sweep_wave_lag(KPT<R> kp) {
   sweepWaveBody<R, M, PP, XD, true, P>(kp, XD ? blockIdx.x : xcdBlock());
 }
 
@@ -460,7 +461,7 @@ __attribute__((amdgpu_waves_per_eu(kMinWavesLag<R, M, PP, XD, P>))) void k_sweep
 // the first sweep with the Lagrange update
 template <class R, int M, bool XD, class P>
 __global__ __launch_bounds__((XD ? 256 : 64 * kYWaves<R, false>))
-__attribute__((amdgpu_waves_per_eu(kMinWavesLag<R, M, false, XD, P>))) void k_sweep_wave_lag_batch(BatchLaunchT<R> bl) {
+__attribute__((amdgpu_waves_per_eu(kMinWavesLag<R, M, false, XD>))) void k_sweep_wave_lag_batch(BatchLaunchT<R> bl) {
   batchRun<true>(bl, [&](const KPT<R>& kp, unsigned local, unsigned, unsigned) {
     sweepWaveBody<R, M, false, XD, true, P>(kp, local);
   });
@@ -468,7 +469,7 @@ __attribute__((amdgpu_waves_per_eu(kMinWavesLag<R, M, false, XD, P>))) void k_sw
 // all problems of an ensemble in one launch (BatchLaunchT, common.hpp)
 template <class R, int M, bool PP, bool XD, bool ONE, class P>
 __global__ __launch_bounds__((XD ? 256 : 64 * kYWaves<R, PP>))
-__attribute__((amdgpu_waves_per_eu(kMinWavesBatch<R, M, PP, XD, P>))) void k_sweep_wave_batch(BatchLaunchT<R> bl) {
+__attribute__((amdgpu_waves_per_eu(kMinWavesBatch<R, M, PP, XD>))) void k_sweep_wave_batch(BatchLaunchT<R> bl) {
   batchRun<ONE>(bl, [&](const KPT<R>& kp, unsigned local, unsigned, unsigned) {
     sweepWaveBody<R, M, PP, XD, false, P>(kp, local);
   });
