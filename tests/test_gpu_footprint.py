@@ -2,9 +2,10 @@
 stored U_2 and the mixed / pure flags in two integers per cell: its buffers for the nodal
 remap of both sweeps take more, and a device without room for them gets the same
 context without U_2.  2047^2 cells: node arrays of 32 MiB, cell and face arrays just below."""
+import ctypes
+
 import numpy as np
 import pytest
-import torch
 
 import mahyco_amd
 
@@ -14,6 +15,14 @@ from test_gpu_fixed_options import problem
 pytestmark = pytest.mark.gpu
 
 MIB = 1 << 20
+
+
+def free_bytes():
+    """Free device memory, from the HIP runtime the library runs on."""
+    L, free, total = mahyco_amd.library(), ctypes.c_size_t(), ctypes.c_size_t()
+    assert L.hipDeviceSynchronize() == 0
+    assert L.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    return free.value
 
 
 def needed(m, precision):
@@ -33,21 +42,22 @@ def test_context_fits_a_nearly_full_device(m, precision):
         ctx = mahyco_amd.Context(cfg)
         try:
             ctx.run(40)  # the tuning steps, then replays
-            return [ctx.get(n, k) for n, k in names], (free - torch.cuda.mem_get_info()[0]) / MIB
+            return [ctx.get(n, k) for n, k in names], (free - free_bytes()) / MIB
         finally:
             ctx.close()
 
-    torch.cuda.synchronize()
-    free = torch.cuda.mem_get_info()[0]
+    free = free_bytes()
     want, roomy = fields()
     room = needed(m, precision) + 24  # (the runtime's own)
     filler = []
     try:
         for _ in range(3):  # (the runtime hands memory of its own back on the way)
-            more = torch.cuda.mem_get_info()[0] - room * MIB
+            more = free_bytes() - room * MIB
             if more >= 4 * MIB:
-                filler.append(torch.empty(more, dtype=torch.uint8, device="cuda"))
-        free = torch.cuda.mem_get_info()[0]
+                block = ctypes.c_void_p()
+                assert mahyco_amd.library().hipMalloc(ctypes.byref(block), ctypes.c_size_t(more)) == 0
+                filler.append(block)
+        free = free_bytes()
         assert abs(free / MIB - room) <= 24
         got, tight = fields()
         log(f"[footprint] m={m} precision={precision}: {roomy:.0f} MiB, with {room} MiB free {tight:.0f} MiB")
@@ -55,8 +65,8 @@ def test_context_fits_a_nearly_full_device(m, precision):
         for (n, k), a, b in zip(names, got, want):
             assert np.array_equal(a, b), (n, k)
     finally:
-        filler.clear()
-        torch.cuda.empty_cache()
+        for block in filler:
+            assert mahyco_amd.library().hipFree(block) == 0
 
 
 def test_field_access_allocates_nothing():
@@ -66,11 +76,10 @@ def test_field_access_allocates_nothing():
     ctx = mahyco_amd.Context(cfg)
     try:
         ctx.run(1)
-        torch.cuda.synchronize()
-        free = torch.cuda.mem_get_info()[0]
+        free = free_bytes()
         rho = ctx.get("density")
         ctx.set("density", rho)
         ctx.get("velocity_x")
-        assert torch.cuda.mem_get_info()[0] == free
+        assert free_bytes() == free
     finally:
         ctx.close()
